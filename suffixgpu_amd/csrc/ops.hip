@@ -179,26 +179,34 @@ __global__ __launch_bounds__(kOccThreads) void k_first_occ(
 }
 
 // --------------------------------------------------------------- sa_search
+// A search is a chain of dependent rounds (a suffix position, then its
+// tokens), so what bounds a call is rounds times two memory round trips
+// until the lanes fill the chip, and the probes' reads from then on.
+// G = 32 lanes per pattern, compared by octets, cut 2^22 ranks in 5 rounds;
+// G = 8 with a lane per probe takes 7, each with a dependent load per 4
+// matched tokens, but reads 2.5 times fewer probes.  Calls over 2^22
+// suffixes with G = 8 / G = 32: 2,048 patterns 36.3 / 22.1 us, 8,192 44.3 /
+// 31.3, 16,384 52.0 / 55.3 (over 20,000 suffixes 18.2 / 13.6, 26.1 / 16.3,
+// 27.4 / 26.4), so G = 32 up to kWideSearchMax patterns.
 constexpr int kSearchThreads = 256;
-constexpr int kOpGroup = 8;
 
+template <int G, bool kOct>
 __global__ __launch_bounds__(kSearchThreads) void k_sa_search(
     const int32_t* __restrict__ sa, const int32_t* __restrict__ corpus,
     int64_t n, const int32_t* __restrict__ pattern, int64_t batch,
     int64_t width, const int64_t* __restrict__ plen, int64_t* lower,
     int64_t* upper) {
-  const int64_t row =
-      (int64_t)blockIdx.x * (kSearchThreads / kOpGroup) +
-      threadIdx.x / kOpGroup;
+  const int64_t row = (int64_t)blockIdx.x * (kSearchThreads / G) +
+                      threadIdx.x / G;
   if (row >= batch) return;  // whole groups exit together
   const int32_t* pr = pattern + row * width;
   int64_t pl = plen[row];
   pl = pl < 0 ? 0 : (pl > width ? width : pl);
   auto pat_at = [&](int j) -> int32_t { return pr[j]; };
   int64_t lo, hi;
-  kary_bounds<kOpGroup>(sa, corpus, n, nullptr, 0, pat_at, (int)pl, lo, hi,
-                        0u, (uint32_t)n);
-  if (threadIdx.x % kOpGroup == 0) {
+  kary_bounds<G, kOct>(sa, corpus, n, nullptr, 0, pat_at, (int)pl, lo, hi,
+                       0u, (uint32_t)n);
+  if (threadIdx.x % G == 0) {
     lower[row] = lo;
     upper[row] = hi;
   }
@@ -409,6 +417,8 @@ extern "C" int sfx_first_occurrences(const int32_t* mb, int64_t n_cols,
   return (int)hipGetLastError();
 }
 
+constexpr int64_t kWideSearchMax = 1 << 13;
+
 extern "C" int sfx_sa_search(const int32_t* sa, const int32_t* corpus,
                              int64_t n, const int32_t* pattern,
                              int64_t batch, int64_t width,
@@ -419,11 +429,17 @@ extern "C" int sfx_sa_search(const int32_t* sa, const int32_t* corpus,
   if (!sa || !corpus || !plen || !lower || !upper ||
       (width > 0 && !pattern))
     return SFX_EINVAL;
-  const int64_t per_block = kSearchThreads / kOpGroup;
+  const bool wide = batch <= kWideSearchMax;
+  const int64_t per_block = kSearchThreads / (wide ? 32 : 8);
   const int64_t blocks = (batch + per_block - 1) / per_block;
-  hipLaunchKernelGGL(k_sa_search, dim3((unsigned)blocks),
-                     dim3(kSearchThreads), 0, stream, sa, corpus, n, pattern,
-                     batch, width, plen, lower, upper);
+  if (wide)
+    hipLaunchKernelGGL((k_sa_search<32, true>), dim3((unsigned)blocks),
+                       dim3(kSearchThreads), 0, stream, sa, corpus, n,
+                       pattern, batch, width, plen, lower, upper);
+  else
+    hipLaunchKernelGGL((k_sa_search<8, false>), dim3((unsigned)blocks),
+                       dim3(kSearchThreads), 0, stream, sa, corpus, n,
+                       pattern, batch, width, plen, lower, upper);
   return (int)hipGetLastError();
 }
 

@@ -172,6 +172,77 @@ __device__ __forceinline__ int cmp_probes_key(
   return 0;
 }
 
+// The same comparison through sa and the corpus (no key rows): each lane
+// reads its own probe's suffix position, then the lanes of an octet read
+// 32 corpus tokens of one probe's suffix, 4 per lane, so a round is two
+// dependent loads however long the match is.  (One probe per lane, 4 tokens
+// a step, takes a dependent load for every 4 tokens a probe shares with the
+// pattern, and a narrow range's probes share nearly all of them.)  A corpus
+// position is only 4-byte aligned; its 16 bytes are one load all the same.
+struct __attribute__((packed, aligned(4))) Tokens4 {
+  int32_t t[4];
+};
+
+template <int G, class ProbeFn, class PatFn>
+__device__ __forceinline__ int cmp_probes_corpus(
+    const int32_t* __restrict__ sa, const int32_t* __restrict__ corpus,
+    int64_t n, ProbeFn probe_of, const int32_t (&pc)[4], PatFn pat_at,
+    int plen) {
+  constexpr int kParts = 8;          // lanes per probe: 32 tokens
+  constexpr int kRows = G / kParts;  // probes per load instruction
+  constexpr int kInstr = G / kRows;
+  static_assert(G % kParts == 0, "whole octets per group");
+  const int ln = lane_id();
+  const int gl = ln % G;
+  const int gbase = ln - gl;
+  const int part = gl % kParts;
+  const int sub = gl / kParts;
+  const int kn = plen < 4 * kParts ? plen : 4 * kParts;
+  const bool live = 4 * part < kn;
+  const int32_t own = sa[probe_of(gl)];  // n < 2^31
+  Tokens4 v[kInstr];
+#pragma unroll
+  for (int i = 0; i < kInstr; ++i) {
+    const int64_t at =
+        (int64_t)__shfl(own, gbase + i * kRows + sub) + 4 * part;
+    if (live && at >= 0 && at + 3 < n) {
+      v[i] = *reinterpret_cast<const Tokens4*>(corpus + at);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        v[i].t[j] = live && at + j < n ? corpus[at + j > 0 ? at + j : 0] : -1;
+    }
+  }
+  int cv = 0;
+#pragma unroll
+  for (int i = 0; i < kInstr; ++i) {
+    bool mis = false, neg = false;
+#pragma unroll
+    for (int j = 3; j >= 0; --j) {  // the lowest differing token wins
+      if (live && 4 * part + j < kn && v[i].t[j] != pc[j]) {
+        mis = true;
+        neg = v[i].t[j] < pc[j];
+      }
+    }
+    const uint64_t bm = ballot(mis);
+    const uint64_t bn = ballot(mis && neg);
+    const int ob = gbase + kParts * (gl % kRows);  // own probe's octet
+    const uint32_t seg = (uint32_t)(bm >> ob) & 0xffu;
+    const int lb = seg ? __builtin_ctz(seg) : 0;
+    const bool nb = (bn >> (ob + lb)) & 1ull;
+    const int r = seg == 0 ? 0 : (nb ? -1 : 1);
+    cv = i == gl / kRows ? r : cv;
+  }
+  if (cv != 0 || plen <= 4 * kParts) return cv;
+  for (int j = 4 * kParts; j < plen; ++j) {
+    const int64_t idx = (int64_t)own + j;
+    const int32_t t = idx < n ? corpus[idx] : -1;
+    const int32_t pj = pat_at(j);
+    if (t != pj) return t < pj ? -1 : 1;
+  }
+  return 0;
+}
+
 // Exact lower bound (first rank with cmp >= 0) and upper bound (first rank
 // with cmp > 0) of one pattern.  Called by all G lanes of an aligned group
 // with identical arguments; returns the bounds on every lane of the group.
@@ -184,7 +255,9 @@ __device__ __forceinline__ int cmp_probes_key(
 // one bound left, or the bounds split), so each lane's probe and both
 // bounds' updates are computed for every phase with selects: no phase
 // branches for the wave to run one after another.
-template <int G, class PatFn>
+// kCorpusOct: without keys, compare by lane octets (cmp_probes_corpus);
+// more registers, so the step kernels leave it off.
+template <int G, bool kCorpusOct = false, class PatFn>
 __device__ __forceinline__ void kary_bounds(
     const int32_t* __restrict__ sa, const int32_t* __restrict__ corpus,
     int64_t n, const int32_t* __restrict__ keys, int kw, PatFn pat_at,
@@ -198,7 +271,8 @@ __device__ __forceinline__ void kary_bounds(
   const int gbase = ln - gl;
   constexpr bool kCoop = G % 8 == 0;  // rows read by lane octets
   int32_t pt[kCoop ? 4 : 32];
-  if (keys) {
+  static_assert(!kCorpusOct || kCoop, "octets");
+  if (keys || kCorpusOct) {
     // cooperative: pattern tokens 4 * (gl % 8) .. + 3; else all of them
     const int j0 = kCoop ? 4 * (gl % 8) : 0;
 #pragma unroll
@@ -223,7 +297,9 @@ __device__ __forceinline__ void kary_bounds(
                               (uint32_t)(kq + 1) * c);
     };
     int cv;
-    if constexpr (kCoop) {
+    if constexpr (kCorpusOct) {
+      cv = cmp_probes_corpus<G>(sa, corpus, n, probe_of, pt, pat_at, plen);
+    } else if constexpr (kCoop) {
       cv = keys ? cmp_probes_key<G>(keys, kw, sa, corpus, n, probe_of, pt,
                                     pat_at, plen)
                 : cmp_suffix(sa, corpus, n, probe_of(gl), pat_at, plen);

@@ -270,6 +270,36 @@ def _rand_expand(rng, b, r, k, vocab=9):
     return cont.astype(I32), occ, cap
 
 
+@pytest.mark.parametrize("n", [1, 2, 37, 3000])
+@pytest.mark.parametrize("width", [1, 4, 31, 32, 33, 70])
+def test_sa_search_widths_and_batches(gpu, n, width):
+    """Patterns shorter and longer than the 32 tokens an octet compares,
+    running past the end of the corpus, on both lane counts (up to 8192
+    patterns and past it)."""
+    from suffixgpu_amd import kernels
+    rng = np.random.default_rng(n * 100 + width)
+    corpus = rng.integers(0, 2, size=n).astype(I32)
+    corpus[n // 2:] = corpus[:n - n // 2]  # long repeats
+    sa = o_build_sa(corpus)
+    b = 40
+    pat = np.full((b, width), -1, I32)
+    plen = rng.integers(0, width + 1, size=b)
+    for i in range(b):
+        st = rng.integers(0, n)
+        seg = corpus[st:st + plen[i]]
+        pat[i, :seg.shape[0]] = seg
+        pat[i, seg.shape[0]:plen[i]] = rng.integers(0, 2)
+        if i % 4 == 0 and plen[i]:
+            pat[i, plen[i] - 1] = rng.integers(-1, 3)
+    es, ee = o_search(sa, corpus, pat, plen)
+    for rows in (b, 8192, 8193):
+        rep = np.arange(rows) % b
+        lo, hi = kernels.sa_search(T(sa.astype(I32), gpu), T(corpus, gpu),
+                                   T(pat[rep], gpu), T(plen[rep], gpu))
+        np.testing.assert_array_equal(N(lo), es[rep])
+        np.testing.assert_array_equal(N(hi), ee[rep])
+
+
 @pytest.mark.parametrize("r", [1, 4, 30, 128, 256, 700])
 @pytest.mark.parametrize("minp", [0.0, 0.1])
 def test_expand_chain(gpu, r, minp):
