@@ -217,6 +217,20 @@ int sfx_propose_step(const sfx_params* p, const sfx_index* index,
                      void* workspace, size_t workspace_bytes,
                      hipStream_t stream);
 
+/* The same step with scratch for rows that do not fit a compute unit's LDS
+ * (about 26,000 tokens at the defaults): sfx_row_scratch_size() bytes (0:
+ * the rows need none), 16-byte aligned, never initialised, dead after the
+ * call's work on `stream` -- a launch before the step's spreads the match
+ * of every row over the chip.  With less scratch, or none, one workgroup
+ * streams each such row, as sfx_propose_step does; the results are equal. */
+size_t sfx_row_scratch_size(const sfx_params* p, int64_t batch, int64_t seq);
+int sfx_propose_step_rows(const sfx_params* p, const sfx_index* index,
+                          const sfx_batch* batch, int32_t* draft,
+                          int32_t* num_valid, int32_t* new_counts,
+                          void* workspace, size_t workspace_bytes,
+                          void* row_scratch, size_t row_scratch_bytes,
+                          hipStream_t stream);
+
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): sfx_propose_step with no workspace argument.  The

@@ -124,6 +124,13 @@ SIGNATURES = {
                                  ctypes.POINTER(SfxIndex),
                                  ctypes.POINTER(SfxBatch), c_p, c_p, c_p,
                                  c_p, ctypes.c_size_t, c_p]),
+    "sfx_row_scratch_size": (ctypes.c_size_t,
+                             [ctypes.POINTER(SfxParams), c_i64, c_i64]),
+    "sfx_propose_step_rows": (c_i32, [ctypes.POINTER(SfxParams),
+                                      ctypes.POINTER(SfxIndex),
+                                      ctypes.POINTER(SfxBatch), c_p, c_p,
+                                      c_p, c_p, ctypes.c_size_t, c_p,
+                                      ctypes.c_size_t, c_p]),
     "sfx_propose_step_noalloc": (c_i32, [ctypes.POINTER(SfxParams),
                                          ctypes.POINTER(SfxIndex),
                                          ctypes.POINTER(SfxBatch), c_p, c_p,

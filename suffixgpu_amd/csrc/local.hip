@@ -66,6 +66,12 @@ size_t local_lds_bytes(const sfx_params& p, int64_t S, int chunk,
                    : layout_bytes(p, S, chunk, nthreads, mb_full);
 }
 
+size_t split_lds_bytes(const sfx_params& p) {
+  return (size_t)split_layout(p.max_pattern_len, p.num_thresholds,
+                              p.max_occurrences, p.k, kLocalThreads / kWave)
+      .total;
+}
+
 int launch_local_step(LocalArgs a, hipStream_t stream) {
   a.chunk = local_chunk(a.p, a.bt.seq, kMaxLds, kWideThreads, &a.mb_full);
   if (a.chunk < 0) return -1;

@@ -8,6 +8,11 @@
 
 namespace sfx {
 
+// How the local role reads its row (a template argument of the step).
+constexpr int kRowLds = 0;     // whole in LDS
+constexpr int kRowStream = 1;  // in HBM, streamed through LDS in chunks
+constexpr int kRowSplit = 2;   // matched by an earlier launch, see below
+
 enum LocalMode { kLocalGather = 0, kLocalForward = 1, kLocalStep = 2 };
 
 struct LocalArgs {
@@ -27,11 +32,12 @@ struct LocalArgs {
   StepWs ws;
   int chunk;  // 0: the whole row is staged in LDS; else streamed in chunks
   int mb_full;  // streamed: LDS holds the match lengths of the whole row
+  RowScratch rs;  // split rows: what the match launch left for the step
 };
 
 struct LocalLayout {
   int row, mb, pat, hist, cand, found, thr, scan, occ, A, H, chain, nv,
-      score, misc, total;
+      score, misc, offs, total;
 };
 
 __host__ __device__ inline int lds_take(int& off, int bytes) {
@@ -57,13 +63,15 @@ __host__ __device__ inline int stream_halo(int P) { return (P + 3) & ~3; }
 __host__ __device__ inline LocalLayout local_layout(int S, int P, int C,
                                                     int R, int K, int nwaves,
                                                     int chunk = 0,
-                                                    int mb_full = 0) {
+                                                    int mb_full = 0,
+                                                    int offs = 0) {
   const int nthreads = nwaves * kWave;
   const int span = chunk > 0 && !mb_full ? chunk : S;
   LocalLayout L;
   int off = 0;
   L.row = lds_take(off, (chunk > 0 ? chunk + stream_halo(P) : S) * 4);
   L.mb = lds_take(off, mb_bytes(span, nthreads));
+  L.offs = lds_take(off, offs);
   L.pat = lds_take(off, P * 4);
   L.hist = lds_take(off, (P + 1) * 4);
   L.cand = lds_take(off, C * 4);
@@ -81,6 +89,16 @@ __host__ __device__ inline LocalLayout local_layout(int S, int P, int C,
   return L;
 }
 
+// A split row's layout: no row and no match lengths, but per candidate the
+// output offsets of kOffsParts parts (an odd stride: the lanes of a wave
+// read one part's offsets of all candidates).
+constexpr int kOffsParts = kWave;
+constexpr int kOffsStride = kOffsParts + 1;
+__host__ __device__ inline LocalLayout split_layout(int P, int C, int R,
+                                                    int K, int nwaves) {
+  return local_layout(0, P, C, R, K, nwaves, 0, 0, C * kOffsStride * 4);
+}
+
 constexpr int kLocalThreads = 512;
 // The local-only decode step over rows of kWideMinSeq tokens or more runs
 // one 1024-thread workgroup per row: the row scans (match lengths,
@@ -91,6 +109,219 @@ constexpr int kLocalThreads = 512;
 // B <= 128 the same.
 constexpr int kWideThreads = 1024;
 constexpr int64_t kWideMinSeq = 8192;
+
+// Candidates: thr-th largest match_back = largest L with #{mb >= L} >=
+// thr; zero below min_match_len or when masked; adjacent duplicates
+// zeroed (local_matcher.py:134-157).  Called by wave 0: suffix sums of the
+// histogram (kCounts: hist[L] holds #{mb >= L} already), then one ballot
+// per threshold (#{mb >= L} is monotone in L, so the largest qualifying L
+// is the number of qualifying L).
+template <bool kCounts = false>
+__device__ __forceinline__ void local_candidates(const sfx_params& p, int S,
+                                                 const RowState& st,
+                                                 int32_t* hist,
+                                                 const int32_t* thr_lds,
+                                                 int32_t* cand) {
+  const int ln = lane_id();
+  const int P = p.max_pattern_len;
+  const int C = p.num_thresholds;
+  // P <= 64: lane ln holds #{mb >= P - ln} in a register (one DPP scan);
+  // longer patterns keep the suffix counts in hist[].
+  const bool in_reg = P <= kWave;
+  int sfx = 0;
+  if (in_reg) {
+    const int Lv = P - ln;
+    const uint32_t x = Lv >= 1 ? (uint32_t)hist[Lv] : 0u;
+    sfx = (int)(kCounts ? x : wave_incl_scan(x));
+  }
+  int carry = 0;
+  for (int top = in_reg || kCounts ? 0 : P; top >= 1; top -= kWave) {
+    const int Lv = top - ln;
+    int x = Lv >= 1 ? hist[Lv] : 0;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int y = __shfl_up(x, o);
+      if (ln >= o) x += y;
+    }
+    x += carry;
+    if (Lv >= 1) hist[Lv] = x;
+    carry = __shfl(x, kWave - 1);
+  }
+  wave_lds_sync();
+  // Lane c holds threshold c, copied to LDS at the start of the block
+  // (a varying index into the kernel arguments is a vector load from the
+  // argument segment in device memory; issued there, its latency hides
+  // behind the row staging).
+  const int thr_l = ln < C ? thr_lds[ln] : (int)0x80000000;
+  if (in_reg) {
+    // Eight thresholds per step, unrolled: each takes one ballot, and the
+    // min_match_len, mask and duplicate rules are scalar selects, with no
+    // branch per threshold.  A threshold above S qualifies no L.
+    const int mml = p.min_match_len;
+    const bool live = ln < P;
+    int prev_raw = -1;
+    for (int c0 = 0; c0 < C; c0 += 8) {
+      int outv = 0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int thr = __builtin_amdgcn_readlane(thr_l, c0 + j);
+        const int t = thr < 1 ? 1 : thr;
+        int v = popc(ballot(live && sfx >= t));
+        if (!(thr <= S && v >= mml && st.mask)) v = 0;
+        const int raw = v;
+        if (c0 + j > 0 && raw == prev_raw) v = 0;
+        prev_raw = raw;
+        outv = ln == j ? v : outv;
+      }
+      if (ln < 8 && c0 + ln < C) cand[c0 + ln] = outv;
+    }
+  } else {
+    const int maxthr = (int)(wave_all_max((uint32_t)thr_l ^ 0x80000000u) ^
+                             0x80000000u);
+    const int w = min(maxthr, S);
+    int prev_raw = -1;
+    for (int c = 0; c < C; ++c) {
+      const int thr = __builtin_amdgcn_readlane(thr_l, c);
+      int v = 0;
+      if (thr <= w) {
+        const int t = thr < 1 ? 1 : thr;
+        for (int base = 1; base <= P; base += kWave) {
+          const int Lv = base + ln;
+          v += popc(ballot(Lv <= P && hist[Lv] >= t));
+        }
+      }
+      if (!(v >= p.min_match_len && st.mask)) v = 0;
+      const int raw = v;
+      if (c > 0 && raw == prev_raw) v = 0;
+      prev_raw = raw;
+      if (ln == 0) cand[c] = v;
+    }
+  }
+}
+
+// From the first R ends per candidate on: the gather outputs, or expansion,
+// the best candidate, and the draft or the handover to the final pick.
+template <int NT>
+__device__ __forceinline__ void local_finish(
+    const LocalArgs& a, unsigned char* smem, const LocalLayout& L, int b,
+    const RowState& st, const int32_t* src_row) {
+  constexpr int NW = NT / kWave;
+  const sfx_params& p = a.p;
+  const int tid = threadIdx.x;
+  const int wv = tid / kWave;
+  const int ln = tid % kWave;
+  const int S = (int)a.bt.seq;
+  const int C = p.num_thresholds;
+  const int R = p.max_occurrences;
+  const int K = p.k;
+  const int64_t q = st.q;
+  const int32_t* cand = (const int32_t*)(smem + L.cand);
+  const int32_t* found = (const int32_t*)(smem + L.found);
+  const int32_t* occ = (const int32_t*)(smem + L.occ);
+  int32_t* Abuf = (int32_t*)(smem + L.A);
+  int32_t* chain = (int32_t*)(smem + L.chain);
+  int32_t* res_nv = (int32_t*)(smem + L.nv);
+  float* res_score = (float*)(smem + L.score);
+  int* misc = (int*)(smem + L.misc);
+
+  SFX_TRACE_POINT(4);
+  if (a.mode == kLocalGather) {
+    for (int c = tid; c < C; c += NT) {
+      if (a.cand_out) a.cand_out[(int64_t)b * C + c] = cand[c];
+      if (a.occ_out) a.occ_out[(int64_t)b * C + c] = min(found[c], R);
+    }
+    if (a.cont_out) {
+      const int total = C * R * K;
+      int32_t* out = a.cont_out + (int64_t)b * total;
+      for (int e = tid; e < total; e += NT) {
+        const int c = e / (R * K);
+        const int r = (e / K) % R;
+        const int j = e % K;
+        int32_t v = -1;
+        if (r < min(found[c], R)) {
+          const int64_t idx = (int64_t)occ[c * R + r] + j;
+          if (idx < q) v = src_row[idx < S - 1 ? idx : S - 1];
+        }
+        out[e] = v;
+      }
+    }
+    return;
+  }
+
+  // One wave per candidate: majority-vote expansion from the LDS row (HBM
+  // when streamed).
+  for (int c = wv; c < C; c += NW) {
+    const int cv = cand[c];
+    const int64_t oc = cv > 0 ? (int64_t)min(found[c], R) : 0;
+    const int64_t cap = spec_cap(p, cv);
+    const int32_t* oc_list = occ + c * R;
+    auto cont_at = [&](int r, int d) -> int32_t {
+      const int64_t idx = (int64_t)oc_list[r] + d;
+      return idx < q ? src_row[idx < S - 1 ? idx : S - 1] : -1;
+    };
+    const ExpandResult er = expand_wave<false>(
+        cont_at, NoWeight(), R, oc, K, cap, p.min_token_prob, p.alpha,
+        Abuf + wv * ((R + 3) & ~3), nullptr,
+        (int32_t*)(smem + L.H) + wv * 2 * kHashSlots, chain + c * K);
+    if (ln == 0) {
+      res_nv[c] = er.nv;
+      res_score[c] = er.score;
+    }
+    if (c < 6) SFX_TRACE_WAVE(10 + c);
+  }
+  __syncthreads();
+
+  SFX_TRACE_POINT(5);
+  // select_local_best (local_matcher.py:245-263).
+  if (tid == 0) {
+    int best = 0;
+    float bkey = local_key(res_score[0], cand[0]);
+    for (int c = 1; c < C; ++c) {
+      const float key = local_key(res_score[c], cand[c]);
+      if (key > bkey) {
+        bkey = key;
+        best = c;
+      }
+    }
+    const int64_t cap = spec_cap(p, cand[best]);
+    const int64_t cap0 = cap > 0 ? cap : 0;
+    misc[0] = best;
+    misc[1] = (int)((int64_t)res_nv[best] < cap0 ? res_nv[best] : cap0);
+  }
+  __syncthreads();
+  const int best = misc[0];
+  const int emit = misc[1];
+  const int32_t* bchain = chain + best * K;
+
+  if (a.mode == kLocalForward) {
+    for (int j = tid; j < K; j += NT)
+      a.draft[(int64_t)b * K + j] = j < emit ? bchain[j] : -1;
+    if (tid == 0) {
+      a.num_valid[b] = emit;
+      if (a.len_out) a.len_out[b] = cand[best];
+      if (a.occ1_out)
+        a.occ1_out[b] = cand[best] > 0 ? min(found[best], R) : 0;
+      if (a.score_out) a.score_out[b] = res_score[best];
+    }
+    return;
+  }
+
+  // Decode step.
+  if (!a.global_on) {
+    for (int j = tid; j < K; j += NT)
+      a.draft[(int64_t)b * K + j] = j < emit ? bchain[j] : -1;
+    if (tid == 0) a.num_valid[b] = emit;
+    return;
+  }
+  for (int j = tid; j < K; j += NT)
+    ws_store(a.ws.l_chain + (int64_t)b * K + j, bchain[j]);
+  if (tid == 0) {
+    ws_store(a.ws.l_emit + b, emit);
+    ws_store(a.ws.l_score + b, res_score[best]);
+  }
+  if (block_arrive<false>(a.ws.pick + b, 3u, misc + 2))
+    final_pick(p, a.ws, b, a.draft, a.num_valid, misc + 4);
+}
 
 // kStream: the row stays in HBM.  match_back is computed over chunks of
 // a.chunk positions staged through LDS.  With a.mb_full the match lengths
@@ -124,11 +355,6 @@ __device__ __forceinline__ void local_body(const LocalArgs& a,
   int32_t* thr_lds = (int32_t*)(smem + L.thr);
   uint32_t* scan = (uint32_t*)(smem + L.scan);
   int32_t* occ = (int32_t*)(smem + L.occ);
-  int32_t* Abuf = (int32_t*)(smem + L.A);
-  int32_t* chain = (int32_t*)(smem + L.chain);
-  int32_t* res_nv = (int32_t*)(smem + L.nv);
-  float* res_score = (float*)(smem + L.score);
-  int* misc = (int*)(smem + L.misc);
 
   SFX_TRACE_POINT(0);
   if (tid < C) thr_lds[tid] = p.thresholds[tid];
@@ -335,84 +561,7 @@ __device__ __forceinline__ void local_body(const LocalArgs& a,
   }
 
   SFX_TRACE_POINT(2);
-  // Candidates: thr-th largest match_back = largest L with #{mb >= L} >=
-  // thr; zero below min_match_len or when masked; adjacent duplicates
-  // zeroed (local_matcher.py:134-157).  Wave 0: suffix sums of the
-  // histogram, then one ballot per threshold (#{mb >= L} is monotone in L,
-  // so the largest qualifying L is the number of qualifying L).
-  if (wv == 0) {
-    // P <= 64: lane ln holds #{mb >= P - ln} in a register (one DPP scan);
-    // longer patterns keep the suffix counts in hist[].
-    const bool in_reg = P <= kWave;
-    int sfx = 0;
-    if (in_reg) {
-      const int Lv = P - ln;
-      sfx = (int)wave_incl_scan(Lv >= 1 ? (uint32_t)hist[Lv] : 0u);
-    }
-    int carry = 0;
-    for (int top = in_reg ? 0 : P; top >= 1; top -= kWave) {
-      const int Lv = top - ln;
-      int x = Lv >= 1 ? hist[Lv] : 0;
-#pragma unroll
-      for (int o = 1; o < kWave; o <<= 1) {
-        const int y = __shfl_up(x, o);
-        if (ln >= o) x += y;
-      }
-      x += carry;
-      if (Lv >= 1) hist[Lv] = x;
-      carry = __shfl(x, kWave - 1);
-    }
-    wave_lds_sync();
-    // Lane c holds threshold c, copied to LDS at the start of the block
-    // (a varying index into the kernel arguments is a vector load from the
-    // argument segment in device memory; issued there, its latency hides
-    // behind the row staging).
-    const int thr_l = ln < C ? thr_lds[ln] : (int)0x80000000;
-    if (in_reg) {
-      // Eight thresholds per step, unrolled: each takes one ballot, and the
-      // min_match_len, mask and duplicate rules are scalar selects, with no
-      // branch per threshold.  A threshold above S qualifies no L.
-      const int mml = p.min_match_len;
-      const bool live = ln < P;
-      int prev_raw = -1;
-      for (int c0 = 0; c0 < C; c0 += 8) {
-        int outv = 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int thr = __builtin_amdgcn_readlane(thr_l, c0 + j);
-          const int t = thr < 1 ? 1 : thr;
-          int v = popc(ballot(live && sfx >= t));
-          if (!(thr <= S && v >= mml && st.mask)) v = 0;
-          const int raw = v;
-          if (c0 + j > 0 && raw == prev_raw) v = 0;
-          prev_raw = raw;
-          outv = ln == j ? v : outv;
-        }
-        if (ln < 8 && c0 + ln < C) cand[c0 + ln] = outv;
-      }
-    } else {
-      const int maxthr = (int)(wave_all_max((uint32_t)thr_l ^ 0x80000000u) ^
-                               0x80000000u);
-      const int w = min(maxthr, S);
-      int prev_raw = -1;
-      for (int c = 0; c < C; ++c) {
-        const int thr = __builtin_amdgcn_readlane(thr_l, c);
-        int v = 0;
-        if (thr <= w) {
-          const int t = thr < 1 ? 1 : thr;
-          for (int base = 1; base <= P; base += kWave) {
-            const int Lv = base + ln;
-            v += popc(ballot(Lv <= P && hist[Lv] >= t));
-          }
-        }
-        if (!(v >= p.min_match_len && st.mask)) v = 0;
-        const int raw = v;
-        if (c > 0 && raw == prev_raw) v = 0;
-        prev_raw = raw;
-        if (ln == 0) cand[c] = v;
-      }
-    }
-  }
+  if (wv == 0) local_candidates(p, S, st, hist, thr_lds, cand);
   __syncthreads();
 
   SFX_TRACE_POINT(3);
@@ -447,108 +596,147 @@ __device__ __forceinline__ void local_body(const LocalArgs& a,
     }
   }
 
-  SFX_TRACE_POINT(4);
-  if (a.mode == kLocalGather) {
-    for (int c = tid; c < C; c += NT) {
-      if (a.cand_out) a.cand_out[(int64_t)b * C + c] = cand[c];
-      if (a.occ_out) a.occ_out[(int64_t)b * C + c] = min(found[c], R);
+  local_finish<NT>(a, smem, L, b, st, src_row);
+}
+
+// The local role of a split row: k_row_match (row_match.hip) has applied the
+// step's scatter and left the row's match lengths, and per length and part
+// of kRowPart positions the number of ends matching at least that long.
+// What remains is short and reads little: the counts' totals give the
+// candidates; a scan of a candidate's counts over the parts gives every
+// part's first output slot, so each wave takes parts of its own and reads
+// only those that hold one of the first R ends of some candidate.  The
+// expansion reads continuations from HBM.
+template <int NT>
+__device__ __forceinline__ void local_split_body(const LocalArgs& a,
+                                                 unsigned char* smem, int b) {
+  constexpr int NW = NT / kWave;
+  const sfx_params& p = a.p;
+  const int tid = threadIdx.x;
+  const int wv = tid / kWave;
+  const int ln = tid % kWave;
+  const int S = (int)a.bt.seq;
+  const int P = p.max_pattern_len;
+  const int C = p.num_thresholds;
+  const int R = p.max_occurrences;
+  const int K = p.k;
+  const LocalLayout L = split_layout(P, C, R, K, NW);
+  int32_t* hist = (int32_t*)(smem + L.hist);
+  int32_t* cand = (int32_t*)(smem + L.cand);
+  int32_t* found = (int32_t*)(smem + L.found);
+  int32_t* thr_lds = (int32_t*)(smem + L.thr);
+  int32_t* occ = (int32_t*)(smem + L.occ);
+  int32_t* offs = (int32_t*)(smem + L.offs);
+
+  SFX_TRACE_POINT(0);
+  if (tid < C) {
+    thr_lds[tid] = p.thresholds[tid];
+    found[tid] = 0;
+  }
+  const RowState st = row_state(a.bt, b);
+  if (!st.mask) {
+    for (int j = tid; j < K; j += NT) a.draft[(int64_t)b * K + j] = -1;
+    if (tid == 0) a.num_valid[b] = 0;
+    return;
+  }
+  const int qe = (int)(st.q < 0 ? 0 : (st.q < S ? st.q : S));
+  // one row's counts and lengths are less than 2^32 bytes: 32-bit offsets
+  const uint32_t nparts = (uint32_t)a.rs.parts;
+  const uint8_t* mb = a.rs.mb + (int64_t)b * nparts * kRowPart;
+  const int np = (qe + kRowPart - 1) / kRowPart;  // parts with ends
+  const int32_t* cnt = a.rs.count + (int64_t)b * (P + 1) * nparts;
+
+  SFX_TRACE_POINT(1);
+  // #{mb >= len} of the row: a wave per length, four lengths in flight.
+  for (int l0 = 1 + wv; l0 <= P; l0 += 4 * NW) {
+    uint32_t sum[4] = {0, 0, 0, 0};
+    for (int k = ln; k < np; k += kWave) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int len = l0 + u * NW;
+        if (len <= P) sum[u] += (uint32_t)cnt[(uint32_t)len * nparts + k];
+      }
     }
-    if (a.cont_out) {
-      const int total = C * R * K;
-      int32_t* out = a.cont_out + (int64_t)b * total;
-      for (int e = tid; e < total; e += NT) {
-        const int c = e / (R * K);
-        const int r = (e / K) % R;
-        const int j = e % K;
-        int32_t v = -1;
-        if (r < min(found[c], R)) {
-          const int64_t idx = (int64_t)occ[c * R + r] + j;
-          if (idx < q) v = src_row[idx < S - 1 ? idx : S - 1];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const uint32_t all = wave_incl_scan(sum[u]);
+      if (ln == kWave - 1 && l0 + u * NW <= P) hist[l0 + u * NW] = (int)all;
+    }
+  }
+  __syncthreads();
+  SFX_TRACE_POINT(2);
+  if (wv == 0) local_candidates<true>(p, S, st, hist, thr_lds, cand);
+  __syncthreads();
+
+  SFX_TRACE_POINT(3);
+  for (int k0 = 0; k0 < np; k0 += kOffsParts) {
+    // candidate c's first slot in part k0 + lane, -1 where the part holds
+    // none of its first R ends
+    for (int c = wv; c < C; c += NW) {
+      const int len = cand[c];
+      const uint32_t n = len > 0 && k0 + ln < np
+                             ? (uint32_t)cnt[(uint32_t)len * nparts + k0 + ln]
+                             : 0u;
+      const uint32_t kept = (uint32_t)found[c];
+      const uint32_t end = kept + wave_incl_scan(n);
+      offs[c * kOffsStride + ln] =
+          n > 0 && end - n < (uint32_t)R ? (int)(end - n) : -1;
+      if (ln == kWave - 1) found[c] = (int)min(end, (uint32_t)R);
+    }
+    __syncthreads();
+    const int kn = min(kOffsParts, np - k0);
+    for (int k = wv; k < kn; k += NW) {
+      const int off = ln < C ? offs[ln * kOffsStride + k] : -1;
+      uint64_t open = ballot(off >= 0);
+      if (!open) continue;
+      // the part's match lengths, 64 consecutive ones per lane
+      constexpr int kWords = kRowPart / kWave / 16;
+      const uint32_t at = (uint32_t)((k0 + k) * kRowPart + ln * 16 * kWords);
+      const uint4* src = reinterpret_cast<const uint4*>(mb + at);
+      for (; open; open &= open - 1) {
+        const int c = __builtin_ctzll(open);
+        const ByteGe ge = byte_ge_init(cand[c]);
+        uint32_t mine = 0;
+#pragma unroll
+        for (int u = 0; u < kWords; ++u) {
+          const uint4 w = src[u];
+          mine += __popc(bytes_ge(w.x, ge)) + __popc(bytes_ge(w.y, ge)) +
+                  __popc(bytes_ge(w.z, ge)) + __popc(bytes_ge(w.w, ge));
         }
-        out[e] = v;
+        uint32_t slot = (uint32_t)__builtin_amdgcn_readlane(off, c) +
+                        wave_incl_scan(mine) - mine;
+        if (mine > 0 && slot < (uint32_t)R) {
+#pragma unroll
+          for (int u = 0; u < kWords; ++u) {
+            const uint4 w = src[u];
+            const uint32_t v[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              for (uint32_t m = bytes_ge(v[e], ge); m; m &= m - 1) {
+                if (slot < (uint32_t)R)
+                  occ[c * R + slot] = (int32_t)at + 16 * u + 4 * e +
+                                      (__builtin_ctz(m) >> 3);
+                ++slot;
+              }
+            }
+          }
+        }
       }
     }
-    return;
+    __syncthreads();
+    bool more = false;
+    for (int c = 0; c < C; ++c) more |= cand[c] > 0 && found[c] < R;
+    if (!more) break;
+    __syncthreads();  // found is rewritten below
   }
-
-  // One wave per candidate: majority-vote expansion from the LDS row (HBM
-  // when streamed).
-  for (int c = wv; c < C; c += NW) {
-    const int cv = cand[c];
-    const int64_t oc = cv > 0 ? (int64_t)min(found[c], R) : 0;
-    const int64_t cap = spec_cap(p, cv);
-    const int32_t* oc_list = occ + c * R;
-    auto cont_at = [&](int r, int d) -> int32_t {
-      const int64_t idx = (int64_t)oc_list[r] + d;
-      return idx < q ? src_row[idx < S - 1 ? idx : S - 1] : -1;
-    };
-    const ExpandResult er = expand_wave<false>(
-        cont_at, NoWeight(), R, oc, K, cap, p.min_token_prob, p.alpha,
-        Abuf + wv * ((R + 3) & ~3), nullptr,
-        (int32_t*)(smem + L.H) + wv * 2 * kHashSlots, chain + c * K);
-    if (ln == 0) {
-      res_nv[c] = er.nv;
-      res_score[c] = er.score;
-    }
-    if (c < 6) SFX_TRACE_WAVE(10 + c);
-  }
-  __syncthreads();
-
-  SFX_TRACE_POINT(5);
-  // select_local_best (local_matcher.py:245-263).
-  if (tid == 0) {
-    int best = 0;
-    float bkey = local_key(res_score[0], cand[0]);
-    for (int c = 1; c < C; ++c) {
-      const float key = local_key(res_score[c], cand[c]);
-      if (key > bkey) {
-        bkey = key;
-        best = c;
-      }
-    }
-    const int64_t cap = spec_cap(p, cand[best]);
-    const int64_t cap0 = cap > 0 ? cap : 0;
-    misc[0] = best;
-    misc[1] = (int)((int64_t)res_nv[best] < cap0 ? res_nv[best] : cap0);
-  }
-  __syncthreads();
-  const int best = misc[0];
-  const int emit = misc[1];
-  const int32_t* bchain = chain + best * K;
-
-  if (a.mode == kLocalForward) {
-    for (int j = tid; j < K; j += NT)
-      a.draft[(int64_t)b * K + j] = j < emit ? bchain[j] : -1;
-    if (tid == 0) {
-      a.num_valid[b] = emit;
-      if (a.len_out) a.len_out[b] = cand[best];
-      if (a.occ1_out)
-        a.occ1_out[b] = cand[best] > 0 ? min(found[best], R) : 0;
-      if (a.score_out) a.score_out[b] = res_score[best];
-    }
-    return;
-  }
-
-  // Decode step.
-  if (!a.global_on) {
-    for (int j = tid; j < K; j += NT)
-      a.draft[(int64_t)b * K + j] = j < emit ? bchain[j] : -1;
-    if (tid == 0) a.num_valid[b] = emit;
-    return;
-  }
-  for (int j = tid; j < K; j += NT)
-    ws_store(a.ws.l_chain + (int64_t)b * K + j, bchain[j]);
-  if (tid == 0) {
-    ws_store(a.ws.l_emit + b, emit);
-    ws_store(a.ws.l_score + b, res_score[best]);
-  }
-  if (block_arrive<false>(a.ws.pick + b, 3u, misc + 2))
-    final_pick(p, a.ws, b, a.draft, a.num_valid, misc + 4);
+  local_finish<NT>(a, smem, L, b, st, a.bt.tokens + (int64_t)b * S);
 }
 
 // The local-only decode step with kWideThreads per row (local.hip); -1
 // when its layout does not fit a CU's LDS (the caller keeps the fused
 // step's 512-thread form).
 int launch_local_step(LocalArgs a, hipStream_t stream);
+// The match launch of split rows (row_match.hip).
+int launch_row_match(const LocalArgs& a, hipStream_t stream);
 
 }  // namespace sfx

@@ -26,11 +26,20 @@ struct StepArgs {
   int global_on;
 };
 
-template <bool kStream>
+template <int kRow>
+__device__ __forceinline__ void step_local(const LocalArgs& a,
+                                           unsigned char* smem, int b) {
+  if constexpr (kRow == kRowSplit)
+    local_split_body<kLocalThreads>(a, smem, b);
+  else
+    local_body<kRow == kRowStream>(a, smem, b);
+}
+
+template <int kRow>
 __global__ __launch_bounds__(kGlobalThreads) void k_step(StepArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   if (!a.global_on) {
-    local_body<kStream>(a.l, smem, blockIdx.x);
+    step_local<kRow>(a.l, smem, blockIdx.x);
     return;
   }
   // Blocks are ordered by role (role 0: SA, 1..dparts: delta parts,
@@ -51,9 +60,9 @@ __global__ __launch_bounds__(kGlobalThreads) void k_step(StepArgs a) {
   const int b = (int)(blockIdx.x % B);
   const int role = slot == 0 ? per - 1 : (slot == per - 1 ? 0 : slot);
   if (role == per - 1)
-    local_body<kStream>(a.l, smem, b);
+    step_local<kRow>(a.l, smem, b);
   else
-    global_body<!kStream>(a.g, smem, b, role);
+    global_body<kRow != kRowStream>(a.g, smem, b, role);
 }
 
 }  // namespace sfx
@@ -86,11 +95,33 @@ static __global__ __launch_bounds__(256) void k_zero_words(uint32_t* w,
 
 namespace {
 
+template <int kRow>
+int launch_rows(const StepArgs& a, unsigned blocks, size_t lds,
+                hipStream_t stream) {
+  static std::atomic<uint64_t> lds_opt{0};
+  allow_max_lds((const void*)k_step<kRow>, lds_opt);
+  hipLaunchKernelGGL(k_step<kRow>, dim3(blocks), dim3(kGlobalThreads), lds,
+                     stream, a);
+  return (int)hipGetLastError();
+}
+
+// Split rows: the bytes of row scratch, 0 for rows that fit LDS whole (or
+// a layout or grid that does not fit).
+size_t split_scratch_bytes(const sfx_params& p, int64_t batch, int64_t seq) {
+  if (batch < 1 || batch > 65535 || local_chunk(p, seq) <= 0 ||
+      split_lds_bytes(p) > kMaxLds)
+    return 0;
+  return row_scratch_layout(p.max_pattern_len, batch, seq, nullptr, nullptr);
+}
+
 // The fused step over `workspace` laid out with counter arrays of
-// `counter_rows` rows (-1: the batch size).
+// `counter_rows` rows (-1: the batch size).  Rows that do not fit LDS whole
+// are split over the chip when `row_scratch` holds the match launch's
+// results, else streamed.
 int launch_step(const sfx_params* p, const sfx_index* ix, const sfx_batch* bt,
                 int32_t* draft, int32_t* num_valid, int32_t* new_counts,
                 void* workspace, size_t workspace_bytes, int64_t counter_rows,
+                void* row_scratch, size_t row_scratch_bytes,
                 hipStream_t stream) {
   if (!p || !bt || !draft || !num_valid) return SFX_EINVAL;
   int rc = check_local(*p, *bt);
@@ -106,7 +137,11 @@ int launch_step(const sfx_params* p, const sfx_index* ix, const sfx_batch* bt,
   a.l.draft = draft;
   a.l.num_valid = num_valid;
   a.l.new_counts = new_counts;
-  if (!global_on && bt->seq >= kWideMinSeq) {
+  const size_t split_need = split_scratch_bytes(*p, bt->batch, bt->seq);
+  const bool split = split_need > 0 && row_scratch &&
+                     row_scratch_bytes >= split_need;
+  if (split && ((uintptr_t)row_scratch & 15u) != 0) return SFX_EINVAL;
+  if (!global_on && !split && bt->seq >= kWideMinSeq) {
     // local-only rows of 8192 tokens or more: one 1024-thread workgroup
     // per row when its layout fits
     rc = launch_local_step(a.l, stream);
@@ -122,7 +157,8 @@ int launch_step(const sfx_params* p, const sfx_index* ix, const sfx_batch* bt,
   size_t cap = kMaxLds;
   auto fits = [&](size_t c) {
     size_t glds = 0;
-    return local_chunk(*p, bt->seq, c) >= 0 &&
+    return (split ? split_lds_bytes(*p) <= c
+                  : local_chunk(*p, bt->seq, c) >= 0) &&
            (!global_on || merge_waves_for(*p, *ix, dparts, &glds, c) > 0);
   };
   const unsigned cus = (unsigned)device_cus();
@@ -130,10 +166,17 @@ int launch_step(const sfx_params* p, const sfx_index* ix, const sfx_batch* bt,
     cap = kThirdLds;
   else if (blocks > cus && fits(kHalfLds))
     cap = kHalfLds;
-  a.l.chunk = local_chunk(*p, bt->seq, cap, kLocalThreadsDefault,
-                          &a.l.mb_full);
-  size_t lds = local_lds_bytes(*p, bt->seq, a.l.chunk, kLocalThreadsDefault,
-                               a.l.mb_full);
+  size_t lds = 0;
+  if (split) {
+    row_scratch_layout(p->max_pattern_len, bt->batch, bt->seq, row_scratch,
+                       &a.l.rs);
+    lds = split_lds_bytes(*p);
+  } else {
+    a.l.chunk = local_chunk(*p, bt->seq, cap, kLocalThreadsDefault,
+                            &a.l.mb_full);
+    lds = local_lds_bytes(*p, bt->seq, a.l.chunk, kLocalThreadsDefault,
+                          a.l.mb_full);
+  }
   if (global_on) {
     rc = check_global(*p, *ix, bt->batch);
     if (rc) return rc;
@@ -171,18 +214,13 @@ int launch_step(const sfx_params* p, const sfx_index* ix, const sfx_batch* bt,
   if (lds > kMaxLds) return SFX_EINVAL;
   if (bt->batch == 0) return 0;
   lds = one_per_cu_lds(lds, blocks);
-  if (a.l.chunk == 0) {
-    static std::atomic<uint64_t> lds_opt{0};
-    allow_max_lds((const void*)k_step<false>, lds_opt);
-    hipLaunchKernelGGL(k_step<false>, dim3(blocks), dim3(kGlobalThreads), lds,
-                       stream, a);
-  } else {
-    static std::atomic<uint64_t> lds_opt{0};
-    allow_max_lds((const void*)k_step<true>, lds_opt);
-    hipLaunchKernelGGL(k_step<true>, dim3(blocks), dim3(kGlobalThreads), lds,
-                       stream, a);
+  if (split) {
+    rc = launch_row_match(a.l, stream);
+    if (rc) return rc;
+    return launch_rows<kRowSplit>(a, blocks, lds, stream);
   }
-  return (int)hipGetLastError();
+  return a.l.chunk == 0 ? launch_rows<kRowLds>(a, blocks, lds, stream)
+                        : launch_rows<kRowStream>(a, blocks, lds, stream);
 }
 
 constexpr int64_t kScratchRows = SFX_NOALLOC_MAX_ROWS;
@@ -226,7 +264,29 @@ extern "C" int sfx_propose_step(const sfx_params* p, const sfx_index* ix,
                                 void* workspace, size_t workspace_bytes,
                                 hipStream_t stream) {
   return launch_step(p, ix, bt, draft, num_valid, new_counts, workspace,
-                     workspace_bytes, -1, stream);
+                     workspace_bytes, -1, nullptr, 0, stream);
+}
+
+extern "C" size_t sfx_row_scratch_size(const sfx_params* p, int64_t batch,
+                                       int64_t seq) {
+  sfx_batch bt = {};
+  bt.batch = batch;
+  bt.seq = seq;
+  // any address: check_local takes the sizes into account and reads nothing
+  bt.tokens = reinterpret_cast<int32_t*>(sizeof(int32_t));
+  bt.num_tokens = bt.tokens;
+  if (!p || check_local(*p, bt)) return 0;
+  return split_scratch_bytes(*p, batch, seq);
+}
+
+extern "C" int sfx_propose_step_rows(
+    const sfx_params* p, const sfx_index* ix, const sfx_batch* bt,
+    int32_t* draft, int32_t* num_valid, int32_t* new_counts, void* workspace,
+    size_t workspace_bytes, void* row_scratch, size_t row_scratch_bytes,
+    hipStream_t stream) {
+  return launch_step(p, ix, bt, draft, num_valid, new_counts, workspace,
+                     workspace_bytes, -1, row_scratch, row_scratch_bytes,
+                     stream);
 }
 
 extern "C" int sfx_propose_step_noalloc(const sfx_params* p,
@@ -238,7 +298,7 @@ extern "C" int sfx_propose_step_noalloc(const sfx_params* p,
   if (!p || !bt) return SFX_EINVAL;
   if (!ix)  // local-only steps use no workspace
     return launch_step(p, nullptr, bt, draft, num_valid, new_counts, nullptr,
-                       0, -1, stream);
+                       0, -1, nullptr, 0, stream);
   if (bt->batch < 0) return SFX_EINVAL;
   if (bt->batch > kScratchRows ||
       step_ws_layout(*p, bt->batch, ix->delta_capacity, nullptr, nullptr,
@@ -248,5 +308,6 @@ extern "C" int sfx_propose_step_noalloc(const sfx_params* p,
   const int rc = scratch_of_current_device(stream, &ws);
   if (rc) return rc;
   return launch_step(p, ix, bt, draft, num_valid, new_counts, ws,
-                     (size_t)SFX_NOALLOC_SCRATCH_BYTES, kScratchRows, stream);
+                     (size_t)SFX_NOALLOC_SCRATCH_BYTES, kScratchRows, nullptr,
+                     0, stream);
 }

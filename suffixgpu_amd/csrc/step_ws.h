@@ -92,6 +92,26 @@ __host__ __device__ inline uint32_t delta_bucket(int32_t t, int hbits) {
   return ((uint32_t)t * 0x9E3779B1u) >> (32 - hbits);
 }
 
+// Split rows: positions per part of the match launch, and its results.
+constexpr int kRowPart = 4096;
+struct RowScratch {
+  int64_t parts;   // per row: ceil(S / kRowPart)
+  uint8_t* mb;     // [B, parts * kRowPart] match lengths
+  int32_t* count;  // [B, P + 1, parts] ends of a part matching >= len
+};
+
+inline size_t row_scratch_layout(int P, int64_t B, int64_t S, void* base,
+                                 RowScratch* out) {
+  RowScratch r;
+  r.parts = (S + kRowPart - 1) / kRowPart;
+  char* c = (char*)base;
+  const size_t mb = (size_t)B * (size_t)r.parts * kRowPart;
+  r.mb = (uint8_t*)c;
+  r.count = (int32_t*)(c ? c + mb : nullptr);
+  if (out) *out = r;
+  return mb + (size_t)B * (size_t)(P + 1) * (size_t)r.parts * 4;
+}
+
 // Largest delta part (positions) whose match_back bytes stay in LDS;
 // longer parts use StepWs::d_mb.
 constexpr int64_t kDeltaMbLdsMax = 65540;

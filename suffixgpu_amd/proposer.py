@@ -5,7 +5,8 @@ propose_with_update, propose, poll, harvest_finished, harvest_rows,
 ingest_active, load_model).  Device tensors in and out, no host
 synchronisation on the step, static shapes: a step is one kernel launch on
 the current stream (local, SA-search and delta-scan workgroups per row), so
-``torch.cuda.graph`` captures it as a single node.
+``torch.cuda.graph`` captures it as a single node; rows too long for a
+compute unit's LDS take a second launch before it.
 
 Local candidates use support thresholds 2^0..2^(C-1); global candidates use
 length caps max(2, P >> i) for i < C-1 plus 2, deduplicated, descending
@@ -105,6 +106,16 @@ class SuffixGPUDrafter:
         # per-slot progress of ingest_active with device keys
         self._ingested_dev: torch.Tensor | None = None
         self._ws: dict[tuple, torch.Tensor] = {}
+        # Rows of this many tokens or more do not fit a CU's LDS (the need
+        # for scratch grows with the row): a step takes scratch for them.
+        lo, hi = 1, 1 << 30
+        while lo < hi:
+            mid = (lo + hi) // 2
+            if lib().sfx_row_scratch_size(self._params, 1, mid):
+                hi = mid
+            else:
+                lo = mid + 1
+        self._split_seq = lo
         if enable_global:
             self.global_index = GlobalIndex(
                 capacity=global_capacity, delta_capacity=delta_capacity,
@@ -205,7 +216,7 @@ class SuffixGPUDrafter:
         bt, keep = _lib.make_batch(tokens, num_tokens, sampled=sampled,
                                    valid_count=valid_cnt, mask=mask,
                                    limit=limit)
-        b = tokens.shape[0]
+        b, s = tokens.shape
         dev = tokens.device
         draft = torch.empty(b, self.k, dtype=torch.int32, device=dev)
         num_valid = torch.empty(b, dtype=torch.int32, device=dev)
@@ -215,20 +226,26 @@ class SuffixGPUDrafter:
             return draft, num_valid, new
         L = lib()
         cur = torch.cuda.current_stream(dev).cuda_stream
-        if self.global_index is None:
-            check(L.sfx_propose_step(self._params, None, bt,
-                                     draft.data_ptr(), num_valid.data_ptr(),
-                                     _lib.ptr(new), None, 0, cur),
-                  "propose")
-            del keep
-            return draft, num_valid, new
-        ws = self._workspace(b, cur)
-        rc = L.sfx_propose_step(self._params,
-                                self.global_index.index_struct(), bt,
-                                draft.data_ptr(), num_valid.data_ptr(),
-                                _lib.ptr(new), ws.data_ptr(), ws.numel(),
-                                cur)
-        if rc != 0:
+        ix = ws = None
+        nws = 0
+        if self.global_index is not None:
+            ws = self._workspace(b, cur)
+            nws = ws.numel()
+            ix = self.global_index.index_struct()
+        if s < self._split_seq:
+            rc = L.sfx_propose_step(self._params, ix, bt, draft.data_ptr(),
+                                    num_valid.data_ptr(), _lib.ptr(new),
+                                    _lib.ptr(ws), nws, cur)
+        else:
+            # scratch from the current stream's pool (in a capture, the
+            # graph's), dead once the step has run
+            rows = torch.empty(L.sfx_row_scratch_size(self._params, b, s),
+                               dtype=torch.uint8, device=dev)
+            rc = L.sfx_propose_step_rows(
+                self._params, ix, bt, draft.data_ptr(), num_valid.data_ptr(),
+                _lib.ptr(new), _lib.ptr(ws), nws, rows.data_ptr(),
+                rows.numel(), cur)
+        if rc != 0 and ws is not None:
             ws.zero_()  # never leave handover counters half set
         check(rc, "propose")
         del keep

@@ -374,3 +374,69 @@ def test_step_wave_grid_split_delta_vs_oracle(gpu, b):
     np.testing.assert_array_equal(N(draft), ed)
     np.testing.assert_array_equal(N(nv), env)
     assert (env > 0).sum() > b // 2
+
+
+def _rows_step(gpu, p, tokens, nt, sampled, mask, scratch):
+    """One local-only step through the C ABI, with or without row scratch."""
+    from suffixgpu_amd import _lib
+    L = _lib.lib()
+    b, s = tokens.shape
+    rows = T(tokens, gpu)
+    bt, keep = _lib.make_batch(
+        rows, T(nt, gpu), sampled=None if sampled is None else T(sampled, gpu),
+        mask=None if mask is None else T(mask, gpu), limit=s)
+    out = [torch.full((b, p.k), -9, dtype=torch.int32, device=gpu),
+           torch.full((b,), -9, dtype=torch.int32, device=gpu),
+           torch.full((b,), -9, dtype=torch.int32, device=gpu)]
+    n = int(L.sfx_row_scratch_size(p, b, s))
+    assert n > 0, "the rows fit LDS"
+    # whatever the memory held before must not matter
+    ws = torch.full((n,), 0x5b, dtype=torch.uint8, device=gpu)
+    cur = torch.cuda.current_stream().cuda_stream
+    rc = L.sfx_propose_step_rows(
+        p, None, bt, *[o.data_ptr() for o in out], None, 0,
+        ws.data_ptr() if scratch else None, n if scratch else 0, cur)
+    assert rc == 0
+    torch.cuda.synchronize()
+    del keep
+    return [N(o) for o in out] + [N(rows)]
+
+
+@pytest.mark.parametrize("s,P,R,C", [
+    (40960, 32, 128, 8), (40963, 32, 128, 8), (70001, 1, 16, 8),
+    (36866, 3, 128, 8), (40960, 5, 4, 1), (40960, 64, 128, 8),
+    (40960, 65, 128, 32), (36865, 255, 300, 8), (12290, 32, 2000, 8),
+    (266240, 32, 128, 8), (300001, 7, 2, 8)])
+def test_split_rows_match_streamed(gpu, s, P, R, C):
+    """Rows split over the chip against the same rows streamed by one
+    workgroup each: counts at the edges of parts, sampled ids across an
+    edge and with gaps, row lengths off the 4-token grid, more than one
+    chunk of 64 parts, matches of every length up to P."""
+    from suffixgpu_amd import _lib
+    rng = np.random.default_rng(s + P)
+    p = _lib.make_params(16, P, R, 1, [1 << min(i, 14) for i in range(C)],
+                         (), 2.0, 0.0, 0.1, 0.0)
+    part = 4096
+    nt = np.array([0, 1, part - 3, part, part + 1, 2 * part - 2, 3 * part,
+                   s - 17, s - 5, s, s // 2], I32)
+    b = len(nt)
+    tokens = rng.integers(0, 3, size=(b, s)).astype(I32)
+    tokens[3] = 7                                  # one token throughout
+    tokens[4] = np.arange(s) % 5                   # periodic
+    tokens[5] = rng.integers(0, 1 << 30, size=s)   # no matches
+    half = rng.integers(0, 50, size=900)
+    tokens[7] = np.resize(half, s)                 # long repeats
+    tokens[10, : s // 3] = 9
+    sampled = np.full((b, 17), -1, I32)
+    for i in range(b):
+        n = rng.integers(1, 17)
+        sampled[i, :n] = tokens[i, rng.integers(0, s - 20):][:n]
+    sampled[2, 5] = -1
+    sampled[6] = -1                                # nothing accepted
+    for smp, mask in ((sampled, None),
+                      (None, np.arange(b) % 4 != 2), (None, None)):
+        got = _rows_step(gpu, p, tokens, nt, smp, mask, True)
+        exp = _rows_step(gpu, p, tokens, nt, smp, mask, False)
+        for g, e in zip(got, exp):
+            np.testing.assert_array_equal(g, e)
+    assert (exp[1] > 0).sum() >= 4
