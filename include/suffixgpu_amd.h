@@ -337,12 +337,19 @@ int sfx_delta_index_build(const int32_t* delta, const int64_t* delta_len,
  *             64 bytes per workgroup instead of 16 KB, and one with work
  *             starts a memory round trip later.  Results never depend on
  *             it.  Other flag bits are rejected (SFX_EINVAL);
- *   finish -- sa[0:m] from the workspace, sa[m:n_total] the identity.
+ *   finish -- sa[0:m] from the workspace, sa[m:n_total] the identity;
+ *   finish_if_final -- the same, but nothing is written unless the array
+ *             became final in rounds first .. last (the rounds enqueued
+ *             since the previous finish_if_final): a caller that enqueues
+ *             rounds ahead of its host reads appends one to each batch of
+ *             rounds, and the output follows the round that finished.
  * The workspace's u32 state block at sfx_sa_build_flag_offset(m) (64
  * bytes to copy) holds [0] nonzero once the array is final, [2] the round
- * that found it final, [7] the round the build stalled at (0: none) and
- * [8] a mask with bit r set for every round r that ran radix launches,
- * for an asynchronous copy to the host.  sfx_sa_build enqueues the radix
+ * that found it final, [7] the round the build stalled at (0: none),
+ * [8] a mask with bit r set for every round r that ran radix launches and
+ * (from byte 64 on) [16 + r] the largest group entering round r, for an
+ * asynchronous copy to the host: once round r has run unstalled, [16 + r +
+ * 1] = 0 means that the array is final.  sfx_sa_build enqueues the radix
  * launches for every round.  The first 16 * m bytes of the workspace carry
  * nothing from one launch of a build to the next (the radix key buffers):
  * between launches, e.g. after finish, a caller may use them, as the
@@ -361,6 +368,10 @@ int sfx_sa_build_rounds(int64_t m, int32_t first, int32_t count,
 int sfx_sa_build_finish(int64_t m, int64_t n_total, void* sa, int32_t sa_is64,
                         void* workspace, size_t workspace_bytes,
                         hipStream_t stream);
+int sfx_sa_build_finish_if_final(int64_t m, int32_t first, int32_t last,
+                                 int64_t n_total, void* sa, int32_t sa_is64,
+                                 void* workspace, size_t workspace_bytes,
+                                 hipStream_t stream);
 
 /* global_index.py:235-240 _finish_swap: in-place copy of a finished
  * rebuild into the live buffers (corpus, sa: capacity int32 each), one

@@ -82,6 +82,9 @@ SIGNATURES = {
                                     ctypes.c_size_t, c_p]),
     "sfx_sa_build_finish": (c_i32, [c_i64, c_i64, c_p, c_i32, c_p,
                                     ctypes.c_size_t, c_p]),
+    "sfx_sa_build_finish_if_final": (c_i32, [c_i64, c_i32, c_i32, c_i64, c_p,
+                                             c_i32, c_p, ctypes.c_size_t,
+                                             c_p]),
     "sfx_index_swap": (c_i32, [c_p, c_p, c_p, c_p, c_i64, c_p, c_i32, c_p]),
     "sfx_delta_append": (c_i32, [ctypes.POINTER(SfxAppendDoc), c_i32, c_p,
                                  c_i64, c_p, c_i64, c_p]),

@@ -1317,9 +1317,18 @@ __global__ __launch_bounds__(256) void k_rank_keys4(const int32_t* corpus,
   if (first4 && e == r * W4) reinterpret_cast<int4*>(first4)[r] = v;
 }
 
+// first > 0: written only if the array became final in rounds first .. last
+// (every launch of those rounds precedes this one): round last left no
+// group of two or more, and round first entered with one.
 template <typename T>
 __global__ __launch_bounds__(256) void k_sa_out(const uint32_t* sa, int64_t m,
-                                                int64_t n_total, T* out) {
+                                                int64_t n_total, T* out,
+                                                const uint32_t* state,
+                                                int first, int last) {
+  if (first > 0 &&
+      (state[kStalled] || state[kMaxGrp + last + 1] != 0 ||
+       (first > 1 && state[kMaxGrp + first] == 0)))
+    return;
   // four outputs per thread; sa is a 256-byte aligned workspace array
   const int64_t j0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (j0 >= n_total) return;
@@ -1585,14 +1594,15 @@ extern "C" size_t sfx_sa_build_workspace_size(int64_t m) {
 namespace {
 
 int launch_out(const uint32_t* sa, int64_t m, int64_t n_total, void* sa_out,
-               int32_t sa_is64, hipStream_t stream) {
+               int32_t sa_is64, const uint32_t* state, int first, int last,
+               hipStream_t stream) {
   const unsigned out_blocks = (unsigned)((n_total + 1023) / 1024);
   if (sa_is64)
     hipLaunchKernelGGL(k_sa_out<int64_t>, dim3(out_blocks), dim3(256), 0,
-                       stream, sa, m, n_total, (int64_t*)sa_out);
+                       stream, sa, m, n_total, (int64_t*)sa_out, state, first, last);
   else
     hipLaunchKernelGGL(k_sa_out<int32_t>, dim3(out_blocks), dim3(256), 0,
-                       stream, sa, m, n_total, (int32_t*)sa_out);
+                       stream, sa, m, n_total, (int32_t*)sa_out, state, first, last);
   return (int)hipGetLastError();
 }
 
@@ -1650,12 +1660,24 @@ int build_rounds(int64_t m, int first, int count, int flags,
   return (int)hipGetLastError();
 }
 
+// first > 0: only if rounds first .. last made the array final.
 int build_finish(int64_t m, int64_t n_total, void* sa_out, int32_t sa_is64,
-                 void* workspace, hipStream_t stream) {
-  if (m <= 1) return launch_out(nullptr, 0, n_total, sa_out, sa_is64, stream);
+                 void* workspace, hipStream_t stream, int first = 0,
+                 int last = 0) {
+  if (m <= 1)
+    return launch_out(nullptr, 0, n_total, sa_out, sa_is64, nullptr, 0, 0,
+                      stream);
   SaWs w;
   sa_ws_layout(m, workspace, &w);
-  return launch_out(w.sa, m, n_total, sa_out, sa_is64, stream);
+  return launch_out(w.sa, m, n_total, sa_out, sa_is64, w.state, first, last,
+                    stream);
+}
+
+bool finish_args_ok(int64_t m, int64_t n_total, const void* sa_out,
+                    const void* workspace, size_t workspace_bytes) {
+  return m >= 0 && n_total >= m && n_total <= 0x7fffffffLL &&
+         (n_total == 0 ||
+          (sa_out && ws_ok(m, workspace, workspace_bytes)));
 }
 
 }  // namespace
@@ -1715,12 +1737,24 @@ extern "C" int sfx_sa_build_finish(int64_t m, int64_t n_total, void* sa_out,
                                    int32_t sa_is64, void* workspace,
                                    size_t workspace_bytes,
                                    hipStream_t stream) {
-  if (m < 0 || n_total < m || m > 0x7fffffffLL || n_total > 0x7fffffffLL)
+  if (!finish_args_ok(m, n_total, sa_out, workspace, workspace_bytes))
     return SFX_EINVAL;
   if (n_total == 0) return 0;
-  if (!sa_out) return SFX_EINVAL;
-  if (!ws_ok(m, workspace, workspace_bytes)) return SFX_EINVAL;
   return build_finish(m, n_total, sa_out, sa_is64, workspace, stream);
+}
+
+extern "C" int sfx_sa_build_finish_if_final(int64_t m, int32_t first,
+                                            int32_t last, int64_t n_total,
+                                            void* sa_out, int32_t sa_is64,
+                                            void* workspace,
+                                            size_t workspace_bytes,
+                                            hipStream_t stream) {
+  if (!finish_args_ok(m, n_total, sa_out, workspace, workspace_bytes) ||
+      first < 1 || last < first || last > total_rounds(m))
+    return SFX_EINVAL;
+  if (n_total == 0) return 0;
+  return build_finish(m, n_total, sa_out, sa_is64, workspace, stream, first,
+                      last);
 }
 
 extern "C" size_t sfx_delta_index_bytes(int64_t delta_capacity) {

@@ -33,8 +33,9 @@ from suffixgpu_amd import _lib
 from suffixgpu_amd._lib import check, lib, require_gpu, stream_of
 from suffixgpu_amd.expand import expand_chain
 from suffixgpu_amd.suffix_array import (DEFAULT_RADIX_MASK, STATE_WORDS,
-                                        BuildState, enqueue_rounds,
-                                        sa_workspace_bytes, state_view)
+                                        BuildState, _build_adaptive,
+                                        enqueue_rounds, sa_workspace_bytes,
+                                        state_view)
 
 PAD_TOKEN = torch.iinfo(torch.int32).max
 # Tokens of every suffix kept next to the suffix array (one 128-byte row
@@ -498,12 +499,28 @@ class GlobalIndex:
         return self._sa_ws
 
     def _build_staging_sa(self, dst: torch.Tensor, m: int) -> None:
-        """staging_sa[:m] = SA(dst[:m]); staging_sa[m:] = m .. N-1."""
+        """staging_sa[:m] = SA(dst[:m]); staging_sa[m:] = m .. N-1, on the
+        current stream.  The host follows the build and returns when it is
+        final, as the reference's build does (its torch.unique
+        synchronises); under graph capture every round is enqueued instead
+        (a full 2^22-token corpus: 12 idle rounds of 16 launches)."""
         ws = self._sa_workspace()
+        if m > 1 and not torch.cuda.is_current_stream_capturing():
+            state = _build_adaptive(dst, m, self.staging_sa, ws,
+                                    self.sa_radix_hint)
+            self._take_hints(state)
+            return
         check(lib().sfx_sa_build(dst.data_ptr(), m, self.capacity,
                                  self.staging_sa.data_ptr(), 0,
                                  ws.data_ptr(), ws.numel(),
                                  stream_of(self.device)), "SA rebuild")
+
+    def _take_hints(self, state: BuildState) -> None:
+        """The next build's hints from one found final: the rounds the text
+        needed plus 2, and the rounds that took the radix path."""
+        self.sa_round_hint = state.needed + 2
+        self.sa_radix_hint = state.radix_mask & ~1
+        self.sa_final_hint = state.needed + 1
 
     # Background builds, enqueued on the current (rebuild) stream.
     def _staged_build_begin(self, dst: torch.Tensor, m: int) -> None:
@@ -559,9 +576,7 @@ class GlobalIndex:
         L = lib()
         total = int(L.sfx_sa_build_rounds_total(m))
         if state.done:
-            self.sa_round_hint = state.needed + 2
-            self.sa_radix_hint = state.radix_mask & ~1
-            self.sa_final_hint = state.needed + 1
+            self._take_hints(state)
             return True
         if state.stalled:
             nxt, radix = state.stalled, 1 << state.stalled

@@ -9,6 +9,8 @@ array is unique, so it equals the reference's.
 
 from __future__ import annotations
 
+from collections import deque
+
 import torch
 
 from suffixgpu_amd._lib import (SA_ROUNDS_EXPECT_FINAL, SA_ROUNDS_RADIX,
@@ -19,8 +21,8 @@ def sa_workspace_bytes(n: int) -> int:
     return int(lib().sfx_sa_build_workspace_size(int(n)))
 
 
-# Doubling rounds enqueued between two reads of the build's done flag in
-# the adaptive build.
+# Doubling rounds enqueued between two reads of the build's state in the
+# adaptive build.
 SA_CHECK_ROUNDS = 3
 
 # int32 words of the build's state block a host copy reads, and the
@@ -28,6 +30,10 @@ SA_CHECK_ROUNDS = 3
 # two-token groups exceed a workgroup)
 STATE_WORDS = 16
 DEFAULT_RADIX_MASK = 1 << 1
+# the words an adaptive build copies after a batch: past the state block's
+# first words, [MAX_GROUP_WORD + r] is the largest group entering round r
+MAX_GROUP_WORD = 16
+BATCH_STATE_WORDS = 64
 
 
 def _workspace_ok(workspace: torch.Tensor | None, text: torch.Tensor,
@@ -55,10 +61,10 @@ def build_suffix_array_into(text: torch.Tensor, m: int, out: torch.Tensor,
     every doubling round the length allows, with no host read: launches
     after the finishing round return at their first instruction, and the
     call can be captured in a graph or run in the background.
-    adaptive=True enqueues the rounds SA_CHECK_ROUNDS at a time and reads
-    the device's done flag (one synchronisation of the current stream)
-    before enqueuing more, so the build stops within a few launches of the
-    round that finished it (the reference's build synchronises too, on
+    adaptive=True enqueues the rounds SA_CHECK_ROUNDS at a time, one batch
+    ahead of the host's reads of the build state, and returns when the host
+    has seen the array final, so the build stops within a few launches of
+    the round that finished it (the reference's build synchronises too, on
     torch.unique in suffix_gpu/suffix_array.py)."""
     require_gpu(text, out)
     if text.dtype != torch.int32 or not text.is_contiguous():
@@ -78,36 +84,61 @@ def build_suffix_array_into(text: torch.Tensor, m: int, out: torch.Tensor,
 
 
 def _build_adaptive(text: torch.Tensor, m: int, out: torch.Tensor,
-                    workspace: torch.Tensor) -> None:
+                    workspace: torch.Tensor,
+                    radix_mask: int = DEFAULT_RADIX_MASK) -> BuildState:
+    """The adaptive build of m > 1 positions: rounds go out SA_CHECK_ROUNDS
+    at a time, each batch followed by a state copy and an output that is
+    written only if that batch finished the array, and the host waits for a
+    batch with the next one already enqueued, so the GPU never waits for the
+    host between rounds.  ``radix_mask``: rounds expected to need the radix
+    path (any other that does stalls the batch and is enqueued again with
+    it).  Returns the state that found the array final."""
     L = lib()
     st = stream_of(text.device)
     ws, nbytes = workspace.data_ptr(), workspace.numel()
+    is64 = int(out.dtype == torch.int64)
     total = int(L.sfx_sa_build_rounds_total(m))
-    state = state_view(workspace, m)
-    flag = torch.empty(STATE_WORDS, dtype=torch.int32, pin_memory=True)
+    state = state_view(workspace, m, BATCH_STATE_WORDS)
+    flags = torch.empty(2, BATCH_STATE_WORDS, dtype=torch.int32,
+                        pin_memory=True)
     check(L.sfx_sa_build_begin(text.data_ptr(), m, ws, nbytes, st),
           "build_suffix_array")
+    stream = torch.cuda.current_stream(text.device)
+    pending: deque = deque()  # (event, last round, pinned state words)
     first = 1
-    radix_first = True  # round 1 and a resumed round enqueue the radix path
-    while first <= total:
-        n = min(SA_CHECK_ROUNDS, total - first + 1)
-        enqueue_rounds(m, first, n, 1 << first if radix_first else 0, ws,
-                       nbytes, st)
-        flag.copy_(state, non_blocking=True)
-        done = torch.cuda.Event()
-        done.record(torch.cuda.current_stream(text.device))
-        done.synchronize()
-        s = BuildState.of(flag.tolist())
-        if s.done:
-            break
+    sent = 0
+    while True:
+        while len(pending) < 2 and first <= total:
+            n = min(SA_CHECK_ROUNDS, total - first + 1)
+            last = first + n - 1
+            enqueue_rounds(m, first, n, radix_mask, ws, nbytes, st)
+            words = flags[sent & 1]
+            sent += 1
+            words.copy_(state, non_blocking=True)
+            ev = torch.cuda.Event()
+            ev.record(stream)
+            check(L.sfx_sa_build_finish_if_final(
+                m, first, last, out.shape[0], out.data_ptr(), is64, ws,
+                nbytes, st), "build_suffix_array")
+            pending.append((ev, last, words))
+            first = last + 1
+        ev, last, words = pending.popleft()
+        ev.synchronize()
+        w = words.tolist()
+        s = BuildState.of(w)
         if s.stalled:
-            first, radix_first = s.stalled, True
-            continue
-        first += n
-        radix_first = False
-    check(L.sfx_sa_build_finish(m, out.shape[0], out.data_ptr(),
-                                int(out.dtype == torch.int64), ws, nbytes,
-                                st), "build_suffix_array")
+            # the batch behind it returned at once; resume from the round
+            first = s.stalled
+            radix_mask |= 1 << first
+            pending.clear()
+        elif s.done:
+            return s
+        elif w[MAX_GROUP_WORD + last + 1] == 0:  # round last left no group
+            none = next(r for r in range(1, last + 2)
+                        if w[MAX_GROUP_WORD + r] == 0)
+            return BuildState(True, none, 0, s.radix_mask)
+        elif last == total:  # (h has reached m: cannot hold a group)
+            raise RuntimeError("suffix array not final after every round")
 
 
 def build_suffix_array(tokens: torch.Tensor) -> torch.Tensor:
@@ -174,11 +205,12 @@ def enqueue_rounds(m: int, first: int, count: int, radix_mask: int,
         r = r2
 
 
-def state_view(workspace: torch.Tensor, m: int) -> torch.Tensor:
+def state_view(workspace: torch.Tensor, m: int,
+               words: int = STATE_WORDS) -> torch.Tensor:
     """The device words of a build's state block (a view of the byte
     workspace)."""
     off = int(lib().sfx_sa_build_flag_offset(m))
-    return workspace[off:off + 4 * STATE_WORDS].view(torch.int32)
+    return workspace[off:off + 4 * words].view(torch.int32)
 
 
 class BuildState:

@@ -100,6 +100,14 @@ def test_argument_errors_are_reported_before_any_launch():
     assert lib.sfx_sa_build_rounds(1, 1, 1, 4, None, 0, None) == -1
     assert lib.sfx_sa_build_rounds(1, 1, 1, -1, None, 0, None) == -1
     assert lib.sfx_sa_build_rounds(1, 1, 1, 3, None, 0, None) == 0
+    # the conditional output: rounds 1 <= first <= last <= the total
+    for first, last in ((0, 1), (2, 1), (1, 99)):
+        assert lib.sfx_sa_build_finish_if_final(8, first, last, 8, 16, 0, 16,
+                                                1 << 20, None) == -1
+    assert lib.sfx_sa_build_finish_if_final(8, 1, 1, 7, 16, 0, 16, 1 << 20,
+                                            None) == -1
+    assert lib.sfx_sa_build_finish_if_final(8, 1, 1, 8, 16, 0, 16, 0,
+                                            None) == -1
     assert lib.sfx_index_swap(None, None, None, None, -1, None, 0,
                               None) == -1
     assert lib.sfx_index_swap(None, None, None, None, 16, None, 0,

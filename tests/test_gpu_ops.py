@@ -201,6 +201,48 @@ def test_build_suffix_array_stall_and_resume(gpu):
     np.testing.assert_array_equal(N(out), o_build_sa(t))
 
 
+@pytest.mark.parametrize("period,n", [(0, 2), (0, 900), (2, 9), (3, 400),
+                                      (40, 5000), (3000, 9001), (1, 5000)])
+def test_build_suffix_array_adaptive_batches(gpu, period, n):
+    """The adaptive build over texts whose last round falls on either side
+    of a batch's end, from none (distinct tokens) to every round (one
+    repeated token, whose rounds also need the radix path), and the output
+    that waits for a batch's end: untouched before it, whole after it."""
+    from suffixgpu_amd import _lib
+    from suffixgpu_amd.suffix_array import (build_suffix_array_into,
+                                            enqueue_rounds, read_build_state,
+                                            sa_workspace_bytes)
+    rng = np.random.default_rng(5)
+    t = (rng.permutation(n) if period == 0 else
+         np.resize(rng.permutation(period), n)).astype(I32)
+    exp = o_build_sa(t)
+    out = torch.full((n + 3,), -9, dtype=torch.int64, device=gpu)
+    build_suffix_array_into(T(t, gpu), n, out, adaptive=True)
+    np.testing.assert_array_equal(
+        N(out), np.concatenate([exp, [n, n + 1, n + 2]]))
+
+    L = _lib.lib()
+    st = _lib.stream_of(gpu)
+    ws = torch.empty(sa_workspace_bytes(n), dtype=torch.uint8, device=gpu)
+    dt = T(t, gpu)
+    total = int(L.sfx_sa_build_rounds_total(n))
+    _lib.check(L.sfx_sa_build_begin(dt.data_ptr(), n, ws.data_ptr(),
+                                    ws.numel(), st), "begin")
+    outs = []
+    for r in range(1, total + 1):
+        enqueue_rounds(n, r, 1, -1, ws.data_ptr(), ws.numel(), st)
+        o = torch.full((n,), -9, dtype=torch.int32, device=gpu)
+        _lib.check(L.sfx_sa_build_finish_if_final(
+            n, r, r, n, o.data_ptr(), 0, ws.data_ptr(), ws.numel(), st),
+            "finish")
+        outs.append(N(o))
+    s = read_build_state(ws, n)
+    # the round that left no group (a later one records that it found none)
+    last = max(s.needed, 1) if s.done else total
+    for r, o in enumerate(outs, 1):
+        np.testing.assert_array_equal(o, exp if r == last else -9)
+
+
 @pytest.mark.parametrize("final_from", [1, 2, 4])
 def test_build_suffix_array_expect_final_flag(gpu, final_from):
     """Rounds flagged as expected to find the array final (a rebuild's
