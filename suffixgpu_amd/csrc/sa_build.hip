@@ -23,7 +23,7 @@
 //    its length; one that runs on into the next tile is followed), sorts
 //    each of them by its keys in LDS (a 64-lane bitonic sort per
 //    64-position window, then a binary search in every other window of the
-//    group) and writes the new order, heads and sizes back;
+//    group, or merges of the windows where a group is large) and writes the new order, heads and sizes back;
 //  * groups above kCap (the radix part): their positions are compacted
 //    into a list keyed (head, rank[i + h] + 1) in SA order, LSD radix
 //    sorted, and the group heads of the sorted list are written back.
@@ -58,6 +58,10 @@ constexpr uint32_t kFinished = 0xffffffffu;  // gp[] of a finished position
 // gp[] of a position finished by the previous round: its final rank is in
 // that round's rank buffer only, and the next round copies it to the other
 constexpr uint32_t kJustFinished = 0xfffffffeu;
+// gsz[] of a group that the previous round left with the head it had: both
+// rank buffers hold that head for all its suffixes, so a round that leaves
+// it again writes no rank.  (Sizes stay below 2^31.)
+constexpr uint32_t kSameHead = 1u << 31;
 // state[] words: [0] done, [1] global list length, [2] round that found no
 // group left, [3] / [4] least / largest token other than PAD (INT32_MAX),
 // [5] h of round 1, [7] round that stalled (0: none), [8] bit r set when
@@ -766,7 +770,7 @@ __global__ __launch_bounds__(NT) void k_grp_rank(
 // of them are a group's head (hcnt[]).  It runs after the round's local
 // launch, which changed only groups of at most kCap.
 __device__ __forceinline__ bool in_big_group(const uint32_t* gsz, uint32_t g) {
-  return g < kJustFinished && gsz[g] > (uint32_t)kCap;
+  return g < kJustFinished && (gsz[g] & ~kSameHead) > (uint32_t)kCap;
 }
 
 // Groups of more than kCap among m suffixes, at most (and at least 1).
@@ -992,20 +996,104 @@ __device__ __forceinline__ uint64_t lane_next64(uint64_t v) {
 }
 
 
-// Entries of c[0 .. len) (ascending, len <= 64) below key, or at most key
-// when `incl`.
+// Entries of c[0 .. len) (ascending, len <= 64) below key.
 __device__ __forceinline__ int count_below(const uint64_t* c, int len,
-                                           uint64_t key, bool incl) {
+                                           uint64_t key) {
   int at = 0;
 #pragma unroll
   for (int step = kWave; step >= 1; step >>= 1) {
     const int q = at + step;
-    if (q <= len) {
-      const uint64_t v = c[q - 1];
-      if (incl ? v <= key : v < key) at = q;
-    }
+    if (q <= len && c[q - 1] < key) at = q;
   }
   return at;
+}
+
+// The same for any len.
+__device__ __forceinline__ int lower_count(const uint64_t* c, int len,
+                                           uint64_t key) {
+  int at = 0;
+  for (int step = 1 << (31 - __builtin_clz(len | 1)); step >= 1; step >>= 1)
+    if (at + step <= len && c[at + step - 1] < key) at += step;
+  return at;
+}
+
+// A tile with a group above kMergeMin merges its windows (merge_windows):
+// a search per level and element (log2 of the group's windows levels)
+// instead of one in each other window of the group.  LDS reads bound both.
+// Round 1 of 4,193,511 template tokens took 139 us counting and 123 us
+// merging; the whole build 883 us with 128 here, 806 with 256, 801 with
+// 512 (small groups cross few windows, so counting wins there).
+constexpr uint32_t kMergeMin = 512;
+constexpr uint32_t kMergeFlag = 1u << 16;
+static_assert(kMergeMin >= kWave && kSlots <= (int)kMergeFlag,
+              "a merged group crosses a window; slots below the flag");
+
+constexpr uint32_t kNoGroup = 0xffffffffu;  // gs of a slot without a group
+
+__device__ __forceinline__ uint32_t group_size(uint32_t gs) {
+  return (gs >> 16) & 0x7fffu;
+}
+
+// Sorts every group of the workgroup's slots from windows that are already
+// sorted: at level L the two halves of each aligned 2L-slot block that lie
+// in one group are merged, L = 64, 128, ... merge_top.  An element's place
+// is its own index plus its count in the other half (a tie keeps the left
+// half first, so the sort is stable).  sk holds the keys by slot, iv the suffix at each of a wave's
+// slots; both hold the sorted order at the end.  Every thread of the
+// workgroup calls it (barriers).
+template <int NW, int kW>
+__device__ __forceinline__ void merge_windows(uint64_t* sk, uint32_t* sid,
+                                              const uint32_t (&gs)[kW],
+                                              uint32_t (&iv)[kW], int wv,
+                                              int n, int merge_top) {
+  const int ln = lane_id();
+  for (int L = kWave; L <= merge_top; L <<= 1) {
+    // the element's slot after this level, 0xffff: not merged (two windows
+    // a word, for the registers)
+    uint32_t dst[(kW + 1) / 2];
+#pragma unroll
+    for (int k = 0; k < kW; ++k) {
+      const int s0 = (wv + k * NW) * kWave + ln;
+      const int blk = s0 & ~(2 * L - 1);
+      const int mid = blk + L;
+      uint32_t gk = gs[k];
+      // (opaque: a group's ends kept per window over the levels take the
+      // kernel past 64 VGPRs)
+      asm volatile("" : "+v"(gk));
+      const int g0 = (int)(gk & 0xffffu);
+      const int g1 = min(g0 + (int)group_size(gk), n);
+      uint32_t d = 0xffffu;
+      if (gk != kNoGroup && g0 < mid && g1 > mid) {
+        const bool left = s0 < mid;
+        const int a0 = left ? mid : max(g0, blk);
+        const int len = (left ? min(g1, mid + L) : mid) - a0;
+        // count below key (left half) or at most key (right half): keys
+        // have 52 bits, so at most key is below key + 1
+        const uint64_t lim = sk[s0] + (left ? 0 : 1);
+        const int at = lower_count(sk + a0, len, lim);
+        d = (uint32_t)(left ? s0 + at : s0 - mid + a0 + at);
+      }
+      dst[k / 2] = k & 1 ? dst[k / 2] | (d << 16) : d;
+    }
+    // (read once the searches are done: held over them, the keys spill)
+    uint64_t ke[kW];
+#pragma unroll
+    for (int k = 0; k < kW; ++k) ke[k] = sk[(wv + k * NW) * kWave + ln];
+    __syncthreads();  // every search has read the keys
+#pragma unroll
+    for (int k = 0; k < kW; ++k) {
+      const uint32_t d = (dst[k / 2] >> (16 * (k & 1))) & 0xffffu;
+      if (d != 0xffffu) {
+        sk[d] = ke[k];
+        sid[d] = iv[k];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kW; ++k)
+      if (((dst[k / 2] >> (16 * (k & 1))) & 0xffffu) != 0xffffu)
+        iv[k] = sid[(wv + k * NW) * kWave + ln];
+  }
 }
 
 // The local part of a round: the groups of at most kCap suffixes.
@@ -1037,7 +1125,7 @@ __device__ __forceinline__ int count_below(const uint64_t* c, int len,
 // has work after all.  (A separate instantiation: a run-time switch
 // changed the load schedule of every round.)
 template <int NT, bool kExpectDone>
-__global__ __launch_bounds__(NT) void k_sa_local(
+__global__ __launch_bounds__(NT, 8) void k_sa_local(
     uint32_t* __restrict__ gp, uint32_t* __restrict__ gsz,
     uint32_t* __restrict__ sa, const uint32_t* __restrict__ rank_cur,
     uint32_t* __restrict__ rank_next, const uint32_t* __restrict__ skip_cur,
@@ -1109,7 +1197,9 @@ __global__ __launch_bounds__(NT) void k_sa_local(
   }
   __shared__ uint64_t sk[kSlots];  // sorted keys, chunk by chunk
   __shared__ uint32_t gmax[NW];
+  __shared__ uint32_t sid[kSlots];
   __shared__ uint32_t skip_out;
+  __shared__ uint32_t wtop[NW];
   const int64_t te = min(ts + (int64_t)kPosTile, m);
   if (threadIdx.x == 0) skip_out = 0;
   // slots cover [ts, ts + n): the tile and the tail of the group that
@@ -1163,18 +1253,20 @@ __global__ __launch_bounds__(NT) void k_sa_local(
   }
 #pragma unroll
   for (int k = 0; k < kW; ++k)  // a group above kCap is the radix part's
-    if (sz[k] > (uint32_t)kCap) g[k] = kFinished;
+    if ((sz[k] & ~kSameHead) > (uint32_t)kCap) g[k] = kFinished;
 
   // 2. per window: sort each chunk; kept for step 3: the suffix now at
-  // the lane (iv), the group's first slot and size (gs: slot | size << 16,
-  // 0xffffffff for no group), the own-chunk counts and the lane the
+  // the lane (iv), the group's first slot and size (gs: slot | size << 16 |
+  // kSameHead, kNoGroup for no group), the own-chunk counts and the lane the
   // element came from (own, a byte each)
   uint32_t gs[kW], own[kW];
 #pragma unroll
   for (int k = 0; k < kW; ++k) {
     own[k] = 0;
     const bool act = g[k] != kFinished;
-    gs[k] = act ? (g[k] - (uint32_t)ts) | (sz[k] << 16) : 0xffffffffu;
+    gs[k] = act ? (g[k] - (uint32_t)ts) | (sz[k] << 16) |
+                      (sz[k] & kSameHead)
+                : kNoGroup;
     const int base = (wv + k * NW) * kWave;
     if (base >= n || ballot(act) == 0) continue;
     const uint32_t gprev = lane_prev(g[k]);
@@ -1210,60 +1302,102 @@ __global__ __launch_bounds__(NT) void k_sa_local(
     own[k] = (uint32_t)(ln - c0) | ((uint32_t)(js - c0) << 8) |
              ((uint32_t)(je - c0 + 1) << 16) | ((uint32_t)from << 24);
   }
+  // the tile's largest group, and the slot bits in which a group's two ends
+  // differ
+  {
+    bool large = false;
+    uint32_t span = 0;
+#pragma unroll
+    for (int k = 0; k < kW; ++k) {
+      if (gs[k] == kNoGroup) continue;
+      const uint32_t g0 = gs[k] & 0xffffu, size = group_size(gs[k]);
+      large |= size > kMergeMin;
+      span |= g0 ^ (g0 + size - 1);
+    }
+    const uint32_t sp = (uint32_t)wave_max_i32((int)span);
+    const bool any = ballot(large) != 0;
+    if (ln == 0) wtop[wv] = sp | (any ? kMergeFlag : 0u);
+  }
   __syncthreads();
+  uint32_t top = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) top |= wtop[w];
+  // the highest slot bit that a group crosses, when the tile is merged
+  const int merge_top =
+      top & kMergeFlag ? 1 << (31 - __builtin_clz(top & (kMergeFlag - 1)))
+                       : 0;
 
-  // 3. counts in the group's other chunks, then the writes
+  // 3. the element's place in its group (stable) and how many of the
+  // group's keys are below and at most its own (lt, leq), then the writes
+  if (merge_top) merge_windows<NW, kW>(sk, sid, gs, iv, wv, n, merge_top);
   uint32_t big = 0;
 #pragma unroll
   for (int k = 0; k < kW; ++k) {
     const int w = wv + k * NW;
     const int base = w * kWave;
-    if (base >= n || gs[k] == 0xffffffffu) continue;
+    if (base >= n || gs[k] == kNoGroup) continue;
     const int g0 = (int)(gs[k] & 0xffffu);
-    const uint32_t osz = gs[k] >> 16;  // the old group's size
+    const uint32_t osz = group_size(gs[k]);   // the old group's size
     const uint32_t oh = (uint32_t)(ts + g0);  // and head
     const int g1 = min(g0 + (int)osz, n);
     const uint64_t ke = sk[base + ln];
-    int stable = (int)(own[k] & 0xff);
-    int lt = (int)((own[k] >> 8) & 0xff);
-    int leq = (int)((own[k] >> 16) & 0xff);
-    const int64_t p_old = ts + base + (int)(own[k] >> 24);
-    for (int w2 = g0 / kWave; w2 <= (g1 - 1) / kWave; ++w2) {
-      if (w2 == w) continue;
-      const int a0 = max(g0, w2 * kWave);
-      const int len = min(g1, w2 * kWave + kWave) - a0;
-      const uint64_t lo_k = sk[a0], hi_k = sk[a0 + len - 1];
-      int l2, e2;
-      if (ke < lo_k) {
-        l2 = e2 = 0;
-      } else if (ke > hi_k) {
-        l2 = e2 = len;
-      } else if (lo_k == hi_k) {  // the whole chunk equals ke
-        l2 = 0;
-        e2 = len;
-      } else {
-        l2 = count_below(sk + a0, len, ke, false);
-        e2 = count_below(sk + a0, len, ke, true);
+    int stable, lt, leq;
+    bool moved = true;
+    if (merge_top) {  // the group's keys are sorted
+      const int s0 = base + ln;
+      stable = s0 - g0;
+      lt = stable;
+      leq = stable + 1;
+      if (s0 > g0 && sk[s0 - 1] == ke)
+        lt = sk[g0] == ke ? 0 : lower_count(sk + g0, stable, ke);
+      if (s0 + 1 < g1 && sk[s0 + 1] == ke)
+        leq = sk[g1 - 1] == ke ? g1 - g0
+                               : stable + lower_count(sk + s0, g1 - s0, ke + 1);
+    } else {
+      stable = (int)(own[k] & 0xff);
+      lt = (int)((own[k] >> 8) & 0xff);
+      leq = (int)((own[k] >> 16) & 0xff);
+      for (int w2 = g0 / kWave; w2 <= (g1 - 1) / kWave; ++w2) {
+        if (w2 == w) continue;
+        const int a0 = max(g0, w2 * kWave);
+        const int len = min(g1, w2 * kWave + kWave) - a0;
+        const uint64_t lo_k = sk[a0], hi_k = sk[a0 + len - 1];
+        int l2, e2;
+        if (ke < lo_k) {
+          l2 = e2 = 0;
+        } else if (ke > hi_k) {
+          l2 = e2 = len;
+        } else if (lo_k == hi_k) {  // the whole chunk equals ke
+          l2 = 0;
+          e2 = len;
+        } else {
+          l2 = count_below(sk + a0, len, ke);
+          e2 = count_below(sk + a0, len, ke + 1);
+        }
+        lt += l2;
+        leq += e2;
+        stable += w2 < w ? e2 : l2;
       }
-      lt += l2;
-      leq += e2;
-      stable += w2 < w ? e2 : l2;
+      moved = g0 + stable != base + (int)(own[k] >> 24);
     }
-    const int64_t np = ts + g0 + stable;
+    const uint32_t np = (uint32_t)(ts + g0 + stable);
     const uint32_t nh = (uint32_t)(ts + g0 + lt);
     const uint32_t size = (uint32_t)(leq - lt);
     const bool fin = size == 1;
-    rank_next[iv[k]] = nh;
+    const bool same = (gs[k] & kSameHead) != 0;
+    if (nh != oh || !same) rank_next[iv[k]] = nh;
     // a group that keeps its order and head rewrites nothing else
-    if (np != p_old || nh != oh || fin) {
+    if (moved || nh != oh || fin) {
       sa[np] = iv[k];
       gp[np] = fin ? kJustFinished : nh;
     }
     if (!fin && stable == lt) {  // the first entry of its new group
-      if (nh != oh || size != osz) gsz[nh] = size;
+      if (nh != oh || size != osz || !same)
+        gsz[nh] = size | (nh == oh ? kSameHead : 0u);
       big = max(big, size);
-      if (b + 1 < nl && (int64_t)nh < te && (int64_t)nh + size > te)
-        skip_out = (uint32_t)((int64_t)nh + size - te);
+      const int over = g0 + leq - (int)(te - ts);
+      if (b + 1 < nl && g0 + lt < (int)(te - ts) && over > 0)
+        skip_out = (uint32_t)over;
     }
   }
   big = (uint32_t)wave_max_i32((int)big);

@@ -243,6 +243,26 @@ def test_build_suffix_array_adaptive_batches(gpu, period, n):
         np.testing.assert_array_equal(o, exp if r == last else -9)
 
 
+@pytest.mark.parametrize("size", [511, 512, 513, 1000, 2048])
+@pytest.mark.parametrize("at", [0, 2500, 4090])
+def test_build_suffix_array_merged_windows(gpu, size, at):
+    """A two-token group on both sides of the size from which a tile's
+    windows are merged, `at` positions into its tile (so that it also runs
+    on into the next one), beside small groups, with few distinct keys (runs
+    of equal ones) and with many, over several rounds."""
+    from suffixgpu_amd.suffix_array import build_suffix_array_into
+    rng = np.random.default_rng(size + at)
+    for keys in (3, 400):
+        # the pair (10, 10) sorts behind `at` positions of small groups
+        small = rng.integers(0, 9, size=at).astype(I32)
+        cont = np.stack([np.full(size, 10), np.full(size, 10),
+                         11 + rng.integers(0, keys, size)], 1)
+        t = np.concatenate([small, cont.reshape(-1)]).astype(I32)
+        out = torch.empty(t.shape[0], dtype=torch.int64, device=gpu)
+        build_suffix_array_into(T(t, gpu), t.shape[0], out, adaptive=True)
+        np.testing.assert_array_equal(N(out), o_build_sa(t))
+
+
 @pytest.mark.parametrize("final_from", [1, 2, 4])
 def test_build_suffix_array_expect_final_flag(gpu, final_from):
     """Rounds flagged as expected to find the array final (a rebuild's
