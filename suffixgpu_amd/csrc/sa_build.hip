@@ -1693,6 +1693,126 @@ __global__ __launch_bounds__(256) void k_dix_start(
   }
 }
 
+// The whole index in one launch, for deltas of at most kDixOneMax
+// positions: every workgroup reads the whole delta (L2-resident after the
+// first) and places the positions of its own range of R buckets, whose
+// first entry is its count of positions in lower buckets.  Wave w takes the
+// positions w * 64 * steps .. + 64 * steps - 1, one per lane and step, so a
+// position's place in its bucket is its wave's first place (a scan over the
+// waves' counts), the earlier steps and the lower lanes.  The nine launches
+// below take 45 us at 2^16 positions and as much again in the gaps between
+// them; this one takes 10 us (16 with a full delta), bound by the hashing of
+// every position in every workgroup.  Four rows harvested into a delta of
+// 2^16: 162 -> 125 us with this and the chunks of k_ingest_move.
+constexpr int kDixThreads = 1024;
+constexpr int kDixWaves = kDixThreads / kWave;
+constexpr int kDixUnroll = 8;  // steps a wave loads at once
+constexpr int64_t kDixOneMax = 1 << 16;
+constexpr int kDixGroups = 256;      // workgroups at most: one per CU
+constexpr int kDixRangeMin = 64;     // buckets a workgroup owns, at least
+constexpr int kDixRangeMax = 1 << (kDeltaBucketBitsMax - 8);
+static_assert(kDixRangeMax <= kDixThreads &&
+                  kDixRangeMax * kDixGroups >= (1 << kDeltaBucketBitsMax),
+              "a thread per bucket of a range");
+
+__global__ __launch_bounds__(kDixThreads) void k_dix_one(
+    const int32_t* __restrict__ delta, const int64_t* __restrict__ delta_len,
+    int64_t D, int hbits, int R, int4* __restrict__ ent,
+    uint32_t* __restrict__ start) {
+  __shared__ uint32_t cnt[kDixWaves * kDixRangeMax];
+  __shared__ uint32_t red[kDixWaves];
+  const int tid = threadIdx.x;
+  const int wv = tid / kWave;
+  const int ln = lane_id();
+  int64_t dl64 = *delta_len;
+  dl64 = dl64 < 0 ? 0 : (dl64 > D ? D : dl64);
+  const int dl = (int)dl64;
+  const uint32_t lo = (uint32_t)blockIdx.x * (uint32_t)R;
+  const int steps = (dl + kDixThreads - 1) / kDixThreads;
+  const int p0 = wv * kWave * steps + ln;
+  // f(position, token, live) for each of the wave's steps; the next
+  // kDixUnroll steps' tokens are on their way while these are worked on
+  auto each_step = [&](auto f) {
+    int32_t cur[kDixUnroll], nxt[kDixUnroll];
+    auto load = [&](int32_t (&t)[kDixUnroll], int s0) {
+#pragma unroll
+      for (int u = 0; u < kDixUnroll; ++u) {
+        const int p = p0 + (s0 + u) * kWave;
+        t[u] = s0 + u < steps && p < dl ? delta[p] : 0;
+      }
+    };
+    load(cur, 0);
+    for (int s0 = 0; s0 < steps; s0 += kDixUnroll) {
+      load(nxt, s0 + kDixUnroll);
+#pragma unroll
+      for (int u = 0; u < kDixUnroll; ++u) {
+        const int p = p0 + (s0 + u) * kWave;
+        f(p, cur[u], s0 + u < steps && p < dl);
+      }
+#pragma unroll
+      for (int u = 0; u < kDixUnroll; ++u) cur[u] = nxt[u];
+    }
+  };
+  for (int e = tid; e < kDixWaves * R; e += kDixThreads) cnt[e] = 0;
+  __syncthreads();
+  // counts by wave and bucket; positions in lower buckets
+  uint32_t* mine = cnt + wv * R;
+  uint32_t below = 0;
+  each_step([&](int, int32_t t, bool live) {
+    const uint32_t bk = delta_bucket(t, hbits);
+    below += live && bk < lo;
+    uint64_t todo = ballot(live && bk - lo < (uint32_t)R);
+    while (todo) {
+      const uint32_t lead = (uint32_t)__builtin_amdgcn_readlane(
+          (int)bk, __builtin_ctzll(todo));
+      const uint64_t peers = todo & ballot(bk == lead);
+      if (ln == 0) atomicAdd(&mine[lead - lo], (uint32_t)popc(peers));
+      todo &= ~peers;
+    }
+  });
+  uint32_t base;
+  block_exscan1<kDixThreads>(below, red, &base);
+  // bucket totals, their prefix, and each wave's first place
+  uint32_t c = 0;
+  if (tid < R)
+    for (int w = 0; w < kDixWaves; ++w) c += cnt[w * R + tid];
+  uint32_t all;
+  uint32_t at = base + block_exscan1<kDixThreads>(c, red, &all);
+  if (tid < R) {
+    start[lo + tid] = at;
+    for (int w = 0; w < kDixWaves; ++w) {
+      const uint32_t x = cnt[w * R + tid];
+      cnt[w * R + tid] = at;
+      at += x;
+    }
+  }
+  if (blockIdx.x == gridDim.x - 1 && tid == 0) start[lo + R] = (uint32_t)dl;
+  __syncthreads();
+  auto entry = [&](int q, int32_t x) {
+    return make_int4(q, x, q >= 1 ? delta[q - 1] : -1,
+                     q >= 2 ? delta[q - 2] : -1);
+  };
+  each_step([&](int p, int32_t t, bool live) {
+    const uint32_t bk = delta_bucket(t, hbits);
+    uint64_t todo = ballot(live && bk - lo < (uint32_t)R);
+    while (todo) {
+      const int first = __builtin_ctzll(todo);
+      const uint32_t lead =
+          (uint32_t)__builtin_amdgcn_readlane((int)bk, first);
+      const uint64_t peers = todo & ballot(bk == lead);
+      uint32_t b0 = 0;
+      if (ln == first) b0 = atomicAdd(&mine[lead - lo], (uint32_t)popc(peers));
+      b0 = (uint32_t)__builtin_amdgcn_readlane((int)b0, first);
+      if ((peers >> ln) & 1u) ent[b0 + rank_lt(peers)] = entry(p, t);
+      todo &= ~peers;
+    }
+  });
+  // positions past the live length follow every bucket, in order
+  for (int64_t q = dl + (int64_t)blockIdx.x * kDixThreads + tid; q < D;
+       q += (int64_t)gridDim.x * kDixThreads)
+    ent[q] = entry((int)q, delta[q]);
+}
+
 }  // namespace sfx
 
 using namespace sfx;
@@ -1914,6 +2034,15 @@ extern "C" int sfx_delta_index_build(const int32_t* delta,
       workspace_bytes < dix_ws_layout(D, nullptr, nullptr))
     return SFX_EINVAL;
   const int hbits = __builtin_ctzll((unsigned long long)buckets);
+  if (D <= kDixOneMax) {
+    int64_t R = buckets / kDixGroups;
+    R = R < kDixRangeMin ? kDixRangeMin : R;
+    hipLaunchKernelGGL(k_dix_one, dim3((unsigned)(buckets / R)),
+                       dim3(kDixThreads), 0, stream, delta, delta_len, D,
+                       hbits, (int)R, reinterpret_cast<int4*>(entries),
+                       start);
+    return (int)hipGetLastError();
+  }
   DixWs w;
   dix_ws_layout(D, workspace, &w);
   const int64_t nb = (D + kTile - 1) / kTile;

@@ -631,6 +631,41 @@ def test_delta_index_at_odd_capacities(gpu, dcap):
             check_delta_index(g)
 
 
+@pytest.mark.parametrize("dcap,buckets", [
+    (1, 1 << 10), (1000, 1 << 10), (1024, 1 << 17), (5001, 1 << 11),
+    (65535, 1 << 14), (65536, 1 << 14), (65536, 1 << 17), (65537, 1 << 15)])
+def test_delta_index_build_sizes(gpu, dcap, buckets):
+    """The index by its definition on either side of the longest delta that
+    one launch indexes, at the bucket counts of one and of many buckets per
+    workgroup; live lengths from none to all; tokens that are all equal,
+    mostly equal, few (negative and largest among them) and all different."""
+    from types import SimpleNamespace
+    from suffixgpu_amd import _lib
+    L = _lib.lib()
+    rng = np.random.default_rng(dcap)
+    ws = torch.empty(int(L.sfx_delta_index_bytes(dcap)), dtype=torch.uint8,
+                     device=gpu)
+    few = np.array([0, -2, 2**31 - 1, -2**31, 7], I32)
+    texts = [np.full(dcap, 3, I32),
+             np.where(rng.random(dcap) < 0.9, 5,
+                      rng.integers(0, 1 << 17, dcap)).astype(I32),
+             few[rng.integers(0, 5, dcap)],
+             rng.permutation(dcap).astype(I32) * 7]
+    for i, dl in enumerate((dcap, max(0, dcap - 1), dcap // 3, 0, dcap + 9)):
+        t = texts[i % 4]
+        delta = T(t, gpu)
+        n = torch.tensor(dl, dtype=torch.int64, device=gpu)
+        ent = torch.full((dcap, 4), -9, dtype=torch.int32, device=gpu)
+        start = torch.full((buckets + 1,), -9, dtype=torch.int32, device=gpu)
+        _lib.check(L.sfx_delta_index_build(
+            delta.data_ptr(), n.data_ptr(), dcap, ent.data_ptr(),
+            start.data_ptr(), buckets, ws.data_ptr(), ws.numel(),
+            _lib.stream_of(gpu)), "delta index")
+        check_delta_index(SimpleNamespace(
+            delta_buckets=buckets, delta_len=min(dl, dcap), delta=delta,
+            delta_capacity=dcap, _dix_ent=ent, _dix_start=start))
+
+
 def test_round_hint_follows_the_last_build(gpu):
     """The background rebuild's first chunk of doubling rounds is sized
     from the rounds the previous build needed, with the radix path for the
