@@ -79,6 +79,25 @@ def test_first_occurrences(gpu):
         np.testing.assert_array_equal(N(cnt), ec.reshape(-1))
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 255, 4095, 4096, 4099, 12289])
+def test_first_occurrences_edges(gpu, n):
+    """Row lengths around four columns a thread and 4096 a pass (odd rows:
+    every alignment), sparse and dense hits, more and fewer than max_occ,
+    thresholds that nothing or everything reaches and past 32 bits."""
+    from suffixgpu_amd import kernels
+    rng = np.random.default_rng(n)
+    mb = np.where(rng.random((3, n)) < 0.01, rng.integers(0, 30, (3, n)),
+                  rng.integers(0, 3, (3, n))).astype(I32)
+    mb[0, -1] = 31
+    thr = np.array([[31, 1, 2, 20, -1, 1 << 33]] * 3, np.int64)
+    for r in (1, 64, 5000):
+        pos, cnt = kernels.first_occurrences(
+            T(mb, gpu), T(thr.reshape(-1), gpu), 6, r)
+        ep, ec = o_first_occ(mb, thr, r)
+        np.testing.assert_array_equal(N(pos), ep.reshape(-1, r))
+        np.testing.assert_array_equal(N(cnt), ec.reshape(-1))
+
+
 @pytest.mark.parametrize("n,vocab", [(1, 3), (2, 2), (7, 2), (64, 3),
                                      (4095, 4), (4097, 50), (20000, 3),
                                      (70000, 30000)])
