@@ -45,12 +45,23 @@
 namespace sfx {
 
 constexpr int kTile = 4096;     // list entries / SA positions per radix tile
-constexpr int kPosTile = 4096;  // SA positions per local-round tile
 constexpr int kCap = 2048;      // largest group the local part sorts
-constexpr int kSlots = kPosTile + kCap;  // positions a local workgroup reads
-// One 1024-thread workgroup per CU measured faster than 2 x 512 threads or
-// 2048-position tiles: fewer windows per wave, and one barrier pair per
-// 4096 positions.
+// SA positions per local-round tile: 4096 where the tiles fill the chip (one
+// 1024-thread workgroup per CU measured faster there than 2 x 512 threads or
+// 2048-position tiles: fewer windows per wave, and one barrier pair per 4096
+// positions), 2048 for texts of up to kSmallText positions, whose few tiles
+// leave CUs idle (repetitive text of 61,003 tokens 266 -> 230 us, 524,288
+// 382 -> 331).
+constexpr int kPosTile = 4096;
+constexpr int kPosTileSmall = 2048;
+constexpr int64_t kSmallText = 1 << 19;
+__host__ __device__ inline int pos_tile_of(int64_t m) {
+  return m <= kSmallText ? kPosTileSmall : kPosTile;
+}
+// Radix lists of at most this many tiles take a pass in one launch (see
+// k_rs_scatter's kFew); their counts of all passes lie side by side.
+constexpr int kFewTiles = 32;
+constexpr int kFewPasses = 4;
 constexpr int kSaLocalThreads = 1024;
 constexpr int kDigitBits = 9;
 constexpr int kRadix = 1 << kDigitBits;                 // 512
@@ -82,7 +93,7 @@ static_assert(kHRound + 33 <= kStateWords, "an h word per doubling");
 // bitonic sort's chunk and lane fields: ranks + 1 below 2^26.
 constexpr int kTripleBits = 26;
 constexpr int64_t kTripleMaxM = (1ll << kTripleBits) - 2;
-static_assert(kCap <= kPosTile, "a group spans at most two tiles");
+static_assert(kCap <= kPosTileSmall, "a group spans at most two tiles");
 
 struct SaWs {
   uint64_t* keyA;
@@ -95,7 +106,8 @@ struct SaWs {
   uint32_t* sa;       // [m] current suffix order
   uint32_t* gp;       // [m] group head of SA position p, or a finished mark
   uint32_t* gsz;      // [m] size of the group headed at p
-  uint32_t* hist;     // [NB][512] digit counts per tile, then offsets
+  uint32_t* hist;     // [NB][512] digit counts per tile, then offsets (few
+                      // tiles: the counts of each pass, [kFewPasses][NB][512])
   uint32_t* rowsum;   // [512] digit totals
   uint32_t* tcnt;     // [NB] unfinished positions per tile
   uint32_t* blkmax;   // [NB] last group start per tile
@@ -112,7 +124,9 @@ struct SaWs {
 static size_t sa_ws_layout(int64_t n, void* base, SaWs* w) {
   const size_t N = (size_t)(n > 0 ? n : 1);
   const size_t NB = (N + kTile - 1) / kTile;
-  const size_t NL = (N + kPosTile - 1) / kPosTile;
+  // (of either tile size: the layout's size must grow with n)
+  const size_t NL = (N + kPosTileSmall - 1) / kPosTileSmall;
+  const size_t few = kFewPasses * (NB < kFewTiles ? NB : kFewTiles);
   size_t off = 0;
   char* c = (char*)base;
   auto take = [&](size_t bytes) -> void* {
@@ -131,7 +145,7 @@ static size_t sa_ws_layout(int64_t n, void* base, SaWs* w) {
   s.sa = (uint32_t*)take(N * 4);
   s.gp = (uint32_t*)take(N * 4);
   s.gsz = (uint32_t*)take(N * 4);
-  s.hist = (uint32_t*)take((size_t)kRadix * NB * 4);
+  s.hist = (uint32_t*)take(kRadix * (NB < few ? few : NB) * 4);
   s.rowsum = (uint32_t*)take(kRadix * 4);
   s.tcnt = (uint32_t*)take(NB * 4);
   s.blkmax = (uint32_t*)take(NB * 4);
@@ -272,6 +286,15 @@ __device__ __forceinline__ uint64_t token_key(const TokenCoding& c,
                  : (uint64_t)((uint32_t)t0 ^ 0x80000000u);
 }
 
+// Few tiles: clears this block's tile in the counts of the passes from
+// `first` on.
+__device__ __forceinline__ void clear_few_hist(uint32_t* hist, int64_t nb,
+                                               int first) {
+  for (int e = first * kRadix + (int)threadIdx.x; e < kFewPasses * kRadix;
+       e += (int)blockDim.x)
+    hist[((int64_t)(e / kRadix) * nb + blockIdx.x) * kRadix + e % kRadix] = 0;
+}
+
 // vb > 0: the key carries the position in its low vb bits (no value or
 // position arrays), and the token round's first scatter computes the keys
 // from the text itself, so none are written here; vb = 0: key, value and
@@ -334,6 +357,7 @@ __global__ __launch_bounds__(kInitThreads) void k_sa_init(
   __syncthreads();
   if (threadIdx.x < kRadix)
     hist[(int64_t)blockIdx.x * kRadix + threadIdx.x] = hcnt[threadIdx.x];
+  if (nb <= kFewTiles) clear_few_hist(hist, nb, 1);
   if (i0 >= n || vb > 0) return;
   if (i0 + kInitItems <= n) {
     // key, val and pos are 256-byte aligned workspace arrays
@@ -372,6 +396,24 @@ __device__ __forceinline__ uint64_t match_digit(bool act, uint32_t d) {
   return peers;
 }
 
+
+// h[at] += 1 for every active lane, a run of active lanes with the same `at`
+// by one atomic of its first lane (equal keys sit side by side in every
+// pass, and their atomics would serialise on one address).
+__device__ __forceinline__ void add_runs(uint32_t* h, uint32_t at, bool act) {
+  const int ln = lane_id();
+  const uint64_t on = ballot(act);
+  const uint64_t lower = on & (lanes_le(ln) >> 1);
+  const uint32_t prev = (uint32_t)__shfl(
+      (int)at, lower ? kWave - 1 - __builtin_clzll(lower) : ln);
+  const bool start = act && (!lower || prev != at);
+  const uint64_t starts = ballot(start);
+  const uint64_t above = ~lanes_le(ln);
+  const uint64_t next = starts & above;
+  const uint64_t until = next ? (next & -next) - 1 : ~0ull;
+  if (start)
+    atomicAdd(&h[at], (uint32_t)popc(on & until & (above | 1ull << ln)));
+}
 
 // ---------------------------------------------------------------- radix
 // The passes run NT threads per 4096-element tile.  With about one active
@@ -509,13 +551,21 @@ __global__ __launch_bounds__(NT) void k_rs_rowscan(
 // kText: the token round's first pass (packed keys, sh = vb), which keys
 // position idx from text[idx], text[idx + 1] as k_sa_init does instead of
 // reading keys (kin unused).
-template <int NT, bool kVal = true, bool kText = false>
+// kFew: the list has at most kFewTiles tiles and hist holds this pass's plain
+// counts per tile: the block adds up the columns itself (no scan launch), and
+// counts the next pass's digits by destination tile into hnext (null after
+// the last pass; no histogram launch).  A pass is then one launch instead of
+// three, which is what a short list's pass costs: whole builds of repetitive
+// text of 3,000 tokens 186 -> 161 us, 20,000 213 -> 198, 61,003 238 -> 230,
+// 200,000 303 -> 295, but 262,144 302 -> 311 (the columns and the counts'
+// atomics by then cost more than the launches), so kFewTiles is 32.
+template <int NT, bool kVal = true, bool kText = false, bool kFew = false>
 __global__ __launch_bounds__(NT) void k_rs_scatter(
     const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin,
     uint64_t* __restrict__ kout, uint32_t* __restrict__ vout, int sh,
     const uint32_t* __restrict__ hist, int64_t nb,
     const uint32_t* __restrict__ rowsum, const uint32_t* state, int round,
-    const int32_t* __restrict__ text) {
+    const int32_t* __restrict__ text, uint32_t* __restrict__ hnext) {
   static_assert(!(kText && kVal), "the text pass packs the position");
   constexpr int NW = NT / kWave;
   constexpr int kSpan = kTile / NW;
@@ -560,10 +610,25 @@ __global__ __launch_bounds__(NT) void k_rs_scatter(
     }
   }
   for (int e = tid; e < NW * kRadix; e += NT) (&woff[0][0])[e] = 0;
+  // Digit d's total and its count in the tiles before this one.
+  uint32_t dtot = 0, dbefore = 0;
+  if (tid < kRadix) {
+    if (kFew) {
+      const int nbA = (int)tiles_of(A);
+#pragma unroll 8
+      for (int t = 0; t < nbA; ++t) {
+        const uint32_t c = hist[t * kRadix + tid];
+        dtot += c;
+        dbefore += t < (int)blockIdx.x ? c : 0u;
+      }
+    } else {
+      dtot = rowsum[tid];
+      dbefore = hist[(int64_t)blockIdx.x * kRadix + tid];
+    }
+  }
   // Digit d's first output slot: the totals of the digits below it.
   uint32_t tot;
-  const uint32_t dbase =
-      block_exscan1<NT>(tid < kRadix ? rowsum[tid] : 0u, red, &tot);
+  const uint32_t dbase = block_exscan1<NT>(dtot, red, &tot);
   // block_exscan1 ends with a barrier: the counters are zeroed.  Each
   // digit's count of a step is added once, by its lowest lane (equal
   // digits would otherwise serialise on one LDS address).
@@ -585,7 +650,7 @@ __global__ __launch_bounds__(NT) void k_rs_scatter(
   uint32_t ttot;
   const uint32_t ls = block_exscan1<NT>(cnt, red, &ttot);
   if (tid < kRadix) {
-    gdelta[tid] = dbase + hist[(int64_t)blockIdx.x * kRadix + tid] - ls;
+    gdelta[tid] = dbase + dbefore - ls;
     uint32_t run = ls;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
@@ -613,12 +678,17 @@ __global__ __launch_bounds__(NT) void k_rs_scatter(
 #pragma unroll
   for (int i = 0; i < kTile / NT; ++i) {
     const int j = tid + i * NT;
+    uint64_t kk = 0;
+    uint32_t p = 0;
     if (j < nvalid) {
-      const uint64_t kk = sk[j];
-      const uint32_t p = gdelta[digit_of(kk, sh)] + (uint32_t)j;
+      kk = sk[j];
+      p = gdelta[digit_of(kk, sh)] + (uint32_t)j;
       kout[p] = kk;
       if (kVal) vout[p] = sv[j];
     }
+    if (kFew && hnext)
+      add_runs(hnext, p / kTile * kRadix + digit_of(kk, sh + kDigitBits),
+               j < nvalid);
   }
 }
 
@@ -686,7 +756,7 @@ __global__ __launch_bounds__(NT) void k_grp_rank(
     uint32_t* __restrict__ rank_next, uint32_t* __restrict__ sa,
     uint32_t* __restrict__ gp, uint32_t* __restrict__ gsz,
     uint32_t* __restrict__ skip_next, uint32_t* __restrict__ tmax_next,
-    uint32_t* state, int round) {
+    uint32_t pos_tile, uint32_t* state, int round) {
   constexpr int NW = NT / kWave;
   constexpr int kSpan = kTile / NW;
   constexpr int kSteps = kSpan / kWave;
@@ -748,9 +818,10 @@ __global__ __launch_bounds__(NT) void k_grp_rank(
         const uint32_t size = p - head + 1;
         gsz[head] = size;
         big = max(big, size);
-        const uint32_t c = p / kPosTile;
-        if (head / kPosTile < c) skip_next[c] = p + 1 - c * kPosTile;
-        if (size > kOrderMin) atomicMax(&tmax_next[head / kPosTile], size);
+        const uint32_t c = p / pos_tile;
+        const uint32_t hc = head / pos_tile;
+        if (hc < c) skip_next[c] = p + 1 - c * pos_tile;
+        if (size > kOrderMin) atomicMax(&tmax_next[hc], size);
       }
     }
   }
@@ -783,8 +854,10 @@ template <int NT>
 __global__ __launch_bounds__(NT) void k_pos_count(
     const uint32_t* __restrict__ gp, const uint32_t* __restrict__ gsz,
     uint32_t* __restrict__ tcnt, uint32_t* __restrict__ hcnt, int64_t m,
-    const uint32_t* state, int round) {
+    int64_t nb, uint32_t* __restrict__ hist, const uint32_t* state,
+    int round) {
   if (radix_idle(state, round)) return;
+  if (nb <= kFewTiles) clear_few_hist(hist, nb, 0);
   __shared__ uint32_t red[NT / kWave];
   const int64_t base = (int64_t)blockIdx.x * kTile;
   uint32_t c = 0, hc = 0;
@@ -821,7 +894,8 @@ __global__ __launch_bounds__(NT) void k_pos_gather(
     const uint32_t* __restrict__ rank_cur, const uint32_t* __restrict__ tcnt,
     const uint32_t* __restrict__ hcnt, int64_t m, int64_t nb, int round,
     uint64_t* __restrict__ key, uint32_t* __restrict__ val,
-    uint32_t* __restrict__ pos, uint32_t* state) {
+    uint32_t* __restrict__ pos, uint32_t* __restrict__ hist,
+    uint32_t* state) {
   constexpr int NW = NT / kWave;
   constexpr int kSpan = kTile / NW;
   constexpr int kSteps = kSpan / kWave;
@@ -884,17 +958,21 @@ __global__ __launch_bounds__(NT) void k_pos_gather(
     const bool a = gv[s] != kFinished;
     const uint64_t bm = ballot(a);
     const uint64_t hm = ballot(a && gv[s] == (uint32_t)p);
+    const uint32_t o = out + (uint32_t)rank_lt(bm);
+    uint64_t kk = 0;
     if (a) {
-      const uint32_t o = out + (uint32_t)rank_lt(bm);
       // heads at or before p in this step, then the group's ordinal
       const uint32_t q = hrun + (uint32_t)popc(hm & lanes_le(ln)) - 1u;
       const uint32_t i = sa[p];
       const uint64_t k2 =
           (int64_t)i + h < m ? (uint64_t)rank_cur[i + h] + 1 : 0;
-      key[o] = (uint64_t)q * M1 + k2;
+      kk = (uint64_t)q * M1 + k2;
+      key[o] = kk;
       val[o] = i;
       pos[o] = (uint32_t)p;
     }
+    if (nb <= kFewTiles && bm)  // the first pass's counts
+      add_runs(hist, o / kTile * kRadix + digit_of(kk, 0), a);
     out += (uint32_t)popc(bm);
     hrun += (uint32_t)popc(hm);
   }
@@ -1025,8 +1103,7 @@ __device__ __forceinline__ int lower_count(const uint64_t* c, int len,
 // 512 (small groups cross few windows, so counting wins there).
 constexpr uint32_t kMergeMin = 512;
 constexpr uint32_t kMergeFlag = 1u << 16;
-static_assert(kMergeMin >= kWave && kSlots <= (int)kMergeFlag,
-              "a merged group crosses a window; slots below the flag");
+static_assert(kMergeMin >= kWave, "a merged group crosses a window");
 
 constexpr uint32_t kNoGroup = 0xffffffffu;  // gs of a slot without a group
 
@@ -1097,7 +1174,7 @@ __device__ __forceinline__ void merge_windows(uint64_t* sk, uint32_t* sid,
 }
 
 // The local part of a round: the groups of at most kCap suffixes.
-// Workgroup b owns those whose head lies in its kPosTile-position tile b.
+// Workgroup b owns those whose head lies in its kPT-position tile b.
 // It reads the tile and the tail of a group running on into the next
 // tile (at most kCap - 1 positions) as slots s = p - ts; window
 // w = slots 64w .. 64w + 63, held by wave w mod NW, lane = slot mod 64.
@@ -1124,7 +1201,7 @@ __device__ __forceinline__ void merge_windows(uint64_t* sk, uint32_t* sid,
 // before the tile's group marks, which it then reads only if the round
 // has work after all.  (A separate instantiation: a run-time switch
 // changed the load schedule of every round.)
-template <int NT, bool kExpectDone>
+template <int NT, bool kExpectDone, int kPT>
 __global__ __launch_bounds__(NT, 8) void k_sa_local(
     uint32_t* __restrict__ gp, uint32_t* __restrict__ gsz,
     uint32_t* __restrict__ sa, const uint32_t* __restrict__ rank_cur,
@@ -1132,12 +1209,14 @@ __global__ __launch_bounds__(NT, 8) void k_sa_local(
     uint32_t* __restrict__ skip_next, const uint32_t* __restrict__ order,
     int64_t m, int64_t nl, int round, int global_follows, uint32_t* state) {
   constexpr int NW = NT / kWave;
+  constexpr int kSlots = kPT + kCap;  // positions a workgroup reads
+  static_assert(kSlots <= (int)kMergeFlag, "slots below the flag");
   constexpr int kW = kSlots / kWave / NW;  // windows per wave
   static_assert(kSlots % (kWave * NW) == 0, "windows per wave");
-  static_assert(kPosTile % (kWave * NW) == 0, "tile windows per wave");
+  static_assert(kPT % (kWave * NW) == 0, "tile windows per wave");
   // this workgroup's tile (order: NULL for tile = workgroup)
   const int64_t b = order ? (int64_t)order[blockIdx.x] : (int64_t)blockIdx.x;
-  const int64_t ts = b * kPosTile;
+  const int64_t ts = b * kPT;
   const int wv = threadIdx.x / kWave;
   const int ln = lane_id();
   // The tile's group marks are read before the state and skip words are
@@ -1146,7 +1225,7 @@ __global__ __launch_bounds__(NT, 8) void k_sa_local(
   // unfinished: reading them with the marks cost 16 MB more per round at
   // 2^22 tokens, and a round after the array is final reads the marks
   // alone.)  Slot (wv + k * NW) * 64 + ln lies in the tile for k < kWT.
-  constexpr int kWT = kPosTile / kWave / NW;
+  constexpr int kWT = kPT / kWave / NW;
   uint32_t gt[kWT];
 #pragma unroll
   for (int k = 0; k < kWT; ++k) {
@@ -1200,7 +1279,7 @@ __global__ __launch_bounds__(NT, 8) void k_sa_local(
   __shared__ uint32_t sid[kSlots];
   __shared__ uint32_t skip_out;
   __shared__ uint32_t wtop[NW];
-  const int64_t te = min(ts + (int64_t)kPosTile, m);
+  const int64_t te = min(ts + (int64_t)kPT, m);
   if (threadIdx.x == 0) skip_out = 0;
   // slots cover [ts, ts + n): the tile and the tail of the group that
   // runs on into the next tile (its skip word; a run of kCap or more
@@ -1232,7 +1311,7 @@ __global__ __launch_bounds__(NT, 8) void k_sa_local(
     const int slot = (wv + k * NW) * kWave + ln;
     sz[k] = 0;
     kv[k] = 0;
-    if (g[k] == kJustFinished && slot < kPosTile) {
+    if (g[k] == kJustFinished && slot < kPT) {
       rank_next[iv[k]] = (uint32_t)(ts + slot);
       gp[ts + slot] = kFinished;
     }
@@ -1515,44 +1594,49 @@ static int sort_and_rank(SaWs& w, int64_t nb, int64_t m, int round,
                          const int32_t* text, hipStream_t stream) {
   const int vb = round == 0 ? token_round_vb(m) : 0;
   const int nbits = round == 0 ? 2 * kPairBits : round_bits(m);
+  const bool few = nb <= kFewTiles;
   uint64_t* keys[2] = {w.keyA, w.keyB};
   uint32_t* vals[2] = {w.valA, w.valB};
-  int x = 0;
-  for (int sh = vb; sh < vb + nbits; sh += kDigitBits) {
-    // (the token round's first counts come from k_sa_init)
-    if (round > 0 || sh > vb)
-      hipLaunchKernelGGL(k_rs_hist<kRsThreads>, dim3((unsigned)nb),
-                         dim3(kRsThreads), 0, stream, keys[x], sh, w.hist, nb,
-                         w.state, round);
-    hipLaunchKernelGGL(k_rs_rowscan<kRsThreads>, dim3(kScanBlocks),
-                       dim3(kRsThreads), 0, stream, w.hist, nb, w.rowsum,
-                       w.state, round);
+  const dim3 grid((unsigned)nb), block(kRsThreads);
+  int x = 0, pass = 0;
+  for (int sh = vb; sh < vb + nbits; sh += kDigitBits, ++pass) {
+    uint32_t* hist = w.hist;
+    uint32_t* hnext = nullptr;
+    if (few) {
+      hist += (size_t)pass * nb * kRadix;
+      if (sh + kDigitBits < vb + nbits) hnext = hist + (size_t)nb * kRadix;
+    } else {
+      // (the token round's first counts come from k_sa_init)
+      if (round > 0 || sh > vb)
+        hipLaunchKernelGGL(k_rs_hist<kRsThreads>, grid, block, 0, stream,
+                           keys[x], sh, hist, nb, w.state, round);
+      hipLaunchKernelGGL(k_rs_rowscan<kRsThreads>, dim3(kScanBlocks), block,
+                         0, stream, hist, nb, w.rowsum, w.state, round);
+    }
+    auto scatter = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, block, 0, stream, keys[x], vals[x],
+                         keys[x ^ 1], vals[x ^ 1], sh, hist, nb, w.rowsum,
+                         w.state, round, text, hnext);
+    };
     // (the token round's first pass keys the text itself)
     if (vb && sh == vb)
-      hipLaunchKernelGGL((k_rs_scatter<kRsThreads, false, true>),
-                         dim3((unsigned)nb), dim3(kRsThreads), 0, stream,
-                         nullptr, nullptr, keys[x ^ 1], nullptr, sh, w.hist,
-                         nb, w.rowsum, w.state, round, text);
+      few ? scatter(k_rs_scatter<kRsThreads, false, true, true>)
+          : scatter(k_rs_scatter<kRsThreads, false, true, false>);
     else if (vb)
-      hipLaunchKernelGGL((k_rs_scatter<kRsThreads, false>),
-                         dim3((unsigned)nb), dim3(kRsThreads), 0, stream,
-                         keys[x], nullptr, keys[x ^ 1], nullptr, sh, w.hist,
-                         nb, w.rowsum, w.state, round, nullptr);
+      few ? scatter(k_rs_scatter<kRsThreads, false, false, true>)
+          : scatter(k_rs_scatter<kRsThreads, false, false, false>);
     else
-      hipLaunchKernelGGL(k_rs_scatter<kRsThreads>, dim3((unsigned)nb),
-                         dim3(kRsThreads), 0, stream, keys[x], vals[x],
-                         keys[x ^ 1], vals[x ^ 1], sh, w.hist, nb, w.rowsum,
-                         w.state, round, nullptr);
+      few ? scatter(k_rs_scatter<kRsThreads, true, false, true>)
+          : scatter(k_rs_scatter<kRsThreads, true, false, false>);
     x ^= 1;
   }
   const int nx = (round + 1) & 1;
-  hipLaunchKernelGGL(k_grp_reduce<kRsThreads>, dim3((unsigned)nb),
-                     dim3(kRsThreads), 0, stream, keys[x], w.pos, vb,
-                     w.blkmax, w.state, round);
-  hipLaunchKernelGGL(k_grp_rank<kRsThreads>, dim3((unsigned)nb),
-                     dim3(kRsThreads), 0, stream, keys[x], vals[x], w.pos,
-                     vb, w.blkmax, w.rank[nx], w.sa, w.gp, w.gsz, w.skip[nx],
-                     w.tmax[nx], w.state, round);
+  hipLaunchKernelGGL(k_grp_reduce<kRsThreads>, grid, block, 0, stream,
+                     keys[x], w.pos, vb, w.blkmax, w.state, round);
+  hipLaunchKernelGGL(k_grp_rank<kRsThreads>, grid, block, 0, stream, keys[x],
+                     vals[x], w.pos, vb, w.blkmax, w.rank[nx], w.sa, w.gp,
+                     w.gsz, w.skip[nx], w.tmax[nx], (uint32_t)pos_tile_of(m),
+                     w.state, round);
   return (int)hipGetLastError();
 }
 
@@ -1563,7 +1647,8 @@ static int doubling_round(SaWs& w, int64_t nb, int64_t m, int round,
                           int global_path, int expect_done,
                           hipStream_t stream) {
   const int cur = round & 1, nx = (round + 1) & 1;
-  const int64_t nl = (m + kPosTile - 1) / kPosTile;
+  const int pt = pos_tile_of(m);
+  const int64_t nl = (m + pt - 1) / pt;
   // A round enqueued with its radix part has groups above the cap, and
   // groups of up to the cap beside them: its tiles go largest group first.
   // (In rounds of small groups only the order cost more than it saved:
@@ -1571,29 +1656,28 @@ static int doubling_round(SaWs& w, int64_t nb, int64_t m, int round,
   if (global_path)
     hipLaunchKernelGGL(k_sa_order<1024>, dim3(1), dim3(1024), 0, stream,
                        w.tmax[cur], w.tmax[nx], w.order, nl, w.state);
-  if (expect_done)
-    hipLaunchKernelGGL((k_sa_local<kSaLocalThreads, true>),
-                       dim3((unsigned)nl), dim3(kSaLocalThreads), 0, stream,
-                       w.gp, w.gsz, w.sa, w.rank[cur], w.rank[nx],
+  auto local = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nl), dim3(kSaLocalThreads), 0,
+                       stream, w.gp, w.gsz, w.sa, w.rank[cur], w.rank[nx],
                        w.skip[cur], w.skip[nx],
                        global_path ? w.order : nullptr, m, nl, round,
                        global_path, w.state);
+  };
+  if (pt == kPosTileSmall)
+    expect_done ? local(k_sa_local<kSaLocalThreads, true, kPosTileSmall>)
+                : local(k_sa_local<kSaLocalThreads, false, kPosTileSmall>);
   else
-    hipLaunchKernelGGL((k_sa_local<kSaLocalThreads, false>),
-                       dim3((unsigned)nl), dim3(kSaLocalThreads), 0, stream,
-                       w.gp, w.gsz, w.sa, w.rank[cur], w.rank[nx],
-                       w.skip[cur], w.skip[nx],
-                       global_path ? w.order : nullptr, m, nl, round,
-                       global_path, w.state);
+    expect_done ? local(k_sa_local<kSaLocalThreads, true, kPosTile>)
+                : local(k_sa_local<kSaLocalThreads, false, kPosTile>);
   if (!global_path) return (int)hipGetLastError();
   // (blkmax holds the head counts until the group-head pass needs it)
   hipLaunchKernelGGL(k_pos_count<kRsThreads>, dim3((unsigned)nb),
                      dim3(kRsThreads), 0, stream, w.gp, w.gsz, w.tcnt,
-                     w.blkmax, m, w.state, round);
+                     w.blkmax, m, nb, w.hist, w.state, round);
   hipLaunchKernelGGL(k_pos_gather<kRsThreads>, dim3((unsigned)nb),
                      dim3(kRsThreads), 0, stream, w.gp, w.gsz, w.sa,
                      w.rank[cur], w.tcnt, w.blkmax, m, nb, round, w.keyA,
-                     w.valA, w.pos, w.state);
+                     w.valA, w.pos, w.hist, w.state);
   return sort_and_rank(w, nb, m, round, nullptr, stream);
 }
 
@@ -1889,7 +1973,8 @@ int build_begin(const int32_t* text, int64_t m, void* workspace,
   hipLaunchKernelGGL(k_sa_init, dim3(eb), dim3(kInitThreads), 0, stream, text,
                      m, w.keyA, w.valA, w.pos, token_round_vb(m), plo, phi,
                      parts, w.skip[0], w.skip[1], w.tmax[0], w.tmax[1],
-                     (m + kPosTile - 1) / kPosTile, w.hist, nb, w.state);
+                     (m + pos_tile_of(m) - 1) / pos_tile_of(m), w.hist, nb,
+                     w.state);
   return sort_and_rank(w, nb, m, 0, text, stream);
 }
 
@@ -2063,7 +2148,7 @@ extern "C" int sfx_delta_index_build(const int32_t* delta,
     hipLaunchKernelGGL(k_rs_scatter<kRsThreads>, dim3((unsigned)nb),
                        dim3(kRsThreads), 0, stream, keys[x], vals[x],
                        keys[x ^ 1], vals[x ^ 1], sh, w.hist, nb, w.rowsum,
-                       w.state, 0, nullptr);
+                       w.state, 0, nullptr, nullptr);
     x ^= 1;
   }
   // two passes (keys of at most 18 bits): the sorted data is back in

@@ -282,6 +282,29 @@ def test_build_suffix_array_merged_windows(gpu, size, at):
         np.testing.assert_array_equal(N(out), o_build_sa(t))
 
 
+@pytest.mark.parametrize("n", [2047, 2049, 131072, 131073, 524288, 524289])
+def test_build_suffix_array_tile_sizes(gpu, n):
+    """Both sides of a local tile, of the longest text whose radix passes
+    are one launch each and of the longest that takes the small tile: few
+    tokens (groups above the cap, radix rounds), runs of one token and a
+    long repeat."""
+    from suffixgpu_amd.suffix_array import build_suffix_array_into
+    rng = np.random.default_rng(n)
+    t = rng.integers(0, 20, n).astype(I32)
+    t[n // 3:n // 3 + n // 8] = t[:n // 8]
+    t[n // 2:n // 2 + min(n // 8, 3000)] = 7
+    out = torch.empty(n, dtype=torch.int64, device=gpu)
+    build_suffix_array_into(T(t, gpu), n, out, adaptive=True)
+    got = N(out)
+    # sorted by definition: a permutation, each suffix below the next
+    assert np.array_equal(np.sort(got), np.arange(n))
+    rank = np.empty(n + 1, np.int64)
+    rank[got], rank[n] = np.arange(n), -1
+    a, b = got[:-1], got[1:]
+    assert np.all((t[a] < t[b]) |
+                  ((t[a] == t[b]) & (rank[a + 1] < rank[b + 1])))
+
+
 @pytest.mark.parametrize("final_from", [1, 2, 4])
 def test_build_suffix_array_expect_final_flag(gpu, final_from):
     """Rounds flagged as expected to find the array final (a rebuild's
