@@ -41,6 +41,17 @@ def global_caps(max_pattern_len: int, num_backoff: int) -> list[int]:
     return sorted(set(caps), reverse=True)
 
 
+# Local-only rows of fewer tokens than this go without the match launch even
+# where they do not fit a CU's LDS: the step's one 1024-thread workgroup per
+# row streams them about as fast as two launches take, or faster (30,000
+# tokens, 1 / 2 / 8 / 32 rows: 23.8 / 25.4 / 26.8 / 31.7 us streamed, 22.2 /
+# 32.5 / 32.5 / 33.3 split; 44,000: 22.6 / 24.8 / 32.1 / 36.4 and 17.6 / 28.2
+# / 28.2 / 31.4; 60,000: 36.4 / 36.3 / 38.6 / 51.1 and 25.6 / 26.6 / 29.9 /
+# 30.8).  With global memory on, a row has 512 threads and splitting wins
+# from the first length on (30,000, 1 / 8 rows: 32.1 / 41.1 and 28.4 / 32.3).
+SPLIT_MIN_LOCAL = 49152
+
+
 class SuffixGPUDrafter:
     """Device-resident suffix-decoding drafter (vLLM NgramProposerGPU
     contract: device tensors in, device tensors out, no host sync)."""
@@ -115,7 +126,7 @@ class SuffixGPUDrafter:
                 hi = mid
             else:
                 lo = mid + 1
-        self._split_seq = lo
+        self._split_seq = lo if enable_global else max(lo, SPLIT_MIN_LOCAL)
         if enable_global:
             self.global_index = GlobalIndex(
                 capacity=global_capacity, delta_capacity=delta_capacity,

@@ -440,3 +440,32 @@ def test_split_rows_match_streamed(gpu, s, P, R, C):
         for g, e in zip(got, exp):
             np.testing.assert_array_equal(g, e)
     assert (exp[1] > 0).sum() >= 4
+
+
+@pytest.mark.parametrize("over", [-1, 0])
+def test_local_rows_around_the_split_length(gpu, over):
+    """A local-only drafter on either side of the row length from which its
+    steps take the match launch, against the oracle."""
+    from suffixgpu_amd import SuffixGPUDrafter
+    from suffixgpu_amd.proposer import SPLIT_MIN_LOCAL
+    s = SPLIT_MIN_LOCAL + over
+    rng = np.random.default_rng(s)
+    kw = dict(k=8, max_pattern_len=16, max_occurrences=32, num_backoff=6,
+              max_spec_factor=2.0, min_token_prob=0.05)
+    d = SuffixGPUDrafter(device=gpu, **kw)
+    o = DrafterOracle(**kw)
+    assert (s >= d._split_seq) == (over == 0)
+    rows = np.resize(rng.integers(0, 40, 7000), (3, s)).astype(I32)
+    rows[1] = rng.integers(0, 5, s)
+    nt = np.array([s - 20, s // 2, 4097], I32)
+    sampled = np.full((3, 9), -1, I32)
+    sampled[0, :4] = rows[0, nt[0]:nt[0] + 4]
+    sampled[1, :2] = 3
+    sampled[2, :1] = rows[2, nt[2]]
+    dev = T(rows, gpu)
+    draft, nv, cnt = d.propose_with_update(T(nt, gpu), dev, T(sampled, gpu))
+    exp_rows = rows.copy()
+    exp = o.propose_with_update(nt, exp_rows, sampled)
+    for g, e in zip((draft, nv, cnt), exp):
+        np.testing.assert_array_equal(N(g), e)
+    np.testing.assert_array_equal(N(dev), exp_rows)
