@@ -431,42 +431,44 @@ __global__ __launch_bounds__(NT) void k_rs_hist(
   constexpr int kItems = kTile / NT;
   if (radix_idle(state, round)) return;
   const int64_t A = state[kLen];
-  const int64_t base = (int64_t)blockIdx.x * kTile;
-  if (base >= A) return;
-  // Waves w, w + kRsHists, ... share a histogram; the sub-histograms are
-  // summed at the end.  A wave's lanes hold consecutive entries, and equal
-  // keys sit next to each other in every pass (suffixes inside repeated
-  // text share their key until h outgrows the repeat), so each run of
-  // equal digits adds its length with one atomic from its first lane:
-  // same-address LDS atomics within a wave would serialise.
   __shared__ uint32_t h[kRsHists][kRadix];
-  const int tid = threadIdx.x;
-  const int ln = lane_id();
-  const int hw = (tid / kWave) % kRsHists;
-  for (int e = tid; e < kRsHists * kRadix; e += NT) (&h[0][0])[e] = 0;
-  uint32_t d[kItems];
+  for (int64_t tile = blockIdx.x; tile * kTile < A; tile += gridDim.x) {
+    const int64_t base = tile * kTile;
+    // Waves w, w + kRsHists, ... share a histogram; the sub-histograms are
+    // summed at the end.  A wave's lanes hold consecutive entries, and equal
+    // keys sit next to each other in every pass (suffixes inside repeated
+    // text share their key until h outgrows the repeat), so each run of
+    // equal digits adds its length with one atomic from its first lane:
+    // same-address LDS atomics within a wave would serialise.
+    const int tid = threadIdx.x;
+    const int ln = lane_id();
+    const int hw = (tid / kWave) % kRsHists;
+    for (int e = tid; e < kRsHists * kRadix; e += NT) (&h[0][0])[e] = 0;
+    uint32_t d[kItems];
 #pragma unroll
-  for (int r = 0; r < kItems; ++r) {
-    const int64_t idx = base + (int64_t)r * NT + tid;
-    d[r] = idx < A ? digit_of(key[idx], sh) : kRadix;
-  }
-  __syncthreads();
+    for (int r = 0; r < kItems; ++r) {
+      const int64_t idx = base + (int64_t)r * NT + tid;
+      d[r] = idx < A ? digit_of(key[idx], sh) : kRadix;
+    }
+    __syncthreads();
 #pragma unroll
-  for (int r = 0; r < kItems; ++r) {
-    const uint32_t prev = __shfl_up(d[r], 1);
-    const bool start = ln == 0 || prev != d[r];
-    const uint64_t starts = ballot(start);
-    const uint64_t after = ln == kWave - 1 ? 0ull : starts >> (ln + 1);
-    const uint32_t len =
-        after ? (uint32_t)__builtin_ctzll(after) + 1u : (uint32_t)(kWave - ln);
-    if (start && d[r] < kRadix) atomicAdd(&h[hw][d[r]], len);
-  }
-  __syncthreads();
-  if (tid < kRadix) {
-    uint32_t sum = 0;
+    for (int r = 0; r < kItems; ++r) {
+      const uint32_t prev = __shfl_up(d[r], 1);
+      const bool start = ln == 0 || prev != d[r];
+      const uint64_t starts = ballot(start);
+      const uint64_t after = ln == kWave - 1 ? 0ull : starts >> (ln + 1);
+      const uint32_t len =
+          after ? (uint32_t)__builtin_ctzll(after) + 1u : (uint32_t)(kWave - ln);
+      if (start && d[r] < kRadix) atomicAdd(&h[hw][d[r]], len);
+    }
+    __syncthreads();
+    if (tid < kRadix) {
+      uint32_t sum = 0;
 #pragma unroll
-    for (int w = 0; w < kRsHists; ++w) sum += h[w][tid];
-    hist[(int64_t)blockIdx.x * kRadix + tid] = sum;
+      for (int w = 0; w < kRsHists; ++w) sum += h[w][tid];
+      hist[(int64_t)tile * kRadix + tid] = sum;
+    }
+    __syncthreads();  // the next tile rewrites the shared arrays
   }
 }
 
@@ -573,122 +575,126 @@ __global__ __launch_bounds__(NT) void k_rs_scatter(
   static_assert(kTile % NT == 0 && NT >= kRadix, "tile shape");
   if (radix_idle(state, round)) return;
   const int64_t A = state[kLen];
-  const int64_t base = (int64_t)blockIdx.x * kTile;
-  if (base >= A) return;
   __shared__ uint32_t woff[NW][kRadix];
   __shared__ uint32_t gdelta[kRadix];  // global slot - tile slot, per digit
   __shared__ uint64_t sk[kTile];
   __shared__ uint32_t sv[kVal ? kTile : 1];
   __shared__ uint32_t red[NW];
-  const int tid = threadIdx.x;
-  const int wv = tid / kWave;
-  const int ln = lane_id();
-  const int64_t wbase = base + (int64_t)wv * kSpan;
-  const int nvalid = (int)(A - base < kTile ? A - base : kTile);
-  uint64_t k[kSteps];
-  uint32_t v[kSteps];
-  uint64_t peers[kSteps];  // lanes of the same step holding the same digit
-  if (kText) {
-    const TokenCoding tc =
-        token_coding((int32_t)state[kTokLo], (int32_t)state[kTokHi]);
+  for (int64_t tile = blockIdx.x; tile * kTile < A; tile += gridDim.x) {
+    const int64_t base = tile * kTile;
+    const int tid = threadIdx.x;
+    const int wv = tid / kWave;
+    const int ln = lane_id();
+    const int64_t wbase = base + (int64_t)wv * kSpan;
+    const int nvalid = (int)(A - base < kTile ? A - base : kTile);
+    uint64_t k[kSteps];
+    uint32_t v[kSteps];
+    uint64_t peers[kSteps];  // lanes of the same step holding the same digit
+    if (kText) {
+      const TokenCoding tc =
+          token_coding((int32_t)state[kTokLo], (int32_t)state[kTokHi]);
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-      const int64_t idx = wbase + s * kWave + ln;
-      const int32_t t0 = idx < A ? text[idx] : 0;
-      const int32_t t1 = idx + 1 < A ? text[idx + 1] : 0;
-      k[s] = idx < A ? (token_key(tc, t0, t1, idx + 1 < A) << sh) |
-                           (uint64_t)idx
-                     : 0;
-      v[s] = 0;
-    }
-  } else {
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-      const int64_t idx = wbase + s * kWave + ln;
-      k[s] = idx < A ? kin[idx] : 0;
-      v[s] = kVal && idx < A ? vin[idx] : 0;
-    }
-  }
-  for (int e = tid; e < NW * kRadix; e += NT) (&woff[0][0])[e] = 0;
-  // Digit d's total and its count in the tiles before this one.
-  uint32_t dtot = 0, dbefore = 0;
-  if (tid < kRadix) {
-    if (kFew) {
-      const int nbA = (int)tiles_of(A);
-#pragma unroll 8
-      for (int t = 0; t < nbA; ++t) {
-        const uint32_t c = hist[t * kRadix + tid];
-        dtot += c;
-        dbefore += t < (int)blockIdx.x ? c : 0u;
+      for (int s = 0; s < kSteps; ++s) {
+        const int64_t idx = wbase + s * kWave + ln;
+        const int32_t t0 = idx < A ? text[idx] : 0;
+        const int32_t t1 = idx + 1 < A ? text[idx + 1] : 0;
+        k[s] = idx < A ? (token_key(tc, t0, t1, idx + 1 < A) << sh) |
+                             (uint64_t)idx
+                       : 0;
+        v[s] = 0;
       }
     } else {
-      dtot = rowsum[tid];
-      dbefore = hist[(int64_t)blockIdx.x * kRadix + tid];
+#pragma unroll
+      for (int s = 0; s < kSteps; ++s) {
+        const int64_t idx = wbase + s * kWave + ln;
+        k[s] = idx < A ? kin[idx] : 0;
+        v[s] = kVal && idx < A ? vin[idx] : 0;
+      }
     }
-  }
-  // Digit d's first output slot: the totals of the digits below it.
-  uint32_t tot;
-  const uint32_t dbase = block_exscan1<NT>(dtot, red, &tot);
-  // block_exscan1 ends with a barrier: the counters are zeroed.  Each
-  // digit's count of a step is added once, by its lowest lane (equal
-  // digits would otherwise serialise on one LDS address).
-#pragma unroll
-  for (int s = 0; s < kSteps; ++s) {
-    const bool act = wbase + s * kWave + ln < A;
-    const uint32_t d = digit_of(k[s], sh);
-    peers[s] = match_digit(act, d);
-    if (act && rank_lt(peers[s]) == 0)
-      atomicAdd(&woff[wv][d], (uint32_t)popc(peers[s]));
-  }
-  __syncthreads();
-  // thread d: the tile's count of digit d, then its first tile slot
-  uint32_t cnt = 0;
-  if (tid < kRadix) {
-#pragma unroll
-    for (int w = 0; w < NW; ++w) cnt += woff[w][tid];
-  }
-  uint32_t ttot;
-  const uint32_t ls = block_exscan1<NT>(cnt, red, &ttot);
-  if (tid < kRadix) {
-    gdelta[tid] = dbase + dbefore - ls;
-    uint32_t run = ls;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const uint32_t c = woff[w][tid];
-      woff[w][tid] = run;
-      run += c;
+    for (int e = tid; e < NW * kRadix; e += NT) (&woff[0][0])[e] = 0;
+    // Digit d's total and its count in the tiles before this one.
+    uint32_t dtot = 0, dbefore = 0;
+    if (tid < kRadix) {
+      if (kFew) {
+        const int nbA = (int)tiles_of(A);
+#pragma unroll 8
+        for (int t = 0; t < nbA; ++t) {
+          const uint32_t c = hist[t * kRadix + tid];
+          dtot += c;
+          dbefore += t < (int)tile ? c : 0u;
+        }
+      } else {
+        dtot = rowsum[tid];
+        dbefore = hist[(int64_t)tile * kRadix + tid];
+      }
     }
-  }
-  __syncthreads();
+    // Digit d's first output slot: the totals of the digits below it.
+    uint32_t tot;
+    const uint32_t dbase = block_exscan1<NT>(dtot, red, &tot);
+    // block_exscan1 ends with a barrier: the counters are zeroed.  Each
+    // digit's count of a step is added once, by its lowest lane (equal
+    // digits would otherwise serialise on one LDS address).
 #pragma unroll
-  for (int s = 0; s < kSteps; ++s) {
-    const bool act = wbase + s * kWave + ln < A;
-    const uint32_t d = digit_of(k[s], sh);
-    const int rk = rank_lt(peers[s]);
-    if (act) {
-      const uint32_t p = woff[wv][d] + (uint32_t)rk;
-      sk[p] = k[s];
-      if (kVal) sv[p] = v[s];
+    for (int s = 0; s < kSteps; ++s) {
+      const bool act = wbase + s * kWave + ln < A;
+      const uint32_t d = digit_of(k[s], sh);
+      peers[s] = match_digit(act, d);
+      if (act && rank_lt(peers[s]) == 0)
+        atomicAdd(&woff[wv][d], (uint32_t)popc(peers[s]));
     }
-    wave_lds_sync();  // every lane has read its offset
-    if (act && rk == 0) woff[wv][d] += (uint32_t)popc(peers[s]);
-    wave_lds_sync();
-  }
-  __syncthreads();
+    __syncthreads();
+    // thread d: the tile's count of digit d, then its first tile slot
+    uint32_t cnt = 0;
+    if (tid < kRadix) {
 #pragma unroll
-  for (int i = 0; i < kTile / NT; ++i) {
-    const int j = tid + i * NT;
-    uint64_t kk = 0;
-    uint32_t p = 0;
-    if (j < nvalid) {
-      kk = sk[j];
-      p = gdelta[digit_of(kk, sh)] + (uint32_t)j;
-      kout[p] = kk;
-      if (kVal) vout[p] = sv[j];
+      for (int w = 0; w < NW; ++w) cnt += woff[w][tid];
     }
-    if (kFew && hnext)
-      add_runs(hnext, p / kTile * kRadix + digit_of(kk, sh + kDigitBits),
-               j < nvalid);
+    uint32_t ttot;
+    const uint32_t ls = block_exscan1<NT>(cnt, red, &ttot);
+    if (tid < kRadix) {
+      gdelta[tid] = dbase + dbefore - ls;
+      uint32_t run = ls;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const uint32_t c = woff[w][tid];
+        woff[w][tid] = run;
+        run += c;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      const bool act = wbase + s * kWave + ln < A;
+      const uint32_t d = digit_of(k[s], sh);
+      const int rk = rank_lt(peers[s]);
+      if (act) {
+        const uint32_t p = woff[wv][d] + (uint32_t)rk;
+        sk[p] = k[s];
+        if (kVal) sv[p] = v[s];
+      }
+      wave_lds_sync();  // every lane has read its offset
+      if (act && rk == 0) woff[wv][d] += (uint32_t)popc(peers[s]);
+      wave_lds_sync();
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kTile / NT; ++i) {
+      const int j = tid + i * NT;
+      uint64_t kk = 0;
+      uint32_t p = 0;
+      if (j < nvalid) {
+        kk = sk[j];
+        p = gdelta[digit_of(kk, sh)] + (uint32_t)j;
+        kout[p] = kk;
+        if (kVal) vout[p] = sv[j];
+      }
+      if (kFew && hnext)
+        add_runs(hnext, p / kTile * kRadix + digit_of(kk, sh + kDigitBits),
+                 j < nvalid);
+    }
+    // (the token round has a workgroup per tile: with the loop its scatter
+    // would take more than 64 VGPRs, one workgroup per CU)
+    if (!kVal) break;
   }
 }
 
@@ -713,29 +719,31 @@ __global__ __launch_bounds__(NT) void k_grp_reduce(
   constexpr int kSpan = kTile / NW;
   if (radix_idle(state, round)) return;
   const int64_t A = state[kLen];
-  const int64_t base = (int64_t)blockIdx.x * kTile;
-  if (base >= A) return;
   __shared__ uint32_t smax[NW];
-  const int wv = threadIdx.x / kWave;
-  const int ln = lane_id();
-  const int64_t wbase = base + (int64_t)wv * kSpan;
-  uint32_t mx = 0;
+  for (int64_t tile = blockIdx.x; tile * kTile < A; tile += gridDim.x) {
+    const int64_t base = tile * kTile;
+    const int wv = threadIdx.x / kWave;
+    const int ln = lane_id();
+    const int64_t wbase = base + (int64_t)wv * kSpan;
+    uint32_t mx = 0;
 #pragma unroll
-  for (int s = 0; s < kSpan / kWave; ++s) {
-    const int64_t t = wbase + s * kWave + ln;
-    if (t < A) {
-      const uint64_t kt = key[t] >> vb;
-      if (starts_group(key, t, kt, vb))
-        mx = max(mx, vb ? (uint32_t)t : pos[t]);
+    for (int s = 0; s < kSpan / kWave; ++s) {
+      const int64_t t = wbase + s * kWave + ln;
+      if (t < A) {
+        const uint64_t kt = key[t] >> vb;
+        if (starts_group(key, t, kt, vb))
+          mx = max(mx, vb ? (uint32_t)t : pos[t]);
+      }
     }
-  }
-  mx = (uint32_t)wave_max_i32((int)mx);
-  if (ln == 0) smax[wv] = mx;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t m = 0;
-    for (int w = 0; w < NW; ++w) m = max(m, smax[w]);
-    blkmax[blockIdx.x] = m;
+    mx = (uint32_t)wave_max_i32((int)mx);
+    if (ln == 0) smax[wv] = mx;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      uint32_t m = 0;
+      for (int w = 0; w < NW; ++w) m = max(m, smax[w]);
+      blkmax[tile] = m;
+    }
+    __syncthreads();  // the next tile rewrites the shared arrays
   }
 }
 
@@ -763,75 +771,76 @@ __global__ __launch_bounds__(NT) void k_grp_rank(
   static_assert(kSteps <= 32, "per-entry bits in one word");
   if (radix_idle(state, round)) return;
   const int64_t A = state[kLen];
-  const int64_t base = (int64_t)blockIdx.x * kTile;
-  if (base >= A) return;
   __shared__ uint32_t smax[NW];
   __shared__ uint32_t cred[NW];
   __shared__ uint32_t gmax[NW];
-  uint32_t cm = 0;
-  for (int t = threadIdx.x; t < (int)blockIdx.x; t += NT)
-    cm = max(cm, blkmax[t]);
-  cm = (uint32_t)wave_max_i32((int)cm);
-  if (lane_id() == 0) cred[threadIdx.x / kWave] = cm;
-  const int wv = threadIdx.x / kWave;
-  const int ln = lane_id();
-  const int64_t wbase = base + (int64_t)wv * kSpan;
-  uint32_t st[kSteps];  // start position of a group beginning here, or 0
-  uint32_t single = 0;  // bit s: entry s is a group of its own
-  uint32_t lastb = 0;   // bit s: entry s ends its group
-  uint32_t mx = 0;
+  for (int64_t tile = blockIdx.x; tile * kTile < A; tile += gridDim.x) {
+    const int64_t base = tile * kTile;
+    uint32_t cm = 0;
+    for (int t = threadIdx.x; t < (int)tile; t += NT)
+      cm = max(cm, blkmax[t]);
+    cm = (uint32_t)wave_max_i32((int)cm);
+    if (lane_id() == 0) cred[threadIdx.x / kWave] = cm;
+    const int wv = threadIdx.x / kWave;
+    const int ln = lane_id();
+    const int64_t wbase = base + (int64_t)wv * kSpan;
+    uint32_t st[kSteps];  // start position of a group beginning here, or 0
+    uint32_t single = 0;  // bit s: entry s is a group of its own
+    uint32_t lastb = 0;   // bit s: entry s ends its group
+    uint32_t mx = 0;
 #pragma unroll
-  for (int s = 0; s < kSteps; ++s) {
-    const int64_t t = wbase + s * kWave + ln;
-    st[s] = 0;
-    if (t < A) {
-      const uint64_t kt = key[t] >> vb;
-      const bool first = starts_group(key, t, kt, vb);
-      const bool last = t + 1 == A || (key[t + 1] >> vb) != kt;
-      if (first) st[s] = vb ? (uint32_t)t : pos[t];
-      single |= (uint32_t)(first && last) << s;
-      lastb |= (uint32_t)last << s;
+    for (int s = 0; s < kSteps; ++s) {
+      const int64_t t = wbase + s * kWave + ln;
+      st[s] = 0;
+      if (t < A) {
+        const uint64_t kt = key[t] >> vb;
+        const bool first = starts_group(key, t, kt, vb);
+        const bool last = t + 1 == A || (key[t + 1] >> vb) != kt;
+        if (first) st[s] = vb ? (uint32_t)t : pos[t];
+        single |= (uint32_t)(first && last) << s;
+        lastb |= (uint32_t)last << s;
+      }
+      mx = max(mx, st[s]);
     }
-    mx = max(mx, st[s]);
-  }
-  mx = (uint32_t)wave_max_i32((int)mx);
-  if (ln == 0) smax[wv] = mx;
-  __syncthreads();
-  uint32_t run = 0;
-  for (int w = 0; w < NW; ++w) run = max(run, cred[w]);
-  for (int w = 0; w < wv; ++w) run = max(run, smax[w]);
-  uint32_t big = 0;  // largest group ending in this lane's entries
+    mx = (uint32_t)wave_max_i32((int)mx);
+    if (ln == 0) smax[wv] = mx;
+    __syncthreads();
+    uint32_t run = 0;
+    for (int w = 0; w < NW; ++w) run = max(run, cred[w]);
+    for (int w = 0; w < wv; ++w) run = max(run, smax[w]);
+    uint32_t big = 0;  // largest group ending in this lane's entries
 #pragma unroll
-  for (int s = 0; s < kSteps; ++s) {
-    const int64_t t = wbase + s * kWave + ln;
-    const uint32_t head = max(run, wave_incl_max(st[s]));
-    run = max(run, (uint32_t)__builtin_amdgcn_readlane((int)head, kWave - 1));
-    const bool fin = (single >> s) & 1u;
-    if (t < A) {
-      const uint32_t i =
-          vb ? (uint32_t)(key[t] & ((1ull << vb) - 1)) : val[t];
-      const uint32_t p = vb ? (uint32_t)t : pos[t];
-      rank_next[i] = head;
-      sa[p] = i;
-      gp[p] = fin ? kJustFinished : head;
-      if (((lastb >> s) & 1u) && !fin) {
-        const uint32_t size = p - head + 1;
-        gsz[head] = size;
-        big = max(big, size);
-        const uint32_t c = p / pos_tile;
-        const uint32_t hc = head / pos_tile;
-        if (hc < c) skip_next[c] = p + 1 - c * pos_tile;
-        if (size > kOrderMin) atomicMax(&tmax_next[hc], size);
+    for (int s = 0; s < kSteps; ++s) {
+      const int64_t t = wbase + s * kWave + ln;
+      const uint32_t head = max(run, wave_incl_max(st[s]));
+      run = max(run, (uint32_t)__builtin_amdgcn_readlane((int)head, kWave - 1));
+      const bool fin = (single >> s) & 1u;
+      if (t < A) {
+        const uint32_t i =
+            vb ? (uint32_t)(key[t] & ((1ull << vb) - 1)) : val[t];
+        const uint32_t p = vb ? (uint32_t)t : pos[t];
+        rank_next[i] = head;
+        sa[p] = i;
+        gp[p] = fin ? kJustFinished : head;
+        if (((lastb >> s) & 1u) && !fin) {
+          const uint32_t size = p - head + 1;
+          gsz[head] = size;
+          big = max(big, size);
+          const uint32_t c = p / pos_tile;
+          const uint32_t hc = head / pos_tile;
+          if (hc < c) skip_next[c] = p + 1 - c * pos_tile;
+          if (size > kOrderMin) atomicMax(&tmax_next[hc], size);
+        }
       }
     }
-  }
-  big = (uint32_t)wave_max_i32((int)big);
-  if (ln == 0) gmax[wv] = big;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t g = 0;
-    for (int w = 0; w < NW; ++w) g = max(g, gmax[w]);
-    if (g) atomicMax(&state[kMaxGrp + round + 1], g);
+    big = (uint32_t)wave_max_i32((int)big);
+    if (ln == 0) gmax[wv] = big;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      uint32_t g = 0;
+      for (int w = 0; w < NW; ++w) g = max(g, gmax[w]);
+      if (g) atomicMax(&state[kMaxGrp + round + 1], g);
+    }
   }
 }
 
@@ -1594,6 +1603,8 @@ static int token_round_vb(int64_t m) {
 // LSD radix sort of round r's list (written to keyA / valA) by the low
 // `nbits` bits of its keys (above the vb value bits of the token round's
 // packed keys), then the group heads of the sorted order.
+constexpr int64_t kListBlocks = 256;
+
 static int sort_and_rank(SaWs& w, int64_t nb, int64_t m, int round,
                          const int32_t* text, hipStream_t stream) {
   const int vb = round == 0 ? token_round_vb(m) : 0;
@@ -1601,7 +1612,12 @@ static int sort_and_rank(SaWs& w, int64_t nb, int64_t m, int round,
   const bool few = nb <= kFewTiles;
   uint64_t* keys[2] = {w.keyA, w.keyB};
   uint32_t* vals[2] = {w.valA, w.valB};
-  const dim3 grid((unsigned)nb), block(kRsThreads);
+  // A round's list is usually short, and its length known on the device
+  // only: a workgroup per CU, which takes every kListBlocks-th tile (a
+  // workgroup per tile of 4,193,511 positions, most of them idle: 803 us a
+  // build, 794 with these).
+  const int64_t blocks = round == 0 || nb < kListBlocks ? nb : kListBlocks;
+  const dim3 grid((unsigned)blocks), block(kRsThreads);
   int x = 0, pass = 0;
   for (int sh = vb; sh < vb + nbits; sh += kDigitBits, ++pass) {
     uint32_t* hist = w.hist;
@@ -1789,7 +1805,7 @@ __global__ __launch_bounds__(256) void k_dix_start(
 // position's place in its bucket is its wave's first place (a scan over the
 // waves' counts), the earlier steps and the lower lanes.  The nine launches
 // below take 45 us at 2^16 positions and as much again in the gaps between
-// them; this one takes 10 us (16 with a full delta), bound by the hashing of
+// them; this one takes 10 us (16-25 with a full delta), bound by the hashing of
 // every position in every workgroup.  Four rows harvested into a delta of
 // 2^16: 162 -> 125 us with this and the chunks of k_ingest_move.
 constexpr int kDixThreads = 1024;
