@@ -885,9 +885,8 @@ __device__ __forceinline__ void global_body(const GlobalArgs& a,
             r0 = 0;
             r1 = (uint32_t)N;
           }
-          kary_bounds<G, true, 4>(a.ix.sa, a.ix.corpus, N, keys,
-                                  (int)a.ix.key_width, pat_at, l, lo, hi, r0,
-                                  r1);
+          kary_bounds<G>(a.ix.sa, a.ix.corpus, N, keys, (int)a.ix.key_width,
+                         pat_at, l, lo, hi, r0, r1);
         }
       }
       if (tid % G == 0) {

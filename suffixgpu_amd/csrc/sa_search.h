@@ -41,6 +41,45 @@ __device__ __forceinline__ int cmp_suffix(const int32_t* __restrict__ sa,
   return 0;
 }
 
+// The same comparison from the rank's key row: keys[rank * kw + j] holds
+// corpus[sa[rank] + j] (or -1 past the end) for j < kw, so patterns of up
+// to kw tokens are decided by one row load (kw * 4 bytes, one line for
+// kw = 32); longer patterns continue in the corpus.  pt holds the first
+// min(plen, 32) pattern tokens in registers, so the token loop waits on
+// nothing but the row.
+template <class PatFn>
+__device__ __forceinline__ int cmp_suffix_key(
+    const int32_t* __restrict__ keys, int kw,
+    const int32_t* __restrict__ sa, const int32_t* __restrict__ corpus,
+    int64_t n, int64_t rank, const int32_t (&pt)[32], PatFn pat_at,
+    int plen) {
+  const int4* row = reinterpret_cast<const int4*>(keys + rank * kw);
+  const int kn = plen < kw ? plen : kw;
+  int4 w[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    if (4 * q < kn) w[q] = row[q];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int t4[4] = {w[q].x, w[q].y, w[q].z, w[q].w};
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = 4 * q + u;
+      if (j >= kn) break;
+      if (t4[u] != pt[j]) return t4[u] < pt[j] ? -1 : 1;
+    }
+  }
+  if (plen <= kw) return 0;
+  const int64_t pos = sa[rank];
+  for (int j = kw; j < plen; ++j) {
+    const int64_t idx = pos + j;
+    const int32_t t = idx < n ? corpus[idx] : -1;
+    const int32_t pj = pat_at(j);
+    if (t != pj) return t < pj ? -1 : 1;
+  }
+  return 0;
+}
+
 // Probe k of a range [lo, hi) cut by NP probes: lo + floor((hi - lo) *
 // (k + 1) c / 2^32) with c = floor(2^32 / (NP + 1)), one 32x32->64
 // multiply (ranks stay below 2^31).  kc = (k + 1) c < 2^32, so the probes
@@ -62,98 +101,141 @@ __device__ __forceinline__ void kary_narrow(uint32_t& lo, uint32_t& hi,
   hi = nhi;
 }
 
-// Comparison of a group's G probes at once (G % 8 == 0).  Instruction i
-// loads 32 tokens of probes i * G/8 .. + G/8 - 1, one 16-byte part per lane:
-// lanes 8s .. 8s + 7 of the group read probe i * G/8 + s's, so each load
-// instruction of the wave touches one or two lines per 8 lanes.  (With one
-// probe per lane it touched 64 lines, and the CU's vector L1 serves the
-// distinct lines of an instruction one after another: the waves of a
-// workgroup then queued behind each other, about 0.4 us apart.)  The tokens
-// are the rank's key row, or without key rows those of its suffix in the
-// corpus: each lane then reads its own probe's suffix position first, so a
-// round is two dependent loads however long the match is.  (One probe per
-// lane, 4 tokens a step, takes a dependent load for every 4 tokens a probe
-// shares with the pattern, and a narrow range's probes share nearly all of
-// them.)  A corpus position is only 4-byte aligned; its 16 bytes are one
-// load all the same.  Two ballots per instruction give every probe's first
+// Key-row comparison of a group's G probes at once (G % 8 == 0, keys not
+// NULL).  Instruction i loads the rows of probes i * G/8 .. + G/8 - 1, one
+// 16-byte part per lane: lanes 8s .. 8s + 7 of the group read probe
+// i * G/8 + s's row, so each load instruction of the wave touches one
+// line per 8 lanes.  (With one row per lane it touched 64 lines, and the
+// CU's vector L1 serves the distinct lines of an instruction one after
+// another: the waves of a workgroup then queued behind each other, about
+// 0.4 us apart.)  Two ballots per instruction give every row's first
 // differing token and its sign; each lane keeps its own probe's result
 // (probe gl: instruction gl / (G/8), octet gl % (G/8)) and finishes it in
-// the corpus when the pattern is longer than what was read and all of it
-// ties.  pc holds pattern tokens 4 * (gl % 8) .. + 3.  probe_of(q) is probe
-// q's rank.  Returns -1 / 0 / +1 for the lane's own probe.
-struct __attribute__((packed, aligned(4))) Tokens4 {
-  int32_t t[4];
-};
-
-// kKeys: from key rows.  kBatch: instructions in flight at once (kInstr, or
-// half of them where the registers are short).
-template <int G, bool kKeys, int kBatch, class ProbeFn, class PatFn>
-__device__ __forceinline__ int cmp_probes(
+// the corpus when the pattern is longer than the row and the row ties.
+// pc holds pattern tokens 4 * (gl % 8) .. + 3.  probe_of(q) is probe q's
+// rank.  Returns -1 / 0 / +1 for the lane's own probe.
+template <int G, class ProbeFn, class PatFn>
+__device__ __forceinline__ int cmp_probes_key(
     const int32_t* __restrict__ keys, int kw,
     const int32_t* __restrict__ sa, const int32_t* __restrict__ corpus,
     int64_t n, ProbeFn probe_of, const int32_t (&pc)[4], PatFn pat_at,
     int plen) {
-  constexpr int kParts = 8;             // 16-byte parts of 32 tokens
-  constexpr int kRows = G / kParts;     // probes per load instruction
+  constexpr int kParts = 8;             // 16-byte parts of a 128-byte row
+  constexpr int kRows = G / kParts;     // rows per load instruction
   constexpr int kInstr = G / kRows;     // load instructions per round
-  static_assert(G % kParts == 0 && kInstr % kBatch == 0, "whole octets");
+  static_assert(G % kParts == 0, "whole rows per group");
   const int ln = lane_id();
   const int gl = ln % G;
   const int gbase = ln - gl;
   const int part = gl % kParts;
   const int sub = gl / kParts;
-  const int seen = kKeys ? kw : 4 * kParts;  // tokens read per probe
-  const int kn = plen < seen ? plen : seen;
+  const int kn = plen < kw ? plen : kw;
   const bool live = 4 * part < kn;
-  const int32_t own = kKeys ? 0 : sa[probe_of(gl)];  // n < 2^31
-  int cv = 0;
-#pragma unroll 1
-  for (int i0 = 0; i0 < kInstr; i0 += kBatch) {
-    Tokens4 v[kBatch];
+  int4 v[kInstr];
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int q = (i0 + u) * kRows + sub;
-      if constexpr (kKeys) {
-        int4 w = make_int4(0, 0, 0, 0);
-        if (live)
-          w = reinterpret_cast<const int4*>(keys + probe_of(q) * kw)[part];
-        v[u] = Tokens4{{w.x, w.y, w.z, w.w}};
-      } else {
-        const int32_t pos = __shfl(own, gbase + q);
-        const uint32_t at = (uint32_t)(pos > 0 ? pos : 0) + 4u * part;
-        if (live && (int64_t)at + 3 < n) {
-          v[u] = *reinterpret_cast<const Tokens4*>(corpus + at);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            v[u].t[j] = live && (int64_t)at + j < n ? corpus[at + j] : -1;
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      bool mis = false, neg = false;
-#pragma unroll
-      for (int j = 3; j >= 0; --j) {  // the lowest differing token wins
-        if (live && 4 * part + j < kn && v[u].t[j] != pc[j]) {
-          mis = true;
-          neg = v[u].t[j] < pc[j];
-        }
-      }
-      const uint64_t bm = ballot(mis);
-      const uint64_t bn = ballot(mis && neg);
-      const int ob = gbase + kParts * (gl % kRows);  // own probe's octet
-      const uint32_t seg = (uint32_t)(bm >> ob) & 0xffu;
-      const int lb = seg ? __builtin_ctz(seg) : 0;
-      const bool nb = (bn >> (ob + lb)) & 1ull;
-      const int r = seg == 0 ? 0 : (nb ? -1 : 1);
-      cv = i0 + u == gl / kRows ? r : cv;
+  for (int i = 0; i < kInstr; ++i) {
+    v[i] = make_int4(0, 0, 0, 0);
+    if (live) {
+      const int64_t pr = probe_of(i * kRows + sub);
+      v[i] = reinterpret_cast<const int4*>(keys + pr * kw)[part];
     }
   }
-  if (cv != 0 || plen <= seen) return cv;
-  const int64_t pos = kKeys ? sa[probe_of(gl)] : own;
-  for (int j = seen; j < plen; ++j) {
+  int cv = 0;
+#pragma unroll
+  for (int i = 0; i < kInstr; ++i) {
+    const int32_t t4[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+    bool mis = false, neg = false;
+#pragma unroll
+    for (int j = 3; j >= 0; --j) {  // the lowest differing token wins
+      if (live && 4 * part + j < kn && t4[j] != pc[j]) {
+        mis = true;
+        neg = t4[j] < pc[j];
+      }
+    }
+    const uint64_t bm = ballot(mis);
+    const uint64_t bn = ballot(mis && neg);
+    const int ob = gbase + kParts * (gl % kRows);  // own probe's octet
+    const uint32_t seg = (uint32_t)(bm >> ob) & 0xffu;
+    const int lb = seg ? __builtin_ctz(seg) : 0;
+    const bool nb = (bn >> (ob + lb)) & 1ull;
+    const int r = seg == 0 ? 0 : (nb ? -1 : 1);
+    cv = i == gl / kRows ? r : cv;
+  }
+  if (cv != 0 || plen <= kw) return cv;
+  const int64_t pos = sa[probe_of(gl)];
+  for (int j = kw; j < plen; ++j) {
     const int64_t idx = pos + j;
+    const int32_t t = idx < n ? corpus[idx] : -1;
+    const int32_t pj = pat_at(j);
+    if (t != pj) return t < pj ? -1 : 1;
+  }
+  return 0;
+}
+
+// The same comparison through sa and the corpus (no key rows): each lane
+// reads its own probe's suffix position, then the lanes of an octet read
+// 32 corpus tokens of one probe's suffix, 4 per lane, so a round is two
+// dependent loads however long the match is.  (One probe per lane, 4 tokens
+// a step, takes a dependent load for every 4 tokens a probe shares with the
+// pattern, and a narrow range's probes share nearly all of them.)  A corpus
+// position is only 4-byte aligned; its 16 bytes are one load all the same.
+struct __attribute__((packed, aligned(4))) Tokens4 {
+  int32_t t[4];
+};
+
+template <int G, class ProbeFn, class PatFn>
+__device__ __forceinline__ int cmp_probes_corpus(
+    const int32_t* __restrict__ sa, const int32_t* __restrict__ corpus,
+    int64_t n, ProbeFn probe_of, const int32_t (&pc)[4], PatFn pat_at,
+    int plen) {
+  constexpr int kParts = 8;          // lanes per probe: 32 tokens
+  constexpr int kRows = G / kParts;  // probes per load instruction
+  constexpr int kInstr = G / kRows;
+  static_assert(G % kParts == 0, "whole octets per group");
+  const int ln = lane_id();
+  const int gl = ln % G;
+  const int gbase = ln - gl;
+  const int part = gl % kParts;
+  const int sub = gl / kParts;
+  const int kn = plen < 4 * kParts ? plen : 4 * kParts;
+  const bool live = 4 * part < kn;
+  const int32_t own = sa[probe_of(gl)];  // n < 2^31
+  Tokens4 v[kInstr];
+#pragma unroll
+  for (int i = 0; i < kInstr; ++i) {
+    const int64_t at =
+        (int64_t)__shfl(own, gbase + i * kRows + sub) + 4 * part;
+    if (live && at >= 0 && at + 3 < n) {
+      v[i] = *reinterpret_cast<const Tokens4*>(corpus + at);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        v[i].t[j] = live && at + j < n ? corpus[at + j > 0 ? at + j : 0] : -1;
+    }
+  }
+  int cv = 0;
+#pragma unroll
+  for (int i = 0; i < kInstr; ++i) {
+    bool mis = false, neg = false;
+#pragma unroll
+    for (int j = 3; j >= 0; --j) {  // the lowest differing token wins
+      if (live && 4 * part + j < kn && v[i].t[j] != pc[j]) {
+        mis = true;
+        neg = v[i].t[j] < pc[j];
+      }
+    }
+    const uint64_t bm = ballot(mis);
+    const uint64_t bn = ballot(mis && neg);
+    const int ob = gbase + kParts * (gl % kRows);  // own probe's octet
+    const uint32_t seg = (uint32_t)(bm >> ob) & 0xffu;
+    const int lb = seg ? __builtin_ctz(seg) : 0;
+    const bool nb = (bn >> (ob + lb)) & 1ull;
+    const int r = seg == 0 ? 0 : (nb ? -1 : 1);
+    cv = i == gl / kRows ? r : cv;
+  }
+  if (cv != 0 || plen <= 4 * kParts) return cv;
+  for (int j = 4 * kParts; j < plen; ++j) {
+    const int64_t idx = (int64_t)own + j;
     const int32_t t = idx < n ? corpus[idx] : -1;
     const int32_t pj = pat_at(j);
     if (t != pj) return t < pj ? -1 : 1;
@@ -164,8 +246,7 @@ __device__ __forceinline__ int cmp_probes(
 // Exact lower bound (first rank with cmp >= 0) and upper bound (first rank
 // with cmp > 0) of one pattern.  Called by all G lanes of an aligned group
 // with identical arguments; returns the bounds on every lane of the group.
-// keys[rank * kw + j] (kw = key width, 4 <= kw <= 32, kw % 4 == 0) holds
-// corpus[sa[rank] + j] or -1 past the end; keys may be NULL: then the
+// keys (kw = key width, 4 <= kw <= 32, kw % 4 == 0) may be NULL: then the
 // comparison reads sa and the corpus.  n < 2^31.  The search runs inside
 // [r0, r1], which must hold both bounds (every rank below r0 compares
 // below the pattern, every rank from r1 on above it); [0, n] always does.
@@ -174,12 +255,9 @@ __device__ __forceinline__ int cmp_probes(
 // one bound left, or the bounds split), so each lane's probe and both
 // bounds' updates are computed for every phase with selects: no phase
 // branches for the wave to run one after another.
-// kOct: compare by lane octets (cmp_probes); without it (and without keys) a
-// lane reads its own probe's suffix, which takes more dependent loads but
-// fewer reads, for calls whose many patterns fill the chip.
-// kBatch: of cmp_probes without keys (four keep the step kernels at 80
-// VGPRs).
-template <int G, bool kOct = true, int kBatch = 8, class PatFn>
+// kCorpusOct: without keys, compare by lane octets (cmp_probes_corpus);
+// more registers, so the step kernels leave it off.
+template <int G, bool kCorpusOct = false, class PatFn>
 __device__ __forceinline__ void kary_bounds(
     const int32_t* __restrict__ sa, const int32_t* __restrict__ corpus,
     int64_t n, const int32_t* __restrict__ keys, int kw, PatFn pat_at,
@@ -191,11 +269,15 @@ __device__ __forceinline__ void kary_bounds(
   const int ln = lane_id();
   const int gl = ln % G;
   const int gbase = ln - gl;
-  int32_t pt[4] = {0, 0, 0, 0};  // pattern tokens 4 * (gl % 8) .. + 3
-  if constexpr (kOct) {
+  constexpr bool kCoop = G % 8 == 0;  // rows read by lane octets
+  int32_t pt[kCoop ? 4 : 32];
+  static_assert(!kCorpusOct || kCoop, "octets");
+  if (keys || kCorpusOct) {
+    // cooperative: pattern tokens 4 * (gl % 8) .. + 3; else all of them
+    const int j0 = kCoop ? 4 * (gl % 8) : 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      pt[j] = 4 * (gl % 8) + j < plen ? pat_at(4 * (gl % 8) + j) : 0;
+    for (int j = 0; j < (kCoop ? 4 : 32); ++j)
+      pt[j] = j0 + j < plen ? pat_at(j0 + j) : 0;
   }
   uint32_t lo1 = r0, hi1 = r1, lo2 = r0, hi2 = r1;
   while (lo1 < hi1 || lo2 < hi2) {
@@ -215,13 +297,17 @@ __device__ __forceinline__ void kary_bounds(
                               (uint32_t)(kq + 1) * c);
     };
     int cv;
-    if constexpr (kOct)
-      cv = keys ? cmp_probes<G, true, 8>(keys, kw, sa, corpus, n, probe_of,
-                                         pt, pat_at, plen)
-                : cmp_probes<G, false, kBatch>(keys, kw, sa, corpus, n,
-                                               probe_of, pt, pat_at, plen);
-    else
-      cv = cmp_suffix(sa, corpus, n, probe_of(gl), pat_at, plen);
+    if constexpr (kCorpusOct) {
+      cv = cmp_probes_corpus<G>(sa, corpus, n, probe_of, pt, pat_at, plen);
+    } else if constexpr (kCoop) {
+      cv = keys ? cmp_probes_key<G>(keys, kw, sa, corpus, n, probe_of, pt,
+                                    pat_at, plen)
+                : cmp_suffix(sa, corpus, n, probe_of(gl), pat_at, plen);
+    } else {
+      cv = keys ? cmp_suffix_key(keys, kw, sa, corpus, n, probe_of(gl), pt,
+                                 pat_at, plen)
+                : cmp_suffix(sa, corpus, n, probe_of(gl), pat_at, plen);
+    }
     const uint64_t m1 = ballot(cv >= 0);
     const uint64_t m2 = ballot(cv > 0);
     const uint32_t full = G == 32 ? 0xffffffffu : ((1u << G) - 1u);
