@@ -206,9 +206,10 @@ int sfx_global_query(const sfx_params* p, const sfx_index* index,
  * index, every row runs an SA-search, a delta-scan and a local workgroup
  * that hand results over through the workspace; whichever finishes a row
  * last writes that row's draft [B,K] i32 and num_valid [B] i32.
- * new_counts [B] i32 may be NULL.  workspace: sfx_step_workspace_size()
- * bytes (0 for local-only), zero-filled once; calls sharing a workspace
- * must not overlap. */
+ * new_counts [B] i32 may be NULL; with index == NULL it may be num_tokens
+ * itself (i32 counts updated in place), with an index the two must not
+ * overlap.  workspace: sfx_step_workspace_size() bytes (0 for local-only),
+ * zero-filled once; calls sharing a workspace must not overlap. */
 size_t sfx_step_workspace_size(const sfx_params* p, int64_t batch,
                                int64_t delta_capacity);
 int sfx_propose_step(const sfx_params* p, const sfx_index* index,

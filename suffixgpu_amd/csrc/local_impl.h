@@ -199,6 +199,16 @@ __device__ __forceinline__ void local_candidates(const sfx_params& p, int S,
   }
 }
 
+// The row's count after the step's scatter.  Called once every thread of the
+// row's local workgroup has read the count before it (behind a barrier), and
+// by no other launch or workgroup: without an index, new_counts may be
+// num_tokens itself.
+__device__ __forceinline__ void store_count(const LocalArgs& a, int b,
+                                            const RowState& st) {
+  if (a.bt.sampled && a.new_counts && threadIdx.x == 0)
+    a.new_counts[b] = (int32_t)st.q;
+}
+
 // From the first R ends per candidate on: the gather outputs, or expansion,
 // the best candidate, and the draft or the handover to the final pick.
 template <int NT>
@@ -400,9 +410,9 @@ __device__ __forceinline__ void local_body(const LocalArgs& a,
         grow[pos] = v;
       }
     }
-    if (a.new_counts && tid == 0) a.new_counts[b] = (int32_t)q;
   }
   __syncthreads();
+  store_count(a, b, st);
 
   if (a.mode == kLocalStep && !st.mask) {
     for (int j = tid; j < K; j += NT) a.draft[(int64_t)b * K + j] = -1;
@@ -634,6 +644,8 @@ __device__ __forceinline__ void local_split_body(const LocalArgs& a,
     found[tid] = 0;
   }
   const RowState st = row_state(a.bt, b);
+  __syncthreads();
+  store_count(a, b, st);
   if (!st.mask) {
     for (int j = tid; j < K; j += NT) a.draft[(int64_t)b * K + j] = -1;
     if (tid == 0) a.num_valid[b] = 0;

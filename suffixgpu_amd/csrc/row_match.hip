@@ -44,7 +44,6 @@ __global__ __launch_bounds__(kMatchThreads) void k_row_match(LocalArgs a) {
       const int32_t v = sp[j];
       if (j < st.cnt && v != -1 && pos < S && pos >= 0) grow[pos] = v;
     }
-    if (a.new_counts && tid == 0) a.new_counts[b] = (int32_t)st.q;
   }
   const int qe = (int)(st.q < 0 ? 0 : (st.q < S ? st.q : S));
   const int lo = k * kRowPart;

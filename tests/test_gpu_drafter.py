@@ -469,3 +469,45 @@ def test_local_rows_around_the_split_length(gpu, over):
     for g, e in zip((draft, nv, cnt), exp):
         np.testing.assert_array_equal(N(g), e)
     np.testing.assert_array_equal(N(dev), exp_rows)
+
+
+@pytest.mark.parametrize("s,scratch", [(9000, False), (40960, False),
+                                       (40960, True)])
+def test_local_step_counts_in_place(gpu, s, scratch):
+    """Local-only steps whose new counts are written over the counts they
+    start from: rows in LDS, streamed and split, drafting and masked.  The
+    only occurrence of each row's tail ends at the row's last tokens, so a
+    count taken twice shows in the draft."""
+    from suffixgpu_amd import _lib
+    L = _lib.lib()
+    rng = np.random.default_rng(s)
+    kw = dict(k=8, max_pattern_len=16, max_occurrences=32, num_backoff=6,
+              max_spec_factor=2.0, min_token_prob=0.05)
+    p = _lib.make_params(8, 16, 32, 1, [1 << i for i in range(6)], (), 2.0,
+                         0.0, 0.05, 0.0)
+    b = 24
+    rows = np.tile(np.arange(s), (b, 1)).astype(I32)
+    nt = rng.integers(s // 2, s - 10, b).astype(I32)
+    sampled = np.full((b, 9), -1, I32)
+    for i in range(b):
+        n = i % 4                       # none accepted: masked
+        rows[i, nt[i] - 4:nt[i]] = s + np.arange(4)
+        sampled[i, :n] = s + np.arange(n)
+    exp_rows = rows.copy()
+    exp = DrafterOracle(**kw).propose_with_update(nt, exp_rows, sampled)
+    dev, counts = T(rows, gpu), T(nt, gpu)
+    bt, keep = _lib.make_batch(dev, counts, sampled=T(sampled, gpu), limit=s)
+    assert bt.num_tokens == counts.data_ptr()
+    draft = torch.full((b, 8), -9, dtype=torch.int32, device=gpu)
+    nv = torch.full((b,), -9, dtype=torch.int32, device=gpu)
+    n = int(L.sfx_row_scratch_size(p, b, s))
+    assert (n > 0) == (s > 30000)
+    ws = torch.empty(n if scratch else 0, dtype=torch.uint8, device=gpu)
+    _lib.check(L.sfx_propose_step_rows(
+        p, None, bt, draft.data_ptr(), nv.data_ptr(), counts.data_ptr(),
+        None, 0, _lib.ptr(ws) if scratch else None, ws.numel(),
+        torch.cuda.current_stream().cuda_stream), "step")
+    torch.cuda.synchronize()
+    del keep
+    for g, e in zip((draft, nv, counts, dev), (*exp, exp_rows)):
+        np.testing.assert_array_equal(N(g), e)
