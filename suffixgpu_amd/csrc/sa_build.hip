@@ -1015,8 +1015,12 @@ constexpr int kXcds = 8;
 template <int NT>
 __global__ __launch_bounds__(NT) void k_sa_order(
     const uint32_t* __restrict__ tmax, uint32_t* __restrict__ tmax_next,
-    uint32_t* __restrict__ order, int64_t nl, const uint32_t* state) {
-  if (state[kDone]) return;
+    uint32_t* __restrict__ order, int64_t nl, const uint32_t* state,
+    int round) {
+  const uint32_t stalled = state[kStalled];
+  // (tmax_next of a round behind the stalled one is tmax of that one, which
+  // the caller enqueues again)
+  if (state[kDone] || (stalled != 0 && stalled < (uint32_t)round)) return;
   // cleared for the round's radix part, which records its groups there
   for (int64_t t = threadIdx.x; t <= nl; t += NT) tmax_next[t] = 0;
   __shared__ uint32_t cnt[kXcds][kOrderClasses];
@@ -1675,7 +1679,7 @@ static int doubling_round(SaWs& w, int64_t nb, int64_t m, int round,
   // 45-60 us rounds went 15-20 us slower on the template corpus.)
   if (global_path)
     hipLaunchKernelGGL(k_sa_order<1024>, dim3(1), dim3(1024), 0, stream,
-                       w.tmax[cur], w.tmax[nx], w.order, nl, w.state);
+                       w.tmax[cur], w.tmax[nx], w.order, nl, w.state, round);
   auto local = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)nl), dim3(kSaLocalThreads), 0,
                        stream, w.gp, w.gsz, w.sa, w.rank[cur], w.rank[nx],

@@ -220,6 +220,36 @@ def test_build_suffix_array_stall_and_resume(gpu):
     np.testing.assert_array_equal(N(out), o_build_sa(t))
 
 
+def test_build_suffix_array_stall_stops_every_launch(gpu):
+    """Rounds behind a stalled one, with and without radix launches, leave
+    the whole workspace as it is, and the build resumes from there."""
+    from suffixgpu_amd import _lib
+    from suffixgpu_amd.suffix_array import (enqueue_rounds, read_build_state,
+                                            sa_workspace_bytes)
+    m = 6001
+    t = np.full(m, 7, I32)              # every round has a large group
+    L = _lib.lib()
+    st = _lib.stream_of(gpu)
+    text = T(t, gpu)
+    ws = torch.zeros(sa_workspace_bytes(m), dtype=torch.uint8, device=gpu)
+    out = torch.full((m,), -9, dtype=torch.int32, device=gpu)
+    args = (ws.data_ptr(), ws.numel(), st)
+    _lib.check(L.sfx_sa_build_begin(text.data_ptr(), m, *args), "begin")
+    enqueue_rounds(m, 1, 2, 1 << 1, *args)
+    assert read_build_state(ws, m).stalled == 2
+    before = N(ws)
+    enqueue_rounds(m, 3, 3, 1 << 3 | 1 << 4, *args)
+    _lib.check(L.sfx_sa_build_finish_if_final(
+        m, 1, 5, m, out.data_ptr(), 0, *args), "finish")
+    np.testing.assert_array_equal(N(ws), before)
+    assert (N(out) == -9).all()
+    total = int(L.sfx_sa_build_rounds_total(m))
+    enqueue_rounds(m, 2, total - 1, -1, *args)
+    _lib.check(L.sfx_sa_build_finish(m, m, out.data_ptr(), 0, *args),
+               "finish")
+    np.testing.assert_array_equal(N(out), np.arange(m)[::-1])
+
+
 @pytest.mark.parametrize("period,n", [(0, 2), (0, 900), (2, 9), (3, 400),
                                       (40, 5000), (3000, 9001), (1, 5000)])
 def test_build_suffix_array_adaptive_batches(gpu, period, n):
