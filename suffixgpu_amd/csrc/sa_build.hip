@@ -384,35 +384,29 @@ __device__ __forceinline__ uint64_t lanes_le(int ln) {
   return ln == kWave - 1 ? ~0ull : (2ull << ln) - 1;
 }
 
-// Lanes of the wave holding the same digit as the calling lane.
-__device__ __forceinline__ uint64_t match_digit(bool act, uint32_t d) {
+// Active lanes of the wave whose low kBits of v equal the calling lane's.
+template <int kBits>
+__device__ __forceinline__ uint64_t match_bits(bool act, uint32_t v) {
   uint64_t peers = ballot(act);
 #pragma unroll
-  for (int bit = 0; bit < kDigitBits; ++bit) {
-    const bool set = (d >> bit) & 1u;
+  for (int bit = 0; bit < kBits; ++bit) {
+    const bool set = (v >> bit) & 1u;
     const uint64_t m = ballot(act && set);
     peers &= set ? m : ~m;
   }
   return peers;
 }
 
-
-// h[at] += 1 for every active lane, a run of active lanes with the same `at`
-// by one atomic of its first lane (equal keys sit side by side in every
-// pass, and their atomics would serialise on one address).
-__device__ __forceinline__ void add_runs(uint32_t* h, uint32_t at, bool act) {
-  const int ln = lane_id();
-  const uint64_t on = ballot(act);
-  const uint64_t lower = on & (lanes_le(ln) >> 1);
-  const uint32_t prev = (uint32_t)__shfl(
-      (int)at, lower ? kWave - 1 - __builtin_clzll(lower) : ln);
-  const bool start = act && (!lower || prev != at);
-  const uint64_t starts = ballot(start);
-  const uint64_t above = ~lanes_le(ln);
-  const uint64_t next = starts & above;
-  const uint64_t until = next ? (next & -next) - 1 : ~0ull;
-  if (start)
-    atomicAdd(&h[at], (uint32_t)popc(on & until & (above | 1ull << ln)));
+// Few tiles: h[at] += 1 for every active lane, one atomic for all lanes of
+// the wave with the same `at` (a digit count of a tile).  The digits of a
+// small vocabulary are few and alternate from lane to lane, and an atomic for
+// each run of equal ones queued on their addresses: a build of 131,072 tokens
+// of 1,000 values 193 us, 136 with these.
+constexpr int kFewBits = 14;
+static_assert(kFewTiles * kRadix <= 1 << kFewBits, "digit counts of a list");
+__device__ __forceinline__ void add_same(uint32_t* h, uint32_t at, bool act) {
+  const uint64_t peers = match_bits<kFewBits>(act, at);
+  if (act && rank_lt(peers) == 0) atomicAdd(&h[at], (uint32_t)popc(peers));
 }
 
 // ---------------------------------------------------------------- radix
@@ -638,7 +632,7 @@ __global__ __launch_bounds__(NT) void k_rs_scatter(
     for (int s = 0; s < kSteps; ++s) {
       const bool act = wbase + s * kWave + ln < A;
       const uint32_t d = digit_of(k[s], sh);
-      peers[s] = match_digit(act, d);
+      peers[s] = match_bits<kDigitBits>(act, d);
       if (act && rank_lt(peers[s]) == 0)
         atomicAdd(&woff[wv][d], (uint32_t)popc(peers[s]));
     }
@@ -689,7 +683,7 @@ __global__ __launch_bounds__(NT) void k_rs_scatter(
         if (kVal) vout[p] = sv[j];
       }
       if (kFew && hnext)
-        add_runs(hnext, p / kTile * kRadix + digit_of(kk, sh + kDigitBits),
+        add_same(hnext, p / kTile * kRadix + digit_of(kk, sh + kDigitBits),
                  j < nvalid);
     }
     // (the token round has a workgroup per tile: with the loop its scatter
@@ -896,7 +890,9 @@ __global__ __launch_bounds__(NT) void k_pos_count(
 // big_groups_max(m), so the key takes fewer bits than the head would).
 // Each block sums the earlier tiles' counts for its output offset and
 // ordinal base; block 0 also sums them all: the list length (state[kLen]).
-template <int NT>
+// kFew: the list has at most kFewTiles tiles and the first pass's digits are
+// counted here (k_rs_scatter).
+template <int NT, bool kFew>
 __global__ __launch_bounds__(NT) void k_pos_gather(
     const uint32_t* __restrict__ gp, const uint32_t* __restrict__ gsz,
     const uint32_t* __restrict__ sa,
@@ -980,8 +976,8 @@ __global__ __launch_bounds__(NT) void k_pos_gather(
       val[o] = i;
       pos[o] = (uint32_t)p;
     }
-    if (nb <= kFewTiles && bm)  // the first pass's counts
-      add_runs(hist, o / kTile * kRadix + digit_of(kk, 0), a);
+    if (kFew && bm)
+      add_same(hist, o / kTile * kRadix + digit_of(kk, 0), a);
     out += (uint32_t)popc(bm);
     hrun += (uint32_t)popc(hm);
   }
@@ -1698,10 +1694,13 @@ static int doubling_round(SaWs& w, int64_t nb, int64_t m, int round,
   hipLaunchKernelGGL(k_pos_count<kRsThreads>, dim3((unsigned)nb),
                      dim3(kRsThreads), 0, stream, w.gp, w.gsz, w.tcnt,
                      w.blkmax, m, nb, w.hist, w.state, round);
-  hipLaunchKernelGGL(k_pos_gather<kRsThreads>, dim3((unsigned)nb),
-                     dim3(kRsThreads), 0, stream, w.gp, w.gsz, w.sa,
-                     w.rank[cur], w.tcnt, w.blkmax, m, nb, round, w.keyA,
-                     w.valA, w.pos, w.hist, w.state);
+  auto gather = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(kRsThreads), 0, stream,
+                       w.gp, w.gsz, w.sa, w.rank[cur], w.tcnt, w.blkmax, m, nb,
+                       round, w.keyA, w.valA, w.pos, w.hist, w.state);
+  };
+  nb <= kFewTiles ? gather(k_pos_gather<kRsThreads, true>)
+                  : gather(k_pos_gather<kRsThreads, false>);
   return sort_and_rank(w, nb, m, round, nullptr, stream);
 }
 

@@ -335,6 +335,29 @@ def test_build_suffix_array_tile_sizes(gpu, n):
                   ((t[a] == t[b]) & (rank[a + 1] < rank[b + 1])))
 
 
+def _check_suffix_order(t, got):
+    """Sorted by definition: a permutation, each suffix below the next."""
+    n = t.shape[0]
+    assert np.array_equal(np.sort(got), np.arange(n))
+    rank = np.empty(n + 1, np.int64)
+    rank[got], rank[n] = np.arange(n), -1
+    a, b = got[:-1], got[1:]
+    assert np.all((t[a] < t[b]) |
+                  ((t[a] == t[b]) & (rank[a + 1] < rank[b + 1])))
+
+
+@pytest.mark.parametrize("n", [4097, 131072])
+@pytest.mark.parametrize("vocab", [2, 511, 1000, 200000])
+def test_build_suffix_array_few_digits(gpu, n, vocab):
+    """One-launch radix passes over digits of one, two and many values (the
+    counts of a wave's equal digits are added together)."""
+    from suffixgpu_amd.suffix_array import build_suffix_array_into
+    t = np.random.default_rng(n + vocab).integers(0, vocab, n).astype(I32)
+    out = torch.empty(n, dtype=torch.int64, device=gpu)
+    build_suffix_array_into(T(t, gpu), n, out, adaptive=True)
+    _check_suffix_order(t, N(out))
+
+
 @pytest.mark.parametrize("final_from", [1, 2, 4])
 def test_build_suffix_array_expect_final_flag(gpu, final_from):
     """Rounds flagged as expected to find the array final (a rebuild's
