@@ -1603,7 +1603,17 @@ static int token_round_vb(int64_t m) {
 // LSD radix sort of round r's list (written to keyA / valA) by the low
 // `nbits` bits of its keys (above the vb value bits of the token round's
 // packed keys), then the group heads of the sorted order.
-constexpr int64_t kListBlocks = 256;
+// A round's list is usually short, and its length known on the device only,
+// so its launches have a fixed number of workgroups that loop over its tiles:
+// as many as the chip holds at once, two per CU, and one where a workgroup's
+// LDS leaves room for no more (the scatter).  4,193,504 template tokens with
+// every round's radix launches enqueued: 1.50 ms with a workgroup per tile of
+// the text, most of them idle, 1.40 with these, 1.39 with 256 in every launch
+// (adaptive builds 804, 802, 801 us).  One repeated token, whose list is the
+// whole text in every round: 1,500,000 positions 2.96, 2.91 and 3.14 ms,
+// 4,193,504 tokens of two values 2.00, 1.91 and 1.97.
+constexpr int64_t kListBlocks = 512;
+constexpr int64_t kListScatterBlocks = 256;
 
 static int sort_and_rank(SaWs& w, int64_t nb, int64_t m, int round,
                          const int32_t* text, hipStream_t stream) {
@@ -1612,12 +1622,11 @@ static int sort_and_rank(SaWs& w, int64_t nb, int64_t m, int round,
   const bool few = nb <= kFewTiles;
   uint64_t* keys[2] = {w.keyA, w.keyB};
   uint32_t* vals[2] = {w.valA, w.valB};
-  // A round's list is usually short, and its length known on the device
-  // only: a workgroup per CU, which takes every kListBlocks-th tile (a
-  // workgroup per tile of 4,193,511 positions, most of them idle: 803 us a
-  // build, 794 with these).
-  const int64_t blocks = round == 0 || nb < kListBlocks ? nb : kListBlocks;
-  const dim3 grid((unsigned)blocks), block(kRsThreads);
+  // (the token round's list is the whole text)
+  auto list_grid = [&](int64_t most) {
+    return dim3((unsigned)(round == 0 || nb < most ? nb : most));
+  };
+  const dim3 grid = list_grid(kListBlocks), block(kRsThreads);
   int x = 0, pass = 0;
   for (int sh = vb; sh < vb + nbits; sh += kDigitBits, ++pass) {
     uint32_t* hist = w.hist;
@@ -1634,9 +1643,9 @@ static int sort_and_rank(SaWs& w, int64_t nb, int64_t m, int round,
                          0, stream, hist, nb, w.rowsum, w.state, round);
     }
     auto scatter = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, grid, block, 0, stream, keys[x], vals[x],
-                         keys[x ^ 1], vals[x ^ 1], sh, hist, nb, w.rowsum,
-                         w.state, round, text, hnext);
+      hipLaunchKernelGGL(kernel, list_grid(kListScatterBlocks), block, 0,
+                         stream, keys[x], vals[x], keys[x ^ 1], vals[x ^ 1],
+                         sh, hist, nb, w.rowsum, w.state, round, text, hnext);
     };
     // (the token round's first pass keys the text itself)
     if (vb && sh == vb)

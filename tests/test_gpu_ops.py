@@ -346,6 +346,26 @@ def _check_suffix_order(t, got):
                   ((t[a] == t[b]) & (rank[a + 1] < rank[b + 1])))
 
 
+def test_build_suffix_array_long_radix_list(gpu):
+    """A radix list of more tiles than its launches have workgroups, so that
+    every list kernel takes a second tile: all of 2.3M tokens of 8 values
+    lie in groups above the cap after the token round."""
+    from suffixgpu_amd.suffix_array import (build_suffix_array_rounds,
+                                            read_build_state,
+                                            sa_workspace_bytes)
+    n = 2_300_000
+    t = np.random.default_rng(8).integers(0, 8, n).astype(I32)
+    pairs = np.bincount(t[:-1] * 8 + t[1:], minlength=64)
+    listed = int(pairs[pairs > 2048].sum())
+    assert listed > 512 * 4096
+    ws = torch.empty(sa_workspace_bytes(n), dtype=torch.uint8, device=gpu)
+    out = torch.empty(n, dtype=torch.int32, device=gpu)
+    build_suffix_array_rounds(T(t, gpu), n, out, ws, 12, radix_mask=-1)
+    st = read_build_state(ws, n)
+    assert st.done and st.radix_mask & 2
+    _check_suffix_order(t, N(out))
+
+
 @pytest.mark.parametrize("n", [4097, 131072])
 @pytest.mark.parametrize("vocab", [2, 511, 1000, 200000])
 def test_build_suffix_array_few_digits(gpu, n, vocab):
