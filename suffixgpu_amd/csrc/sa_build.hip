@@ -288,10 +288,11 @@ __device__ __forceinline__ uint64_t token_key(const TokenCoding& c,
 
 // Few tiles: clears this block's tile in the counts of the passes from
 // `first` on.
+template <int NT>
 __device__ __forceinline__ void clear_few_hist(uint32_t* hist, int64_t nb,
                                                int first) {
   for (int e = first * kRadix + (int)threadIdx.x; e < kFewPasses * kRadix;
-       e += (int)blockDim.x)
+       e += NT)
     hist[((int64_t)(e / kRadix) * nb + blockIdx.x) * kRadix + e % kRadix] = 0;
 }
 
@@ -357,7 +358,7 @@ __global__ __launch_bounds__(kInitThreads) void k_sa_init(
   __syncthreads();
   if (threadIdx.x < kRadix)
     hist[(int64_t)blockIdx.x * kRadix + threadIdx.x] = hcnt[threadIdx.x];
-  if (nb <= kFewTiles) clear_few_hist(hist, nb, 1);
+  if (nb <= kFewTiles) clear_few_hist<kInitThreads>(hist, nb, 1);
   if (i0 >= n || vb > 0) return;
   if (i0 + kInitItems <= n) {
     // key, val and pos are 256-byte aligned workspace arrays
@@ -410,6 +411,11 @@ __device__ __forceinline__ void add_same(uint32_t* h, uint32_t at, bool act) {
 }
 
 // ---------------------------------------------------------------- radix
+// The kernels of a radix round take their launch's number of workgroups as
+// an argument (nwg): gridDim and blockDim would give each 256 bytes more of
+// arguments to write, and a build whose every round is enqueued has hundreds
+// of idle launches (1,500,000 positions, 394 launches from a slow host: 1.43
+// ms with them, 1.21 without).
 // The passes run NT threads per 4096-element tile.  With about one active
 // tile per CU, 1024 threads (16 waves) keep four times more loads and LDS
 // operations in flight per CU than 256 threads would.
@@ -420,13 +426,13 @@ constexpr int kRsHists = 4;  // LDS sub-histograms of the histogram pass
 template <int NT>
 __global__ __launch_bounds__(NT) void k_rs_hist(
     const uint64_t* __restrict__ key, int sh, uint32_t* hist, int64_t nb,
-    const uint32_t* state, int round) {
+    const uint32_t* state, int round, int nwg) {
   static_assert(kTile % NT == 0 && NT >= kRadix, "tile shape");
   constexpr int kItems = kTile / NT;
   if (radix_idle(state, round)) return;
   const int64_t A = state[kLen];
   __shared__ uint32_t h[kRsHists][kRadix];
-  for (int64_t tile = blockIdx.x; tile * kTile < A; tile += gridDim.x) {
+  for (int64_t tile = blockIdx.x; tile * kTile < A; tile += nwg) {
     const int64_t base = tile * kTile;
     // Waves w, w + kRsHists, ... share a histogram; the sub-histograms are
     // summed at the end.  A wave's lanes hold consecutive entries, and equal
@@ -561,7 +567,7 @@ __global__ __launch_bounds__(NT) void k_rs_scatter(
     uint64_t* __restrict__ kout, uint32_t* __restrict__ vout, int sh,
     const uint32_t* __restrict__ hist, int64_t nb,
     const uint32_t* __restrict__ rowsum, const uint32_t* state, int round,
-    const int32_t* __restrict__ text, uint32_t* __restrict__ hnext) {
+    const int32_t* __restrict__ text, uint32_t* __restrict__ hnext, int nwg) {
   static_assert(!(kText && kVal), "the text pass packs the position");
   constexpr int NW = NT / kWave;
   constexpr int kSpan = kTile / NW;
@@ -574,7 +580,7 @@ __global__ __launch_bounds__(NT) void k_rs_scatter(
   __shared__ uint64_t sk[kTile];
   __shared__ uint32_t sv[kVal ? kTile : 1];
   __shared__ uint32_t red[NW];
-  for (int64_t tile = blockIdx.x; tile * kTile < A; tile += gridDim.x) {
+  for (int64_t tile = blockIdx.x; tile * kTile < A; tile += nwg) {
     const int64_t base = tile * kTile;
     const int tid = threadIdx.x;
     const int wv = tid / kWave;
@@ -708,13 +714,13 @@ __device__ __forceinline__ bool starts_group(const uint64_t* key, int64_t t,
 template <int NT>
 __global__ __launch_bounds__(NT) void k_grp_reduce(
     const uint64_t* __restrict__ key, const uint32_t* __restrict__ pos,
-    int vb, uint32_t* blkmax, const uint32_t* state, int round) {
+    int vb, uint32_t* blkmax, const uint32_t* state, int round, int nwg) {
   constexpr int NW = NT / kWave;
   constexpr int kSpan = kTile / NW;
   if (radix_idle(state, round)) return;
   const int64_t A = state[kLen];
   __shared__ uint32_t smax[NW];
-  for (int64_t tile = blockIdx.x; tile * kTile < A; tile += gridDim.x) {
+  for (int64_t tile = blockIdx.x; tile * kTile < A; tile += nwg) {
     const int64_t base = tile * kTile;
     const int wv = threadIdx.x / kWave;
     const int ln = lane_id();
@@ -758,7 +764,7 @@ __global__ __launch_bounds__(NT) void k_grp_rank(
     uint32_t* __restrict__ rank_next, uint32_t* __restrict__ sa,
     uint32_t* __restrict__ gp, uint32_t* __restrict__ gsz,
     uint32_t* __restrict__ skip_next, uint32_t* __restrict__ tmax_next,
-    uint32_t pos_tile, uint32_t* state, int round) {
+    uint32_t pos_tile, uint32_t* state, int round, int nwg) {
   constexpr int NW = NT / kWave;
   constexpr int kSpan = kTile / NW;
   constexpr int kSteps = kSpan / kWave;
@@ -768,7 +774,7 @@ __global__ __launch_bounds__(NT) void k_grp_rank(
   __shared__ uint32_t smax[NW];
   __shared__ uint32_t cred[NW];
   __shared__ uint32_t gmax[NW];
-  for (int64_t tile = blockIdx.x; tile * kTile < A; tile += gridDim.x) {
+  for (int64_t tile = blockIdx.x; tile * kTile < A; tile += nwg) {
     const int64_t base = tile * kTile;
     uint32_t cm = 0;
     for (int t = threadIdx.x; t < (int)tile; t += NT)
@@ -860,7 +866,7 @@ __global__ __launch_bounds__(NT) void k_pos_count(
     int64_t nb, uint32_t* __restrict__ hist, const uint32_t* state,
     int round) {
   if (radix_idle(state, round)) return;
-  if (nb <= kFewTiles) clear_few_hist(hist, nb, 0);
+  if (nb <= kFewTiles) clear_few_hist<NT>(hist, nb, 0);
   __shared__ uint32_t red[NT / kWave];
   const int64_t base = (int64_t)blockIdx.x * kTile;
   uint32_t c = 0, hc = 0;
@@ -1638,14 +1644,16 @@ static int sort_and_rank(SaWs& w, int64_t nb, int64_t m, int round,
       // (the token round's first counts come from k_sa_init)
       if (round > 0 || sh > vb)
         hipLaunchKernelGGL(k_rs_hist<kRsThreads>, grid, block, 0, stream,
-                           keys[x], sh, hist, nb, w.state, round);
+                           keys[x], sh, hist, nb, w.state, round,
+                           (int)grid.x);
       hipLaunchKernelGGL(k_rs_rowscan<kRsThreads>, dim3(kScanBlocks), block,
                          0, stream, hist, nb, w.rowsum, w.state, round);
     }
     auto scatter = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, list_grid(kListScatterBlocks), block, 0,
-                         stream, keys[x], vals[x], keys[x ^ 1], vals[x ^ 1],
-                         sh, hist, nb, w.rowsum, w.state, round, text, hnext);
+      const dim3 sgrid = list_grid(kListScatterBlocks);
+      hipLaunchKernelGGL(kernel, sgrid, block, 0, stream, keys[x], vals[x],
+                         keys[x ^ 1], vals[x ^ 1], sh, hist, nb, w.rowsum,
+                         w.state, round, text, hnext, (int)sgrid.x);
     };
     // (the token round's first pass keys the text itself)
     if (vb && sh == vb)
@@ -1661,11 +1669,11 @@ static int sort_and_rank(SaWs& w, int64_t nb, int64_t m, int round,
   }
   const int nx = (round + 1) & 1;
   hipLaunchKernelGGL(k_grp_reduce<kRsThreads>, grid, block, 0, stream,
-                     keys[x], w.pos, vb, w.blkmax, w.state, round);
+                     keys[x], w.pos, vb, w.blkmax, w.state, round, (int)grid.x);
   hipLaunchKernelGGL(k_grp_rank<kRsThreads>, grid, block, 0, stream, keys[x],
                      vals[x], w.pos, vb, w.blkmax, w.rank[nx], w.sa, w.gp,
                      w.gsz, w.skip[nx], w.tmax[nx], (uint32_t)pos_tile_of(m),
-                     w.state, round);
+                     w.state, round, (int)grid.x);
   return (int)hipGetLastError();
 }
 
@@ -2173,14 +2181,14 @@ extern "C" int sfx_delta_index_build(const int32_t* delta,
   for (int sh = 0; sh <= hbits; sh += kDigitBits) {
     hipLaunchKernelGGL(k_rs_hist<kRsThreads>, dim3((unsigned)nb),
                        dim3(kRsThreads), 0, stream, keys[x], sh, w.hist, nb,
-                       w.state, 0);
+                       w.state, 0, (int)nb);
     hipLaunchKernelGGL(k_rs_rowscan<kRsThreads>, dim3(kScanBlocks),
                        dim3(kRsThreads), 0, stream, w.hist, nb, w.rowsum,
                        w.state, 0);
     hipLaunchKernelGGL(k_rs_scatter<kRsThreads>, dim3((unsigned)nb),
                        dim3(kRsThreads), 0, stream, keys[x], vals[x],
                        keys[x ^ 1], vals[x ^ 1], sh, w.hist, nb, w.rowsum,
-                       w.state, 0, nullptr, nullptr);
+                       w.state, 0, nullptr, nullptr, (int)nb);
     x ^= 1;
   }
   // two passes (keys of at most 18 bits): the sorted data is back in

@@ -74,3 +74,35 @@ def test_sa_local_round_fits_two_workgroups_per_cu(tmp_path):
         assert r["ScratchSize"] == 0, (name, r)
         assert r["VGPRs"] <= 64, (name, r)
         assert r["Occupancy"] >= 8, (name, r)
+
+
+@pytest.mark.skipif(shutil.which(HIPCC) is None and
+                    not __import__("os").path.exists(HIPCC),
+                    reason="needs hipcc")
+def test_radix_round_kernels_take_short_arguments(tmp_path):
+    """A kernel that reads gridDim or blockDim gets 256 bytes of hidden
+    arguments, which the host writes for every launch.  A build whose every
+    round is enqueued launches the kernels of a radix round hundreds of
+    times, so theirs stay within 128 bytes."""
+    out = tmp_path / "k.s"
+    cmd = [HIPCC, *build.COMMON, "--offload-device-only", "-S",
+           str(build.CSRC / "sa_build.hip"), "-o", str(out)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]
+    sizes = {}
+    size = None
+    for line in out.read_text().splitlines():
+        m = re.match(r"\s+\.kernarg_segment_size: (\d+)", line)
+        if m:
+            size = int(m.group(1))
+        m = re.match(r"\s+\.name:\s+(_Z\S+)", line)
+        if m and size is not None:
+            sizes[m.group(1)] = size
+            size = None
+    parts = ("k_rs_hist", "k_rs_rowscan", "k_rs_scatter", "k_grp_reduce",
+             "k_grp_rank", "k_pos_count", "k_pos_gather", "k_sa_order",
+             "k_sa_local")
+    for part in parts:
+        found = {k: v for k, v in sizes.items() if part in k}
+        assert found, f"no {part} in the kernel list"
+        assert max(found.values()) <= 128, found
