@@ -292,6 +292,31 @@ def test_build_suffix_array_adaptive_batches(gpu, period, n):
         np.testing.assert_array_equal(o, exp if r == last else -9)
 
 
+def test_build_suffix_array_stalls_in_a_row(gpu, monkeypatch):
+    """One repeated token needs the radix path in every round: the stalls
+    hand it out to more and more rounds, and no batch is wasted behind one
+    after the first; random tokens of two values stall once more than the
+    rounds that need it beyond the first."""
+    from suffixgpu_amd import suffix_array as sa
+    batches = []
+    enqueue = sa.enqueue_rounds
+    monkeypatch.setattr(sa, "enqueue_rounds",
+                        lambda m, first, n, *a: (batches.append((first, n)),
+                                                 enqueue(m, first, n, *a)))
+    n = 70000
+    out = torch.empty(n, dtype=torch.int32, device=gpu)
+    sa.build_suffix_array_into(torch.full((n,), 7, dtype=torch.int32,
+                                          device=gpu), n, out, adaptive=True)
+    np.testing.assert_array_equal(N(out), np.arange(n)[::-1])
+    # 16 rounds, 15 of them beyond the one given the path at first
+    assert len(batches) <= 12, batches
+    batches.clear()
+    t = np.random.default_rng(1).integers(0, 2, n).astype(I32)
+    sa.build_suffix_array_into(T(t, gpu), n, out, adaptive=True)
+    _check_suffix_order(t, N(out).astype(np.int64))
+    assert len(batches) <= 5, batches
+
+
 @pytest.mark.parametrize("size", [511, 512, 513, 1000, 2048])
 @pytest.mark.parametrize("at", [0, 2500, 4090])
 def test_build_suffix_array_merged_windows(gpu, size, at):
