@@ -133,20 +133,36 @@ __global__ __launch_bounds__(256) void k_match_back(
 
 // ------------------------------------------------------- first_occurrences
 // One workgroup per threshold row, four columns per thread and pass: a pass
-// is a chain of a load, a count over the waves and a barrier, so few wide
-// passes with the next one's columns on their way beat many narrow ones
-// (512 rows of 8192 columns: 18.6 us in passes of 256 columns with three
-// barriers each, 6.2 us in passes of 4096 with one).
+// is a chain of a load, a count over the waves and a barrier, so wide passes
+// with the next one's columns on their way beat narrow ones as long as the
+// workgroups leave room for them (occ_threads).  Rows of at most kOccMin
+// columns take one column per thread.  The launch alone, us, a column per
+// thread with three barriers a pass / four columns and 1024 threads for every
+// row / now: 64 rows of 8,192 columns with 8 thresholds each 13.1 / 5.6 / 4.8
+// where few columns reach them (9.8 / 4.8 / 4.0 where many do), 256 such rows
+// 21.9 / 18.3 / 13.0, 16 rows of 65,536 85.4 / 16.7 / 15.5, 256 rows of 512
+// 4.0 / 11.8 / 4.0, 64 rows of 128 2.6 / 4.5 / 2.6.
 typedef int32_t Int4Any __attribute__((ext_vector_type(4), aligned(4)));
-constexpr int kOccThreads = 1024;
-constexpr int kOccCols = 4;
+constexpr int kOccMin = 256;
+constexpr int64_t kOccLongRow = 4096;
 
-__global__ __launch_bounds__(kOccThreads) void k_first_occ(
+// 1024 threads while one such workgroup per CU holds every threshold row, 512
+// while two or four do, if a row is long enough for several narrow passes:
+// rows of 4,096 columns (64 x 8 thresholds) 4.2 us with 256 threads, 3.7 with
+// 512; of 2,048 columns 3.3 and 3.2, of 1,024 2.8 and 3.2.
+inline int occ_threads(int64_t n_cols, int64_t rows) {
+  if (n_cols < kOccLongRow || rows > 1024) return 256;
+  return rows <= 256 ? 1024 : 512;
+}
+
+template <int NT, int kCols>
+__global__ __launch_bounds__(NT) void k_first_occ(
     const int32_t* __restrict__ mb, int64_t n_cols,
     const int64_t* __restrict__ thr, int64_t per_row, int R, int64_t* pos,
     int64_t* count) {
-  constexpr int NW = kOccThreads / kWave;
-  constexpr int64_t kPass = (int64_t)kOccThreads * kOccCols;
+  static_assert(kCols == 1 || kCols == 4, "one load per thread and pass");
+  constexpr int NW = NT / kWave;
+  constexpr int64_t kPass = (int64_t)NT * kCols;
   __shared__ int wcnt[2][NW];  // by pass parity: one barrier per pass
   const int64_t row = blockIdx.x;
   const int64_t b = row / per_row;
@@ -157,26 +173,26 @@ __global__ __launch_bounds__(kOccThreads) void k_first_occ(
   int64_t* out = pos + row * R;
   int found = 0;  // the same in every thread
   if (t > 0) {
-    auto load = [&](int64_t i) {
-      Int4Any v = {0, 0, 0, 0};  // (t > 0: a column past the end never hits)
-      if (i + kOccCols <= n_cols) {
-        v = *reinterpret_cast<const Int4Any*>(src + i);
-      } else {
+    auto load = [&](int64_t i, int32_t (&v)[kCols]) {
+      if (kCols == 4 && i + kCols <= n_cols) {
+        const Int4Any w = *reinterpret_cast<const Int4Any*>(src + i);
 #pragma unroll
-        for (int u = 0; u < kOccCols; ++u)
-          if (i + u < n_cols) v[u] = src[i + u];
+        for (int u = 0; u < kCols; ++u) v[u] = w[u];
+      } else {  // (t > 0: a column past the end never hits)
+#pragma unroll
+        for (int u = 0; u < kCols; ++u) v[u] = i + u < n_cols ? src[i + u] : 0;
       }
-      return v;
     };
-    Int4Any cur = load((int64_t)tid * kOccCols);
+    int32_t cur[kCols], nxt[kCols];
+    load((int64_t)tid * kCols, cur);
     int par = 0;
     for (int64_t base = 0; base < n_cols; base += kPass, par ^= 1) {
-      const int64_t i = base + (int64_t)tid * kOccCols;
-      const Int4Any nxt = load(i + kPass);
-      bool hit[kOccCols];
+      const int64_t i = base + (int64_t)tid * kCols;
+      if (base + kPass < n_cols) load(i + kPass, nxt);
+      bool hit[kCols];
       int below = 0, tot = 0;  // hits of lower lanes, of the wave
 #pragma unroll
-      for (int u = 0; u < kOccCols; ++u) {
+      for (int u = 0; u < kCols; ++u) {
         hit[u] = (int64_t)cur[u] >= t;
         const uint64_t bm = ballot(hit[u]);
         below += rank_lt(bm);
@@ -192,16 +208,17 @@ __global__ __launch_bounds__(kOccThreads) void k_first_occ(
         found += c;
       }
 #pragma unroll
-      for (int u = 0; u < kOccCols; ++u) {
+      for (int u = 0; u < kCols; ++u) {
         if (hit[u] && slot < R) out[slot] = i + u;
         slot += hit[u];
       }
       if (found >= R) break;
-      cur = nxt;
+#pragma unroll
+      for (int u = 0; u < kCols; ++u) cur[u] = nxt[u];
     }
   }
   const int f = found < R ? found : R;
-  for (int r = tid; r < R; r += kOccThreads)
+  for (int r = tid; r < R; r += NT)
     if (r >= f) out[r] = 0;
   if (tid == 0) count[row] = f;
 }
@@ -439,9 +456,19 @@ extern "C" int sfx_first_occurrences(const int32_t* mb, int64_t n_cols,
   if (rows == 0) return 0;
   if (!mb || !thr || !pos || !count) return SFX_EINVAL;
   if (max_occ > 0x7fffffff) return SFX_EINVAL;
-  hipLaunchKernelGGL(k_first_occ, dim3((unsigned)rows), dim3(kOccThreads), 0,
-                     stream, mb, n_cols, thr, per_row, (int)max_occ, pos,
-                     count);
+  auto launch = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(threads), 0, stream,
+                       mb, n_cols, thr, per_row, (int)max_occ, pos, count);
+  };
+  const int nt = occ_threads(n_cols, rows);
+  if (n_cols <= kOccMin)
+    launch(k_first_occ<kOccMin, 1>, kOccMin);
+  else if (nt == 256)
+    launch(k_first_occ<256, 4>, 256);
+  else if (nt == 512)
+    launch(k_first_occ<512, 4>, 512);
+  else
+    launch(k_first_occ<1024, 4>, 1024);
   return (int)hipGetLastError();
 }
 

@@ -98,6 +98,25 @@ def test_first_occurrences_edges(gpu, n):
         np.testing.assert_array_equal(N(cnt), ec.reshape(-1))
 
 
+@pytest.mark.parametrize("n", [256, 257, 1025, 4095, 4096, 6000, 9001])
+@pytest.mark.parametrize("rows,c", [(1, 1), (32, 8), (33, 8), (128, 8),
+                                    (1025, 1)])
+def test_first_occurrences_workgroup_sizes(gpu, n, rows, c):
+    """Row lengths and counts of threshold rows on either side of each
+    workgroup size, with hits that are rare, common and everywhere."""
+    from suffixgpu_amd import kernels
+    rng = np.random.default_rng(n + rows)
+    p = np.resize([0.002, 0.1, 1.0], rows)[:, None]
+    mb = np.where(rng.random((rows, n)) < p, rng.integers(1, 9, (rows, n)),
+                  0).astype(I32)
+    thr = rng.integers(0, 9, (rows, c))
+    pos, cnt = kernels.first_occurrences(T(mb, gpu), T(thr.reshape(-1), gpu),
+                                         c, 40)
+    ep, ec = o_first_occ(mb, thr, 40)
+    np.testing.assert_array_equal(N(pos), ep.reshape(-1, 40))
+    np.testing.assert_array_equal(N(cnt), ec.reshape(-1))
+
+
 @pytest.mark.parametrize("n,vocab", [(1, 3), (2, 2), (7, 2), (64, 3),
                                      (4095, 4), (4097, 50), (20000, 3),
                                      (70000, 30000)])
