@@ -227,12 +227,17 @@ __global__ __launch_bounds__(NT) void k_first_occ(
 // A search is a chain of dependent rounds (a suffix position, then its
 // tokens), so what bounds a call is rounds times two memory round trips
 // until the lanes fill the chip, and the probes' reads from then on.
-// G = 32 lanes per pattern, compared by octets, cut 2^22 ranks in 5 rounds;
-// G = 8 with a lane per probe takes 7, each with a dependent load per 4
-// matched tokens, but reads 2.5 times fewer probes.  Calls over 2^22
-// suffixes with G = 8 / G = 32: 2,048 patterns 36.3 / 22.1 us, 8,192 44.3 /
-// 31.3, 16,384 52.0 / 55.3 (over 20,000 suffixes 18.2 / 13.6, 26.1 / 16.3,
-// 27.4 / 26.4), so G = 32 up to kWideSearchMax patterns.
+// G = 32 lanes per pattern, compared by octets (short patterns by a lane per
+// probe), cut 2^22 ranks in 5 rounds; G = 8 with a lane per probe takes 7,
+// each with a dependent load per 4 matched tokens, but reads 2.5 times fewer
+// probes.  Calls over 4,193,504 suffixes with G = 8 / G = 32, us: patterns of
+// 1 .. 32 tokens, 2,048 of them 35.3 / 12.5, 8,192 44.0 / 26.4, 16,384 53.2 /
+// 45.2, 32,768 63.0 / 78.0 (over 20,000 suffixes 22.1 / 9.7, 24.6 / 13.8, 26.2
+// / 22.3, 28.9 / 37.4); of 1 token, 2,048 9.3 / 7.0, 4,096 10.5 / 8.8, 8,192
+// 12.5 / 13.1, 16,384 16.4 / 25.3; of 4 tokens, 4,096 13.3 / 11.5, 8,192 15.8
+// / 17.3.  So G = 32 up to 4,096 patterns of at most 4 tokens, and up to 8,192
+// longer ones (past that, those that turn out short would lose more than the
+// long ones gain).
 constexpr int kSearchThreads = 256;
 
 template <int G, bool kOct>
@@ -473,6 +478,7 @@ extern "C" int sfx_first_occurrences(const int32_t* mb, int64_t n_cols,
 }
 
 constexpr int64_t kWideSearchMax = 1 << 13;
+constexpr int64_t kWideShortMax = 1 << 12;  // patterns of at most 4 tokens
 
 extern "C" int sfx_sa_search(const int32_t* sa, const int32_t* corpus,
                              int64_t n, const int32_t* pattern,
@@ -484,7 +490,7 @@ extern "C" int sfx_sa_search(const int32_t* sa, const int32_t* corpus,
   if (!sa || !corpus || !plen || !lower || !upper ||
       (width > 0 && !pattern))
     return SFX_EINVAL;
-  const bool wide = batch <= kWideSearchMax;
+  const bool wide = batch <= (width <= 4 ? kWideShortMax : kWideSearchMax);
   const int64_t per_block = kSearchThreads / (wide ? 32 : 8);
   const int64_t blocks = (batch + per_block - 1) / per_block;
   if (wide)

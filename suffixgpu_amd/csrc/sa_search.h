@@ -182,6 +182,10 @@ __device__ __forceinline__ int cmp_probes_key(
 struct __attribute__((packed, aligned(4))) Tokens4 {
   int32_t t[4];
 };
+// Patterns of at most this many tokens are compared by a lane per probe all
+// the same: two loads instead of eight and the ballots.  (pc then holds
+// pattern tokens 0 .. 3.)
+constexpr int kLaneCmp = 8;
 
 template <int G, class ProbeFn, class PatFn>
 __device__ __forceinline__ int cmp_probes_corpus(
@@ -200,18 +204,54 @@ __device__ __forceinline__ int cmp_probes_corpus(
   const int kn = plen < 4 * kParts ? plen : 4 * kParts;
   const bool live = 4 * part < kn;
   const int32_t own = sa[probe_of(gl)];  // n < 2^31
-  Tokens4 v[kInstr];
+  auto token = [&](int64_t at) {
+    return at < n ? corpus[at > 0 ? at : 0] : -1;
+  };
+  if (plen <= kLaneCmp) {  // a lane per probe (pc holds tokens 0 .. 3)
+    const bool two = plen > 4;
+    int32_t p2[4];
 #pragma unroll
-  for (int i = 0; i < kInstr; ++i) {
-    const int64_t at =
-        (int64_t)__shfl(own, gbase + i * kRows + sub) + 4 * part;
-    if (live && at >= 0 && at + 3 < n) {
-      v[i] = *reinterpret_cast<const Tokens4*>(corpus + at);
+    for (int j = 0; j < 4; ++j) p2[j] = 4 + j < plen ? pat_at(4 + j) : 0;
+    Tokens4 w, w2;
+    if (own >= 0 && (int64_t)own + 8 <= n) {
+      w = *reinterpret_cast<const Tokens4*>(corpus + own);
+      if (two) w2 = *reinterpret_cast<const Tokens4*>(corpus + own + 4);
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        v[i].t[j] = live && at + j < n ? corpus[at + j > 0 ? at + j : 0] : -1;
+      for (int j = 0; j < 4; ++j) {
+        w.t[j] = token((int64_t)own + j);
+        w2.t[j] = token((int64_t)own + 4 + j);
+      }
     }
+    int r = 0;
+    if (two) {
+#pragma unroll
+      for (int j = 3; j >= 0; --j)
+        if (4 + j < plen && w2.t[j] != p2[j]) r = w2.t[j] < p2[j] ? -1 : 1;
+    }
+#pragma unroll
+    for (int j = 3; j >= 0; --j)
+      if (j < plen && w.t[j] != pc[j]) r = w.t[j] < pc[j] ? -1 : 1;
+    return r;
+  }
+  int32_t at[kInstr];
+#pragma unroll
+  for (int i = 0; i < kInstr; ++i)
+    at[i] = __shfl(own, gbase + i * kRows + sub);
+  Tokens4 v[kInstr];
+  // (a branch per load would make each wait for the one before)
+  if (ballot(own < 0 || (int64_t)own + 4 * kParts > n) == 0) {
+    if (live) {
+#pragma unroll
+      for (int i = 0; i < kInstr; ++i)
+        v[i] = *reinterpret_cast<const Tokens4*>(corpus + at[i] + 4 * part);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < kInstr; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        v[i].t[j] = live ? token((int64_t)at[i] + 4 * part + j) : -1;
   }
   int cv = 0;
 #pragma unroll
@@ -273,8 +313,9 @@ __device__ __forceinline__ void kary_bounds(
   int32_t pt[kCoop ? 4 : 32];
   static_assert(!kCorpusOct || kCoop, "octets");
   if (keys || kCorpusOct) {
-    // cooperative: pattern tokens 4 * (gl % 8) .. + 3; else all of them
-    const int j0 = kCoop ? 4 * (gl % 8) : 0;
+    // cooperative: pattern tokens 4 * (gl % 8) .. + 3 (a pattern that one
+    // lane compares: its first four); else all of them
+    const int j0 = kCoop && !(kCorpusOct && plen <= kLaneCmp) ? 4 * (gl % 8) : 0;
 #pragma unroll
     for (int j = 0; j < (kCoop ? 4 : 32); ++j)
       pt[j] = j0 + j < plen ? pat_at(j0 + j) : 0;

@@ -521,6 +521,36 @@ def test_sa_search_widths_and_batches(gpu, n, width):
         np.testing.assert_array_equal(N(hi), ee[rep])
 
 
+@pytest.mark.parametrize("rows", [1, 64, 4096, 4097])
+@pytest.mark.parametrize("width", [1, 2, 4, 5, 8, 9])
+def test_sa_search_short_patterns(gpu, rows, width):
+    """Patterns that a lane compares by itself and the first that an octet
+    does, side by side in a wave (lengths 0 .. width), over few tokens with a
+    pad among them, many of them at the corpus' end (past which a token
+    compares as -1, the least here, so the order is one); on both lane counts
+    (up to 4096 patterns of at most 4 tokens and past it)."""
+    from suffixgpu_amd import kernels
+    rng = np.random.default_rng(rows * 10 + width)
+    n = 1500
+    corpus = rng.choice(np.array([0, 1, 2, 3, 2**31 - 1], I32), n)
+    sa = o_build_sa(corpus)
+    b = min(rows, 200)
+    plen = rng.integers(0, width + 1, size=b)
+    pat = np.full((b, width), -1, I32)
+    for i in range(b):
+        at = n - rng.integers(1, 12) if i % 2 else rng.integers(0, n)
+        seg = corpus[at:at + plen[i]]
+        pat[i, :seg.shape[0]] = seg
+        if i % 5 == 0 and plen[i]:
+            pat[i, rng.integers(0, plen[i])] = rng.integers(-3, 4)
+    es, ee = o_search(sa, corpus, pat, plen)
+    rep = np.arange(rows) % b
+    lo, hi = kernels.sa_search(T(sa.astype(I32), gpu), T(corpus, gpu),
+                               T(pat[rep], gpu), T(plen[rep], gpu))
+    np.testing.assert_array_equal(N(lo), es[rep])
+    np.testing.assert_array_equal(N(hi), ee[rep])
+
+
 @pytest.mark.parametrize("r", [1, 4, 30, 128, 256, 700])
 @pytest.mark.parametrize("minp", [0.0, 0.1])
 def test_expand_chain(gpu, r, minp):
