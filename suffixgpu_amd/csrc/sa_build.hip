@@ -1823,18 +1823,23 @@ __global__ __launch_bounds__(256) void k_dix_start(
 // first entry is its count of positions in lower buckets.  Wave w takes the
 // positions w * 64 * steps .. + 64 * steps - 1, one per lane and step, so a
 // position's place in its bucket is its wave's first place (a scan over the
-// waves' counts), the earlier steps and the lower lanes.  The nine launches
-// below take 45 us at 2^16 positions and as much again in the gaps between
-// them; this one takes 10 us (16-25 with a full delta), bound by the hashing of
-// every position in every workgroup.  Four rows harvested into a delta of
-// 2^16: 162 -> 125 us with this and the chunks of k_ingest_move.
+// waves' counts), the earlier steps and the lower lanes.  What bounds it is
+// the workgroup whose range has the most frequent token: it places entries in
+// every step, one distinct bucket after another (12 us of reading and
+// counting, 31 of placing for 65,536 Zipf tokens; 19 us in all where no token
+// is frequent).  Capacity 2^16, Zipf text with repeats, 5 / 25 / 50 / 75 / 100%
+// live: 8 / 14 / 24 / 33 / 44 us, the nine launches below 42 / 42 / 43 / 43 /
+// 43 back to back; alone, with the host's wait, 22 / 29 / 39 / 48 / 59 and 65.
 constexpr int kDixThreads = 1024;
 constexpr int kDixWaves = kDixThreads / kWave;
 constexpr int kDixUnroll = 8;  // steps a wave loads at once
+constexpr int kDixFewHits = 16;  // of a step, that LDS may add one by one
 constexpr int64_t kDixOneMax = 1 << 16;
 constexpr int kDixGroups = 256;      // workgroups at most: one per CU
 constexpr int kDixRangeMin = 64;     // buckets a workgroup owns, at least
 constexpr int kDixRangeMax = 1 << (kDeltaBucketBitsMax - 8);
+constexpr int kDixSteps = kDixOneMax / kDixThreads;  // of a wave, at most
+static_assert(kDixSteps == kWave, "a lane per step");
 static_assert(kDixRangeMax <= kDixThreads &&
                   kDixRangeMax * kDixGroups >= (1 << kDeltaBucketBitsMax),
               "a thread per bucket of a range");
@@ -1844,56 +1849,70 @@ __global__ __launch_bounds__(kDixThreads) void k_dix_one(
     int64_t D, int hbits, int R, int4* __restrict__ ent,
     uint32_t* __restrict__ start) {
   __shared__ uint32_t cnt[kDixWaves * kDixRangeMax];
+  __shared__ uint64_t hits[kDixWaves][kDixSteps];
   __shared__ uint32_t red[kDixWaves];
   const int tid = threadIdx.x;
-  const int wv = tid / kWave;
+  const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int ln = lane_id();
   int64_t dl64 = *delta_len;
   dl64 = dl64 < 0 ? 0 : (dl64 > D ? D : dl64);
   const int dl = (int)dl64;
   const uint32_t lo = (uint32_t)blockIdx.x * (uint32_t)R;
   const int steps = (dl + kDixThreads - 1) / kDixThreads;
-  const int p0 = wv * kWave * steps + ln;
-  // f(position, token, live) for each of the wave's steps; the next
-  // kDixUnroll steps' tokens are on their way while these are worked on
-  auto each_step = [&](auto f) {
-    int32_t cur[kDixUnroll], nxt[kDixUnroll];
-    auto load = [&](int32_t (&t)[kDixUnroll], int s0) {
-#pragma unroll
-      for (int u = 0; u < kDixUnroll; ++u) {
-        const int p = p0 + (s0 + u) * kWave;
-        t[u] = s0 + u < steps && p < dl ? delta[p] : 0;
+  const int wbase = wv * kWave * steps;
+  for (int e = tid; e < kDixWaves * R; e += kDixThreads) cnt[e] = 0;
+  hits[wv][ln] = 0;
+  __syncthreads();
+  // Counts by wave and bucket, positions in lower buckets, and each step's
+  // lanes with a position of this range.  The next kDixUnroll steps' tokens
+  // are on their way while these are worked on.
+  uint32_t* mine = cnt + wv * R;
+  uint32_t below = 0;
+  {
+    auto work = [&](int s, int32_t t, bool live) {
+      const uint32_t bk = live ? delta_bucket(t, hbits) : ~0u;
+      below += bk < lo;
+      const uint32_t k = bk - lo;
+      const uint64_t m = ballot(live && k < (uint32_t)R);
+      if (m == 0) return;
+      if (ln == 0) hits[wv][s] = m;
+      if (popc(m) <= kDixFewHits) {
+        if ((m >> ln) & 1u) atomicAdd(&mine[k], 1u);
+        return;
+      }
+      for (uint64_t todo = m; todo;) {  // equal ones would queue in LDS
+        const uint32_t lead = (uint32_t)__builtin_amdgcn_readlane(
+            (int)k, __builtin_ctzll(todo));
+        const uint64_t peers = todo & ballot(k == lead);
+        if (ln == 0) atomicAdd(&mine[lead], (uint32_t)popc(peers));
+        todo &= ~peers;
       }
     };
-    load(cur, 0);
-    for (int s0 = 0; s0 < steps; s0 += kDixUnroll) {
-      load(nxt, s0 + kDixUnroll);
+    int32_t cur[kDixUnroll], nxt[kDixUnroll];
+    auto load = [&](int32_t (&t)[kDixUnroll], int s0, uint32_t last) {
 #pragma unroll
-      for (int u = 0; u < kDixUnroll; ++u) {
-        const int p = p0 + (s0 + u) * kWave;
-        f(p, cur[u], s0 + u < steps && p < dl);
-      }
+      for (int u = 0; u < kDixUnroll; ++u)
+        t[u] = delta[min((uint32_t)(wbase + (s0 + u) * kWave + ln), last)];
+    };
+    // batches of whole steps, then the rest
+    const int full = max(0, min(steps, (dl - wbase) / kWave));
+    const int tail = full / kDixUnroll * kDixUnroll;
+    if (tail > 0) load(cur, 0, ~0u);
+    for (int s0 = 0; s0 < tail; s0 += kDixUnroll) {
+      load(nxt, s0 + kDixUnroll < tail ? s0 + kDixUnroll : s0, ~0u);
+#pragma unroll
+      for (int u = 0; u < kDixUnroll; ++u) work(s0 + u, cur[u], true);
 #pragma unroll
       for (int u = 0; u < kDixUnroll; ++u) cur[u] = nxt[u];
     }
-  };
-  for (int e = tid; e < kDixWaves * R; e += kDixThreads) cnt[e] = 0;
-  __syncthreads();
-  // counts by wave and bucket; positions in lower buckets
-  uint32_t* mine = cnt + wv * R;
-  uint32_t below = 0;
-  each_step([&](int, int32_t t, bool live) {
-    const uint32_t bk = delta_bucket(t, hbits);
-    below += live && bk < lo;
-    uint64_t todo = ballot(live && bk - lo < (uint32_t)R);
-    while (todo) {
-      const uint32_t lead = (uint32_t)__builtin_amdgcn_readlane(
-          (int)bk, __builtin_ctzll(todo));
-      const uint64_t peers = todo & ballot(bk == lead);
-      if (ln == 0) atomicAdd(&mine[lead - lo], (uint32_t)popc(peers));
-      todo &= ~peers;
+    if (tail < steps) {
+      load(cur, tail, (uint32_t)(dl - 1));
+#pragma unroll
+      for (int u = 0; u < kDixUnroll; ++u)
+        if (tail + u < steps)
+          work(tail + u, cur[u], wbase + (tail + u) * kWave + ln < dl);
     }
-  });
+  }
   uint32_t base;
   block_exscan1<kDixThreads>(below, red, &base);
   // bucket totals, their prefix, and each wave's first place
@@ -1912,29 +1931,53 @@ __global__ __launch_bounds__(kDixThreads) void k_dix_one(
   }
   if (blockIdx.x == gridDim.x - 1 && tid == 0) start[lo + R] = (uint32_t)dl;
   __syncthreads();
-  auto entry = [&](int q, int32_t x) {
-    return make_int4(q, x, q >= 1 ? delta[q - 1] : -1,
-                     q >= 2 ? delta[q - 2] : -1);
-  };
-  each_step([&](int p, int32_t t, bool live) {
-    const uint32_t bk = delta_bucket(t, hbits);
-    uint64_t todo = ballot(live && bk - lo < (uint32_t)R);
-    while (todo) {
-      const int first = __builtin_ctzll(todo);
-      const uint32_t lead =
-          (uint32_t)__builtin_amdgcn_readlane((int)bk, first);
-      const uint64_t peers = todo & ballot(bk == lead);
-      uint32_t b0 = 0;
-      if (ln == first) b0 = atomicAdd(&mine[lead - lo], (uint32_t)popc(peers));
-      b0 = (uint32_t)__builtin_amdgcn_readlane((int)b0, first);
-      if ((peers >> ln) & 1u) ent[b0 + rank_lt(peers)] = entry(p, t);
-      todo &= ~peers;
+  // The steps with hits, in order, the tokens of kDixUnroll steps read at
+  // once and by every lane (a load in a branch waits for the one before):
+  // most ranges have hits in a quarter of the steps, but the range of the
+  // most frequent token in all, and it sets the launch's end.
+  const uint64_t own = hits[wv][ln];
+  uint64_t left = ballot(own != 0);
+  while (left) {
+    uint64_t m[kDixUnroll];
+    int q[kDixUnroll];
+    int32_t t[kDixUnroll], t1[kDixUnroll], t2[kDixUnroll];
+#pragma unroll
+    for (int u = 0; u < kDixUnroll; ++u) {
+      const int s = left ? __builtin_ctzll(left) : 0;
+      const uint32_t mlo =
+          (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)own, s);
+      const uint32_t mhi =
+          (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(own >> 32), s);
+      m[u] = left ? (uint64_t)mhi << 32 | mlo : 0ull;
+      left &= left - 1;
+      q[u] = min(wbase + s * kWave + ln, dl - 1);
+      t[u] = delta[q[u]];
+      t1[u] = delta[max(q[u] - 1, 0)];
+      t2[u] = delta[max(q[u] - 2, 0)];
     }
-  });
+#pragma unroll
+    for (int u = 0; u < kDixUnroll; ++u) {
+      const uint32_t k = delta_bucket(t[u], hbits) - lo;
+      for (uint64_t todo = m[u]; todo;) {
+        const int first = __builtin_ctzll(todo);
+        const uint32_t lead =
+            (uint32_t)__builtin_amdgcn_readlane((int)k, first);
+        const uint64_t peers = todo & ballot(k == lead);
+        const uint32_t b0 = mine[lead];
+        if (ln == first) mine[lead] = b0 + (uint32_t)popc(peers);
+        if ((peers >> ln) & 1u)
+          ent[b0 + rank_lt(peers)] =
+              make_int4(q[u], t[u], q[u] >= 1 ? t1[u] : -1,
+                        q[u] >= 2 ? t2[u] : -1);
+        todo &= ~peers;
+      }
+    }
+  }
   // positions past the live length follow every bucket, in order
   for (int64_t q = dl + (int64_t)blockIdx.x * kDixThreads + tid; q < D;
        q += (int64_t)gridDim.x * kDixThreads)
-    ent[q] = entry((int)q, delta[q]);
+    ent[q] = make_int4((int)q, delta[q], q >= 1 ? delta[q - 1] : -1,
+                       q >= 2 ? delta[q - 2] : -1);
 }
 
 }  // namespace sfx
