@@ -9,6 +9,7 @@ can be captured into a HIP graph.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from pathlib import Path
@@ -190,6 +191,21 @@ def lib() -> ctypes.CDLL:
     _check_single_hip_runtime()
     _lib = handle
     return _lib
+
+
+@contextlib.contextmanager
+def unrelated_to_captures():
+    """The calling thread's waits inside have nothing to do with a graph
+    that another thread (or this one, on another stream) is capturing: in
+    HIP's default mode such a wait fails and invalidates that capture.
+    The mode is the thread's own and is put back."""
+    exchange = lib().hipThreadExchangeStreamCaptureMode
+    mode = ctypes.c_int(2)  # hipStreamCaptureModeRelaxed
+    check(exchange(ctypes.byref(mode)), "capture mode")
+    try:
+        yield
+    finally:
+        check(exchange(ctypes.byref(mode)), "capture mode")
 
 
 # Error codes of the C ABI besides hipError_t values.

@@ -14,7 +14,8 @@ from collections import deque
 import torch
 
 from suffixgpu_amd._lib import (SA_ROUNDS_EXPECT_FINAL, SA_ROUNDS_RADIX,
-                                check, lib, require_gpu, stream_of)
+                                check, lib, require_gpu, stream_of,
+                                unrelated_to_captures)
 
 
 def sa_workspace_bytes(n: int) -> int:
@@ -83,6 +84,7 @@ def build_suffix_array_into(text: torch.Tensor, m: int, out: torch.Tensor,
                              stream_of(text.device)), "build_suffix_array")
 
 
+@unrelated_to_captures()
 def _build_adaptive(text: torch.Tensor, m: int, out: torch.Tensor,
                     workspace: torch.Tensor,
                     radix_mask: int = DEFAULT_RADIX_MASK) -> BuildState:

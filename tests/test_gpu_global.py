@@ -1038,3 +1038,51 @@ def test_queries_with_and_without_gram_table(gpu, slots):
                         o.draft(q, ql, p, 12, min_token_prob=0.05,
                                 caps=caps)):
         np.testing.assert_array_equal(N(got), exp)
+
+
+def test_rebuild_beside_another_threads_capture(gpu):
+    """An index without a rebuild stream rebuilds on one thread's stream
+    while another thread captures a graph (in the default, global, mode):
+    neither disturbs the other."""
+    import threading
+    from suffixgpu_amd.global_index import GlobalIndex
+    rng = np.random.default_rng(4)
+    docs = [T(rng.integers(0, 50, 200).astype(I32), gpu) for _ in range(8)]
+    gi = GlobalIndex(1 << 14, 1 << 10, 16, device=gpu, rebuild_threshold=512)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        gi.append_documents(docs[:4])
+    torch.cuda.synchronize()
+    before = gi.swap_count
+    started, failed = threading.Event(), []
+
+    def harvest():
+        started.wait(30)
+        try:
+            with torch.cuda.stream(stream):
+                gi.append_documents(docs[4:])
+        except Exception as e:
+            failed.append(e)
+
+    worker = threading.Thread(target=harvest)
+    worker.start()
+    x = torch.zeros(64, device=gpu)
+    graph = torch.cuda.CUDAGraph()
+    try:
+        with torch.cuda.graph(graph):
+            x += 1
+            started.set()
+            worker.join(30)
+            x += 1
+    finally:
+        started.set()
+        worker.join(30)
+    assert not failed and gi.swap_count > before
+    for _ in range(2):
+        graph.replay()
+    torch.cuda.synchronize()
+    assert N(x).tolist() == [4.0] * 64
+    m = min(gi.active_len + 1, gi.capacity)
+    from oracle.sa import build_suffix_array as o_build_sa
+    np.testing.assert_array_equal(N(gi.sa)[:m], o_build_sa(N(gi.corpus)[:m]))
