@@ -42,13 +42,18 @@ def global_caps(max_pattern_len: int, num_backoff: int) -> list[int]:
 
 
 # Local-only rows of fewer tokens than this go without the match launch even
-# where they do not fit a CU's LDS: the step's one 1024-thread workgroup per
-# row streams them about as fast as two launches take, or faster (30,000
-# tokens, 1 / 2 / 8 / 32 rows: 23.8 / 25.4 / 26.8 / 31.7 us streamed, 22.2 /
-# 32.5 / 32.5 / 33.3 split; 44,000: 22.6 / 24.8 / 32.1 / 36.4 and 17.6 / 28.2
-# / 28.2 / 31.4; 60,000: 36.4 / 36.3 / 38.6 / 51.1 and 25.6 / 26.6 / 29.9 /
-# 30.8).  With global memory on, a row has 512 threads and splitting wins
-# from the first length on (30,000, 1 / 8 rows: 32.1 / 41.1 and 28.4 / 32.3).
+# where they do not fit a CU's LDS.  Between there and 49,152 tokens which form
+# is faster depends on the text more than on the length or the batch (rows
+# filled to 25-100%, streamed by the step's one 1024-thread workgroup a row /
+# split, us: one row of 29,000 / 30,000 / 44,000 tokens 29.2 / 23.8 / 22.6 and
+# 26.6 / 22.2 / 17.6; two rows 29.2 / 25.4 / 24.8 and 26.4 / 32.5 / 28.2; 32
+# rows 29.4 / 31.7 / 36.4 and 31.6 / 33.3 / 31.4), and rows far shorter than
+# the buffer always pay for the second launch, so these keep the one launch.
+# From 49,152 on splitting wins for every batch measured (60,000, 1 / 2 / 8 /
+# 32 rows: 36.4 / 36.3 / 38.6 / 51.1 and 25.6 / 26.6 / 29.9 / 30.8).  With
+# global memory on, a row has 512 threads and splitting wins from the first
+# length on for several rows (28,000, 2 / 4 / 16 rows: 34.6 / 39.4 / 42.3 and
+# 31.4 / 32.9 / 33.6) and is level for one (27,000 .. 36,000: 26.3 and 25.9).
 SPLIT_MIN_LOCAL = 49152
 
 
@@ -138,6 +143,23 @@ class SuffixGPUDrafter:
                 delta_index=global_delta_index)
 
     # ------------------------------------------------------------------
+    @property
+    def split_seq(self) -> int:
+        """Token buffers of at least this many columns take the match
+        launch before the step.  What a row's match costs then hardly grows
+        with the row, but the launch costs 5 us and more when every row is
+        short: in a buffer of 131,072 columns with global memory, 1 / 64
+        rows of about 2,600 tokens 24 / 35 us against 18 / 26 without it,
+        of 13,000 29 / 36 against 33 / 40, of 65,000 and more 26 / 49
+        against 89 / 159.  The host does not know the rows' lengths; a
+        program that does may raise it (1 << 30: never).  It holds for the
+        calls, and the captures, made after it was set."""
+        return self._split_seq
+
+    @split_seq.setter
+    def split_seq(self, columns: int) -> None:
+        self._split_seq = int(columns)
+
     def poll(self) -> None:
         """Called by the host between steps: a background rebuild whose
         event has completed becomes the live index."""

@@ -511,3 +511,68 @@ def test_local_step_counts_in_place(gpu, s, scratch):
     del keep
     for g, e in zip((draft, nv, counts, dev), (*exp, exp_rows)):
         np.testing.assert_array_equal(N(g), e)
+
+
+def test_split_rows_share_the_match_launch(gpu):
+    """More parts than the match launch has workgroups: each takes several
+    parts of its row, over rows from empty to full, against the same rows
+    streamed by one workgroup each."""
+    from suffixgpu_amd import _lib
+    b, s = 300, 40962
+    rng = np.random.default_rng(b)
+    p = _lib.make_params(16, 32, 128, 1, [1 << i for i in range(8)], (), 2.0,
+                         0.0, 0.1, 0.0)
+    tokens = rng.integers(0, 3, size=(b, s)).astype(I32)
+    tokens[::7] = np.resize(rng.integers(0, 50, size=900), s)
+    nt = rng.integers(0, s - 20, b).astype(I32)
+    nt[:5] = (0, 1, 4096, 8193, s)
+    sampled = np.full((b, 17), -1, I32)
+    for i in range(b):
+        n = rng.integers(0, 17)
+        sampled[i, :n] = tokens[i, rng.integers(0, s - 20):][:n]
+    got = _rows_step(gpu, p, tokens, nt, sampled, None, True)
+    exp = _rows_step(gpu, p, tokens, nt, sampled, None, False)
+    for g, e in zip(got, exp):
+        np.testing.assert_array_equal(g, e)
+    assert (exp[1] > 0).sum() > b // 2
+
+
+@pytest.mark.parametrize("enable_global", [False, True])
+def test_split_seq_is_the_callers_choice(gpu, enable_global):
+    """A drafter told never to take the match launch streams the rows that
+    it would split, eagerly and in a capture, with equal results."""
+    s = 50000
+    w, d, o = _global_pair(gpu, seed=9, b=4, s=2048)
+    if not enable_global:
+        from suffixgpu_amd import SuffixGPUDrafter
+        d = SuffixGPUDrafter(device=gpu, **dict(GLOBAL_KW,
+                                                enable_global=False))
+    assert d.split_seq <= s
+    rng = np.random.default_rng(s)
+    rows = np.resize(rng.integers(0, 40, 7000), (3, s)).astype(I32)
+    nt = np.array([s - 20, s // 2, 4097], I32)
+    sampled = np.full((3, 9), -1, I32)
+    for i in range(3):
+        sampled[i, :4] = rows[i, nt[i]:nt[i] + 4]
+    dev = [T(x, gpu) for x in (nt, rows, sampled)]
+    exp = [N(x) for x in d.propose_with_update(*dev)]
+    graphs = []
+    for seq in (d.split_seq, 1 << 30):
+        d.split_seq = seq
+        for g, e in zip(d.propose_with_update(*dev), exp):
+            np.testing.assert_array_equal(N(g), e)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            out = d.propose_with_update(*dev)
+        graphs.append((g, out))
+    # replays over other rows than the captured ones, in turn
+    for shift in (1, 2, 3):
+        cur = np.roll(rows, shift, axis=0)
+        for g, out in graphs:
+            dev[1].copy_(T(cur, gpu))
+            g.replay()
+            torch.cuda.synchronize()
+            fresh = d.propose_with_update(dev[0], T(cur, gpu), dev[2])
+            for a, e in zip(out, fresh):
+                np.testing.assert_array_equal(N(a), N(e))
+    assert (exp[1] > 0).any()
