@@ -302,11 +302,11 @@ def test_ingest_then_cross_request_draft(gpu):
 
 @pytest.mark.parametrize("enable_global", [False, True])
 def test_step_long_rows_vs_oracle(gpu, enable_global):
-    """Rows of 40000 tokens (streamed local role) in the fused step, with
-    and without the global index (without it, rows this long run the
-    1024-thread local-only kernel): rows are windows of the document
-    stream at committed lengths around the 16384-position chunk
-    boundaries."""
+    """Rows of 40000 tokens, which do not fit LDS, with and without the
+    global index (with it they take the match launch, without it the
+    1024-thread local-only kernel streams them): rows are windows of the
+    document stream at committed lengths around the 16384-position chunk
+    boundaries of a streamed row."""
     from suffixgpu_amd import SuffixGPUDrafter
     s, t = 40000, 17
     w, d, o = _global_pair(gpu, seed=9, b=4, s=2048)
@@ -334,6 +334,55 @@ def test_step_long_rows_vs_oracle(gpu, enable_global):
     np.testing.assert_array_equal(N(draft), ed)
     np.testing.assert_array_equal(N(nv), env)
     assert (env > 0).sum() > 0
+
+
+@pytest.mark.parametrize("entry", ["step", "noalloc", "rows"])
+def test_long_rows_with_index_by_entry_point(gpu, entry):
+    """Rows of 40000 tokens with an index through each entry point of the
+    step -- without scratch one workgroup streams a row, with it the match
+    launch spreads them -- against the oracle."""
+    from suffixgpu_amd import _lib
+    L = _lib.lib()
+    s, t = 40000, 17
+    w, d, o = _global_pair(gpu, seed=9, b=4, s=2048)
+    stream = np.concatenate(w.active_docs + w.delta_docs).astype(I32)
+    rng = np.random.default_rng(10)
+    nt = np.array([0, 4096, 16384, 20000, s - t, s], I32)
+    b = len(nt)
+    rows = np.zeros((b, s), dtype=I32)
+    sampled = np.full((b, t), -1, dtype=I32)
+    for i, q in enumerate(nt):
+        off = int(rng.integers(0, stream.shape[0] - s - t))
+        rows[i] = stream[off:off + s]
+        acc = int(rng.integers(1, t + 1))
+        sampled[i, :acc] = stream[off + q:off + q + acc]
+    to = rows.copy()
+    exp = o.propose_with_update(nt, to, sampled)
+    dev = T(rows, gpu)
+    bt, keep = _lib.make_batch(dev, T(nt, gpu), sampled=T(sampled, gpu),
+                               limit=s)
+    out = [torch.full((b, d.k), -9, dtype=torch.int32, device=gpu),
+           torch.full((b,), -9, dtype=torch.int32, device=gpu),
+           torch.full((b,), -9, dtype=torch.int32, device=gpu)]
+    args = [d._params, d.global_index.index_struct(), bt,
+            *[x.data_ptr() for x in out]]
+    cur = torch.cuda.current_stream().cuda_stream
+    ws = d._workspace(b, cur)
+    n = int(L.sfx_row_scratch_size(d._params, b, s))
+    scratch = torch.full((n,), 0x5b, dtype=torch.uint8, device=gpu)
+    if entry == "noalloc":
+        rc = L.sfx_propose_step_noalloc(*args, cur)
+    elif entry == "step":
+        rc = L.sfx_propose_step(*args, ws.data_ptr(), ws.numel(), cur)
+    else:
+        rc = L.sfx_propose_step_rows(*args, ws.data_ptr(), ws.numel(),
+                                     scratch.data_ptr(), n, cur)
+    assert rc == 0 and n > 0
+    torch.cuda.synchronize()
+    del keep
+    for g, e in zip((*out, dev), (*exp, to)):
+        np.testing.assert_array_equal(N(g), e)
+    assert (exp[1] > 0).sum() >= 3
 
 
 @pytest.mark.parametrize("s", [8192, 16384])

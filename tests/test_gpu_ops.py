@@ -390,6 +390,49 @@ def _check_suffix_order(t, got):
                   ((t[a] == t[b]) & (rank[a + 1] < rank[b + 1])))
 
 
+def _past_small_tiles(t, top):
+    """t with distinct larger tokens behind it (finished after the token
+    round), so that the text takes the 4096-position local tile and t's
+    suffixes come first in it."""
+    fill = np.random.default_rng(0).permutation(1 << 19).astype(I32)
+    return np.concatenate([t, top + 1 + fill]).astype(I32)
+
+
+@pytest.mark.parametrize("size", [511, 512, 513, 2047, 2048, 2049])
+@pytest.mark.parametrize("at", [0, 2500, 4090, 4096])
+def test_build_suffix_array_groups_in_large_tiles(gpu, size, at):
+    """A two-token group of a size on either side of the merge and of the
+    cap, `at` positions into a 4096-position tile (past 2500 it runs on into
+    the next one), beside small groups, with few distinct keys and many."""
+    from suffixgpu_amd.suffix_array import build_suffix_array_into
+    rng = np.random.default_rng(size + at)
+    for keys in (3, 400):
+        small = rng.integers(0, 9, size=at).astype(I32)
+        cont = np.stack([np.full(size, 10), np.full(size, 10),
+                         11 + rng.integers(0, keys, size)], 1)
+        t = _past_small_tiles(np.concatenate([small, cont.reshape(-1)]), 500)
+        out = torch.empty(t.shape[0], dtype=torch.int64, device=gpu)
+        build_suffix_array_into(T(t, gpu), t.shape[0], out, adaptive=True)
+        _check_suffix_order(t, N(out))
+
+
+@pytest.mark.parametrize("period", [1, 2, 700])
+@pytest.mark.parametrize("n", [2049, 5000, 9001])
+def test_build_suffix_array_repeats_in_large_tiles(gpu, period, n):
+    """A repeat that needs the radix path in no, some or every round (stalls
+    and their resumption) and many batches of rounds, in a text of 4096-
+    position tiles, adaptively and with every round enqueued."""
+    from suffixgpu_amd.suffix_array import build_suffix_array_into
+    rep = np.resize(np.random.default_rng(n).permutation(period), n)
+    t = _past_small_tiles(rep, period)
+    out = torch.empty(t.shape[0], dtype=torch.int64, device=gpu)
+    for adaptive in (True, False):
+        out.fill_(-9)
+        build_suffix_array_into(T(t, gpu), t.shape[0], out,
+                                adaptive=adaptive)
+        _check_suffix_order(t, N(out))
+
+
 def test_build_suffix_array_long_radix_list(gpu):
     """A radix list of more tiles than its launches have workgroups, so that
     every list kernel takes a second tile: all of 2.3M tokens of 8 values

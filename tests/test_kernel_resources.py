@@ -63,8 +63,9 @@ def test_step_kernels_fit_two_workgroups_per_cu(src, kernel, tmp_path):
                     not __import__("os").path.exists(HIPCC),
                     reason="needs hipcc")
 def test_sa_local_round_fits_two_workgroups_per_cu(tmp_path):
-    """The suffix-array build's local round (1024 threads, 24 KiB of LDS):
-    at most 64 VGPRs (eight waves per SIMD) and no scratch.  A cross-lane
+    """The suffix-array build's local round (1024 threads, 49 KB of LDS with
+    2048-position tiles, 74 KB with 4096): at most 64 VGPRs (eight waves per
+    SIMD) and no scratch.  A cross-lane
     read feeding its sort decision once pushed it to 128 VGPRs with 376
     bytes of scratch per lane."""
     res = _resources("sa_build.hip", tmp_path)
