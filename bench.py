@@ -1141,7 +1141,7 @@ def summarize_api(trace_dir: str) -> dict:
     replay = [s for s in sections
               if s["calls"].get("hipGraphLaunch", 0) == SYNC_CHECK_STEPS]
     # The last section: the device harvests (three ingest launches each,
-    # then the nine of the delta token index's rebuild).
+    # then the delta token index's, one for a delta of up to 2^16).
     harvest = [s for s in sections
                if s["calls"].get("hipLaunchKernel", 0) >= 3 * SYNC_CHECK_STEPS
                and s["calls"].get("hipLaunchKernel", 0)

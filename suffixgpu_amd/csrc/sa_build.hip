@@ -18,12 +18,13 @@
 // A round sorts each group by one of two means, chosen per group on the
 // device from its size:
 //  * groups of at most kCap suffixes: one launch for the round.  A
-//    workgroup owns the groups whose head lies in its 4096-position tile
-//    (a group that started in the tile before is skipped, skip[] holding
+//    workgroup owns the groups whose head lies in its tile of 4096 or 2048
+//    positions (pos_tile_of; a group that started in the tile before is skipped, skip[] holding
 //    its length; one that runs on into the next tile is followed), sorts
 //    each of them by its keys in LDS (a 64-lane bitonic sort per
 //    64-position window, then a binary search in every other window of the
-//    group, or merges of the windows where a group is large) and writes the new order, heads and sizes back;
+//    group, or merges of the windows where a group is large) and writes the
+//    new order, heads and sizes back;
 //  * groups above kCap (the radix part): their positions are compacted
 //    into a list keyed (head, rank[i + h] + 1) in SA order, LSD radix
 //    sorted, and the group heads of the sorted list are written back.
@@ -558,9 +559,10 @@ __global__ __launch_bounds__(NT) void k_rs_rowscan(
 // counts the next pass's digits by destination tile into hnext (null after
 // the last pass; no histogram launch).  A pass is then one launch instead of
 // three, which is what a short list's pass costs: whole builds of repetitive
-// text of 3,000 tokens 186 -> 161 us, 20,000 213 -> 198, 61,003 238 -> 230,
-// 200,000 303 -> 295, but 262,144 302 -> 311 (the columns and the counts'
-// atomics by then cost more than the launches), so kFewTiles is 32.
+// text of 3,000 tokens 186 -> 161 us, 20,000 213 -> 198, 61,003 238 -> 230.
+// A list of 64 tiles would still gain (200,000 tokens 300 -> 290; 262,144 306
+// -> 304), but a wave's counts then take one more ballot each, which the
+// shorter ones pay (131,072 tokens 260 -> 265), so kFewTiles is 32.
 template <int NT, bool kVal = true, bool kText = false, bool kFew = false>
 __global__ __launch_bounds__(NT) void k_rs_scatter(
     const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin,
@@ -1202,12 +1204,15 @@ __device__ __forceinline__ void merge_windows(uint64_t* sk, uint32_t* sid,
 //  2. per window: the lanes of one group form a chunk; one bitonic sort by
 //     (chunk, key, lane) sorts every chunk in place; the sorted keys go to
 //     LDS, and equal-key runs inside the chunk are found by lane masks;
-//  3. per element: counts of keys below / at most its own in every other
-//     chunk of its group (binary search in LDS) give its new position
-//     (ties by old position), its new group's head and its size; it writes
-//     sa, gp, rank_next, and the head writes gsz; skip_next[b + 1] gets
-//     the length of the group running into the next tile, or 0 (the
-//     round's radix part then sets it for a group it sorted).
+//  3. per element: its new position (ties by old position), its new group's
+//     head and size, from counts of keys below / at most its own in every
+//     other chunk of its group (binary search in LDS), or, in a tile with a
+//     group above kMergeMin, from the merged order (merge_windows).  What
+//     changed is written: sa and gp, rank_next unless both rank buffers hold
+//     the head already (kSameHead at the group's size), gsz by a new head;
+//     skip_next[b + 1] gets the length of the group running into the next
+//     tile, or 0 (the round's radix part then sets it for a group it
+//     sorted).
 // Groups above kCap are left to the round's radix launches; when the
 // caller enqueued none (global_follows == 0) this launch marks the round
 // stalled and does nothing.  A round with no group left sets the done
