@@ -224,8 +224,8 @@ int sfx_propose_step(const sfx_params* p, const sfx_index* index,
  * call's work on `stream` -- a launch before the step's spreads the match
  * of every row over the chip.  With less scratch, or none, one workgroup
  * streams each such row, as sfx_propose_step does; the results are equal.
- * What the launch saves grows with the rows' lengths, what it costs (5 us and
- * more) does not, and only the caller may know the lengths: the drafter
+ * What the launch saves grows with the rows' lengths, what it costs (2 to
+ * 6 us) does not, and only the caller may know the lengths: the drafter
  * class gives scratch from the first width that takes any when it has an
  * index, and from 49,152 columns on when it has none. */
 size_t sfx_row_scratch_size(const sfx_params* p, int64_t batch, int64_t seq);

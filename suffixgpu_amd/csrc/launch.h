@@ -77,8 +77,8 @@ int local_chunk(const sfx_params& p, int64_t S, size_t cap = kMaxLds,
 size_t local_lds_bytes(const sfx_params& p, int64_t S, int chunk,
                        int nthreads = kLocalThreadsDefault, int mb_full = 0);
 
-// LDS of a split row's step workgroup.
-size_t split_lds_bytes(const sfx_params& p);
+// LDS of a step with split rows that holds rows of up to `solo` tokens.
+size_t split_lds_bytes(const sfx_params& p, int solo = 0);
 
 int check_global(const sfx_params& p, const sfx_index& ix, int64_t batch);
 int mb_lds_bytes(const sfx_index& ix, int parts);

@@ -66,8 +66,8 @@ size_t local_lds_bytes(const sfx_params& p, int64_t S, int chunk,
                    : layout_bytes(p, S, chunk, nthreads, mb_full);
 }
 
-size_t split_lds_bytes(const sfx_params& p) {
-  return (size_t)split_layout(p.max_pattern_len, p.num_thresholds,
+size_t split_lds_bytes(const sfx_params& p, int solo) {
+  return (size_t)split_layout(solo, p.max_pattern_len, p.num_thresholds,
                               p.max_occurrences, p.k, kLocalThreads / kWave)
       .total;
 }

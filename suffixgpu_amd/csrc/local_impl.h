@@ -33,6 +33,7 @@ struct LocalArgs {
   int chunk;  // 0: the whole row is staged in LDS; else streamed in chunks
   int mb_full;  // streamed: LDS holds the match lengths of the whole row
   RowScratch rs;  // split rows: what the match launch left for the step
+  int solo;  // split: rows of at most this many tokens are held in LDS whole
 };
 
 struct LocalLayout {
@@ -89,14 +90,15 @@ __host__ __device__ inline LocalLayout local_layout(int S, int P, int C,
   return L;
 }
 
-// A split row's layout: no row and no match lengths, but per candidate the
-// output offsets of kOffsParts parts (an odd stride: the lanes of a wave
-// read one part's offsets of all candidates).
+// The layout of a step with split rows: per candidate the output offsets of
+// kOffsParts parts (an odd stride: the lanes of a wave read one part's
+// offsets of all candidates), and room for a row of `solo` tokens.
 constexpr int kOffsParts = kWave;
 constexpr int kOffsStride = kOffsParts + 1;
-__host__ __device__ inline LocalLayout split_layout(int P, int C, int R,
-                                                    int K, int nwaves) {
-  return local_layout(0, P, C, R, K, nwaves, 0, 0, C * kOffsStride * 4);
+__host__ __device__ inline LocalLayout split_layout(int solo, int P, int C,
+                                                    int R, int K,
+                                                    int nwaves) {
+  return local_layout(solo, P, C, R, K, nwaves, 0, 0, C * kOffsStride * 4);
 }
 
 constexpr int kLocalThreads = 512;
@@ -340,8 +342,11 @@ __device__ __forceinline__ void local_finish(
 // match lengths and once more, in order, to compact the first R ends per
 // candidate with the counts carried from chunk to chunk (stopping once
 // every candidate holds R).  The expansion reads continuations from HBM.
-template <bool kStream, int NT = kLocalThreads>
-__device__ __forceinline__ void local_body(const LocalArgs& a,
+// kSolo: a row of a step with split rows that has at most a.solo tokens, for
+// which split_layout has room; the caller finishes it.  Returns false when the
+// row is masked and done.
+template <bool kStream, int NT = kLocalThreads, bool kSolo = false>
+__device__ __forceinline__ bool local_body(const LocalArgs& a,
                                            unsigned char* smem, int b) {
   constexpr int NW = NT / kWave;
   const sfx_params& p = a.p;
@@ -354,8 +359,10 @@ __device__ __forceinline__ void local_body(const LocalArgs& a,
   const int R = p.max_occurrences;
   const int K = p.k;
   const bool mb_full = kStream && a.mb_full;
-  const LocalLayout L = local_layout(S, P, C, R, K, NW, kStream ? a.chunk : 0,
-                                     mb_full ? 1 : 0);
+  const LocalLayout L =
+      kSolo ? split_layout(a.solo, P, C, R, K, NW)
+            : local_layout(S, P, C, R, K, NW, kStream ? a.chunk : 0,
+                           mb_full ? 1 : 0);
   int32_t* row = (int32_t*)(smem + L.row);  // the row, or a staged chunk
   uint8_t* mbuf = (uint8_t*)(smem + L.mb);
   int32_t* pat = (int32_t*)(smem + L.pat);
@@ -410,14 +417,16 @@ __device__ __forceinline__ void local_body(const LocalArgs& a,
         grow[pos] = v;
       }
     }
+    // (the count was read before the row was staged)
+    if (!kStream && a.new_counts && tid == 0) a.new_counts[b] = (int32_t)q;
   }
   __syncthreads();
-  store_count(a, b, st);
+  if (kStream) store_count(a, b, st);
 
   if (a.mode == kLocalStep && !st.mask) {
     for (int j = tid; j < K; j += NT) a.draft[(int64_t)b * K + j] = -1;
     if (tid == 0) a.num_valid[b] = 0;
-    return;
+    return false;
   }
 
   SFX_TRACE_POINT(1);
@@ -606,7 +615,8 @@ __device__ __forceinline__ void local_body(const LocalArgs& a,
     }
   }
 
-  local_finish<NT>(a, smem, L, b, st, src_row);
+  if constexpr (!kSolo) local_finish<NT>(a, smem, L, b, st, src_row);
+  return true;
 }
 
 // The local role of a split row: k_row_match (row_match.hip) has applied the
@@ -618,8 +628,8 @@ __device__ __forceinline__ void local_body(const LocalArgs& a,
 // only those that hold one of the first R ends of some candidate.  The
 // expansion reads continuations from HBM.
 template <int NT>
-__device__ __forceinline__ void local_split_body(const LocalArgs& a,
-                                                 unsigned char* smem, int b) {
+__device__ __forceinline__ bool local_split_front(const LocalArgs& a,
+                                                  unsigned char* smem, int b) {
   constexpr int NW = NT / kWave;
   const sfx_params& p = a.p;
   const int tid = threadIdx.x;
@@ -630,7 +640,7 @@ __device__ __forceinline__ void local_split_body(const LocalArgs& a,
   const int C = p.num_thresholds;
   const int R = p.max_occurrences;
   const int K = p.k;
-  const LocalLayout L = split_layout(P, C, R, K, NW);
+  const LocalLayout L = split_layout(a.solo, P, C, R, K, NW);
   int32_t* hist = (int32_t*)(smem + L.hist);
   int32_t* cand = (int32_t*)(smem + L.cand);
   int32_t* found = (int32_t*)(smem + L.found);
@@ -649,7 +659,7 @@ __device__ __forceinline__ void local_split_body(const LocalArgs& a,
   if (!st.mask) {
     for (int j = tid; j < K; j += NT) a.draft[(int64_t)b * K + j] = -1;
     if (tid == 0) a.num_valid[b] = 0;
-    return;
+    return false;
   }
   const int qe = (int)(st.q < 0 ? 0 : (st.q < S ? st.q : S));
   // one row's counts and lengths are less than 2^32 bytes: 32-bit offsets
@@ -741,7 +751,25 @@ __device__ __forceinline__ void local_split_body(const LocalArgs& a,
     if (!more) break;
     __syncthreads();  // found is rewritten below
   }
-  local_finish<NT>(a, smem, L, b, st, a.bt.tokens + (int64_t)b * S);
+  return true;
+}
+
+// A step with split rows: a row that split_layout has room for is held there
+// whole, as if the buffer were no wider, and the match launch has left it
+// alone.  Both kinds read continuations from HBM and share one expansion.
+template <int NT>
+__device__ __forceinline__ void local_split_body(const LocalArgs& a,
+                                                 unsigned char* smem, int b) {
+  const sfx_params& p = a.p;
+  const RowState st = row_state(a.bt, b);
+  const bool open = a.solo > 0 && st.q <= a.solo
+                        ? local_body<false, NT, true>(a, smem, b)
+                        : local_split_front<NT>(a, smem, b);
+  if (!open) return;
+  const LocalLayout L =
+      split_layout(a.solo, p.max_pattern_len, p.num_thresholds,
+                   p.max_occurrences, p.k, NT / kWave);
+  local_finish<NT>(a, smem, L, b, st, a.bt.tokens + (int64_t)b * a.bt.seq);
 }
 
 // The local-only decode step with kWideThreads per row (local.hip); -1

@@ -20,15 +20,16 @@ constexpr int kMaxPat = 255;
 // chip holds at once, five per CU by their LDS.  One per part kept short rows
 // of a wide buffer waiting for thousands of workgroups without a part.  Steps
 // of 256 rows in a buffer of 131,072 tokens with global memory, us, a
-// workgroup per part / these / one workgroup streaming each row: rows of 2% of
-// the buffer 76 / 43 / 33, of 10% 83 / 49 / 70, of 50-100% 88 / 87 / 379; 64
-// rows 40 / 35 / 26, 40 / 35 / 39, 48 / 50 / 152.
+// workgroup per part / these / these without the rows that the step holds in
+// LDS: rows of 2% of the buffer 76 / 41 / 37, of 10% 83 / 47 / 46, of 50-100%
+// 88 / 86 / 88; 64 rows 40 / 35 / 30, 40 / 36 / 36, 48 / 49 / 49.
 constexpr int64_t kMatchGrid = 1280;
 // Tokens staged before a part's first position: the longest walk reads
 // x(i - 1 - t) for t up to P + 2 (four tokens a step).
 __host__ __device__ inline int match_halo(int P) { return stream_halo(P) + 4; }
 
-// nwg workgroups take a row's parts in turn.
+// nwg workgroups take a row's parts in turn.  Rows of at most a.solo tokens
+// are left to the step.
 __global__ __launch_bounds__(kMatchThreads) void k_row_match(LocalArgs a,
                                                              int nwg) {
   // ends of one wave that matched four tokens, walked after the scan
@@ -49,6 +50,7 @@ __global__ __launch_bounds__(kMatchThreads) void k_row_match(LocalArgs a,
   int32_t* grow = a.bt.tokens + (int64_t)b * S;
   const int32_t* sp =
       a.bt.sampled ? a.bt.sampled + (int64_t)b * a.bt.num_sampled : nullptr;
+  if (st.q <= a.solo) return;
   if (blockIdx.x == 0 && sp) {  // the step's scatter (proposer.py:162-184)
     for (int64_t j = tid; j < a.bt.num_sampled; j += kMatchThreads) {
       const int64_t pos = st.base + j;

@@ -114,6 +114,19 @@ size_t split_scratch_bytes(const sfx_params& p, int64_t batch, int64_t seq) {
   return row_scratch_layout(p.max_pattern_len, batch, seq, nullptr, nullptr);
 }
 
+// The longest row, in steps of 1024 tokens, that a step with split rows holds
+// in LDS whole: what fits `cap` bytes, up to kSoloMax.  Rows of 2% of a buffer
+// of 131,072 columns, 8 / 64 / 256 of them with global memory: 28 / 30 / 37 us
+// a step instead of 31 / 35 / 41 when they take the match launch, of 3-6% 30 /
+// 30 / 42 and 34 / 34 / 42; of 8-12% 34 / 36 / 46 either way (with 12,288
+// tokens here 34 / 37 / 47).
+constexpr int kSoloMax = 8192;
+int solo_tokens(const sfx_params& p, size_t cap) {
+  int n = 0;
+  while (n < kSoloMax && split_lds_bytes(p, n + 1024) <= cap) n += 1024;
+  return n;
+}
+
 // The fused step over `workspace` laid out with counter arrays of
 // `counter_rows` rows (-1: the batch size).  Rows that do not fit LDS whole
 // are split over the chip when `row_scratch` holds the match launch's
@@ -170,7 +183,8 @@ int launch_step(const sfx_params* p, const sfx_index* ix, const sfx_batch* bt,
   if (split) {
     row_scratch_layout(p->max_pattern_len, bt->batch, bt->seq, row_scratch,
                        &a.l.rs);
-    lds = split_lds_bytes(*p);
+    a.l.solo = solo_tokens(*p, cap);
+    lds = split_lds_bytes(*p, a.l.solo);
   } else {
     a.l.chunk = local_chunk(*p, bt->seq, cap, kLocalThreadsDefault,
                             &a.l.mb_full);

@@ -147,11 +147,11 @@ class SuffixGPUDrafter:
     def split_seq(self) -> int:
         """Token buffers of at least this many columns take the match
         launch before the step.  What a row's match costs then hardly grows
-        with the row, but the launch costs 5 us and more when every row is
-        short: in a buffer of 131,072 columns with global memory, 1 / 64
-        rows of about 2,600 tokens 24 / 35 us against 18 / 26 without it,
+        with the row, but the launch itself costs 2 to 6 us when every row
+        is short: in a buffer of 131,072 columns with global memory, 1 / 64
+        rows of about 2,600 tokens 23 / 30 us against 17 / 26 without it,
         of 13,000 29 / 36 against 33 / 40, of 65,000 and more 26 / 49
-        against 89 / 159.  The host does not know the rows' lengths; a
+        against 89 / 160.  The host does not know the rows' lengths; a
         program that does may raise it (1 << 30: never).  It holds for the
         calls, and the captures, made after it was set."""
         return self._split_seq

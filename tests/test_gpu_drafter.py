@@ -625,3 +625,50 @@ def test_split_seq_is_the_callers_choice(gpu, enable_global):
             for a, e in zip(out, fresh):
                 np.testing.assert_array_equal(N(a), N(e))
     assert (exp[1] > 0).any()
+
+
+@pytest.mark.parametrize("b,s", [(12, 40000), (100, 28000), (180, 27002)])
+def test_rows_held_and_split_in_one_step(gpu, b, s):
+    """Rows on either side of the length that a step with split rows holds
+    in LDS, in one batch with an index, at one, two and three workgroups per
+    CU: against the same rows without scratch."""
+    from suffixgpu_amd import _lib
+    L = _lib.lib()
+    w, d, o = _global_pair(gpu, seed=9, b=4, s=2048)
+    t = 17
+    rng = np.random.default_rng(b)
+    stream = np.concatenate(w.active_docs + w.delta_docs).astype(I32)
+    stream = np.resize(stream, max(stream.shape[0], 2 * s))
+    rows = np.zeros((b, s), I32)
+    sampled = np.full((b, t), -1, I32)
+    nt = rng.integers(0, s - t, b).astype(I32)
+    nt[:11] = (0, 1, 4095, 4096, 4097, 8175, 8190, 8191, 8192, 8193, s - t)
+    nt[11:b // 2] = rng.integers(1, 8300, max(0, b // 2 - 11))
+    for i in range(b):
+        off = int(rng.integers(0, stream.shape[0] - s))
+        rows[i] = stream[off:off + s]
+        acc = int(rng.integers(0, t + 1))
+        sampled[i, :acc] = rows[i, nt[i]:nt[i] + acc]
+    cur = torch.cuda.current_stream().cuda_stream
+    n = int(L.sfx_row_scratch_size(d._params, b, s))
+    assert n > 0
+    results = []
+    for scratch in (n, 0):
+        dev = T(rows, gpu)
+        bt, keep = _lib.make_batch(dev, T(nt, gpu), sampled=T(sampled, gpu),
+                                   limit=s)
+        out = [torch.full((b, d.k), -9, dtype=torch.int32, device=gpu),
+               torch.full((b,), -9, dtype=torch.int32, device=gpu),
+               torch.full((b,), -9, dtype=torch.int32, device=gpu)]
+        ws = d._workspace(b, cur)
+        mem = torch.full((n,), 0x5b, dtype=torch.uint8, device=gpu)
+        _lib.check(L.sfx_propose_step_rows(
+            d._params, d.global_index.index_struct(), bt,
+            *[x.data_ptr() for x in out], ws.data_ptr(), ws.numel(),
+            mem.data_ptr(), scratch, cur), "step")
+        torch.cuda.synchronize()
+        del keep
+        results.append([N(x) for x in (*out, dev)])
+    for g, e in zip(*results):
+        np.testing.assert_array_equal(g, e)
+    assert (results[0][1] > 0).sum() > b // 3
